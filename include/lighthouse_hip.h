@@ -40,7 +40,7 @@ extern "C" {
 #define LH_ERR_RUNTIME 5      /* a HIP runtime call (synchronize, copy, symbol lookup) failed */
 
 /* The ABI this header declares; lh_abi_version() of a matching library returns it. */
-#define LH_ABI_VERSION 9
+#define LH_ABI_VERSION 10
 
 #define LH_DTYPE_BF16 0       /* row element type: bfloat16 (the reference configs) */
 #define LH_DTYPE_F16 1        /* row element type: IEEE half */
@@ -265,6 +265,26 @@ int lh_attn_bwd_dq(const void *q, const void *k, const void *v, int64_t sb, int6
                    int split, const int32_t *indices, int B, int H, int n, int D, float scale,
                    const void *dout, const float *lse, const float *delta,
                    void *dq, int dtype, void *stream);
+
+/*
+ * lh_attn_fwd and lh_attn_bwd with flags (parts: bit 0 = dK/dV, bit 1 = dQ; the
+ * outputs of a part that is not asked for may be NULL).  With LH_ATTN_SHAPED a
+ * launch may split its work by its own sizes, B * H and n (here: half blocks of
+ * 128 queries whose keys two halves of a workgroup share, where the heaviest
+ * 256-query block would outlast the rest); the last bits of its results then
+ * depend on them, while with flags = 0 a (b, h) has the same bits alone and
+ * beside others.  Unknown bits give LH_ERR_INVALID_ARG.
+ */
+#define LH_ATTN_SHAPED 1
+int lh_attn_fwd_ex(const void *q, const void *k, const void *v, int64_t sb, int64_t ss, int64_t sh,
+                   const void *qp, const void *kp, const void *vp, int64_t pb, int64_t ps, int64_t ph,
+                   int split, const int32_t *indices, int B, int H, int n, int D, float scale,
+                   void *out, float *lse, int dtype, int flags, void *stream);
+int lh_attn_bwd_ex(int parts, const void *q, const void *k, const void *v, int64_t sb, int64_t ss, int64_t sh,
+                   const void *qp, const void *kp, const void *vp, int64_t pb, int64_t ps, int64_t ph,
+                   int split, const int32_t *indices, int B, int H, int n, int D, float scale,
+                   const void *dout, const float *lse, const float *delta,
+                   void *dq, void *dk, void *dv, int dtype, int flags, void *stream);
 
 /*
  * Work-queue faults of the persistent attention launches (lh_attn_fwd,

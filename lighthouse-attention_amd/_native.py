@@ -52,6 +52,10 @@ _SIGS = {
                               _I, _I, _I, _I, _F, _P, _P, _P, _P, _P, _I, _P]),
     "lh_attn_bwd_dq": (_I, [_P, _P, _P, _L, _L, _L, _P, _P, _P, _L, _L, _L, _I, _P,
                             _I, _I, _I, _I, _F, _P, _P, _P, _P, _I, _P]),
+    "lh_attn_fwd_ex": (_I, [_P, _P, _P, _L, _L, _L, _P, _P, _P, _L, _L, _L, _I, _P,
+                            _I, _I, _I, _I, _F, _P, _P, _I, _I, _P]),
+    "lh_attn_bwd_ex": (_I, [_I, _P, _P, _P, _L, _L, _L, _P, _P, _P, _L, _L, _L, _I, _P,
+                            _I, _I, _I, _I, _F, _P, _P, _P, _P, _P, _P, _I, _I, _P]),
     "lh_attn_status": (_I, [_P]),
     "lh_attn_queue_slot": (_I, [_P, _P]),
     "lh_attn_set_schedule": (_I, [_I, _P]),
@@ -457,8 +461,13 @@ def _bwd_args_check(rows, indices, dout, lse, delta):
     rows.check(indices)
 
 
-def attn_fwd(rows: Rows, indices, B: int, H: int, n: int, D: int = D_SUPPORTED, scale: float | None = None):
+def attn_fwd(rows: Rows, indices, B: int, H: int, n: int, D: int = D_SUPPORTED, scale: float | None = None,
+             shaped: bool = False):
     """Causal attention over the rows named by ``indices`` [B, H, n] (None = identity).
+
+    ``shaped`` (LH_ATTN_SHAPED): the launch may split its work by B * H and n, and the
+    last bits of the result then depend on them; otherwise a (b, h) has the same bits
+    alone and beside others.
 
     Returns ``(O [B, H, n, D] of the rows' dtype, lse fp32 [B, H, n])`` (lse in the
     exp2 domain)."""
@@ -471,8 +480,8 @@ def attn_fwd(rows: Rows, indices, B: int, H: int, n: int, D: int = D_SUPPORTED, 
     out = torch.empty(B, H, n, D, dtype=rows.dtype, device=dev)
     lse = torch.empty(B, H, n, dtype=torch.float32, device=dev)
     with torch.cuda.device(dev):
-        rc = lib().lh_attn_fwd(*rows.args(), _ptr(idx), B, H, n, D, scale, _ptr(out), _ptr(lse), rows.dtype_code,
-                               _stream(dev))
+        rc = lib().lh_attn_fwd_ex(*rows.args(), _ptr(idx), B, H, n, D, scale, _ptr(out), _ptr(lse), rows.dtype_code,
+                                  int(shaped), _stream(dev))
     _check(rc, "lh_attn_fwd")
     _check_queues(dev, "lh_attn_fwd")
     return out, lse
@@ -495,24 +504,27 @@ def attn_bwd_dkdv(rows: Rows, indices, B: int, H: int, n: int, dout, lse, delta,
 
 
 def attn_bwd_dq(rows: Rows, indices, B: int, H: int, n: int, dout, lse, delta, D: int = D_SUPPORTED,
-                scale: float | None = None):
-    """dQ of the gathered rows (query-stationary kernel): [B, H, n, D] of the rows' dtype."""
+                scale: float | None = None, shaped: bool = False):
+    """dQ of the gathered rows (query-stationary kernel): [B, H, n, D] of the rows' dtype.
+    ``shaped`` as in ``attn_fwd``."""
     _bwd_args_check(rows, indices, dout, lse, delta)
     dev = rows.q.device
     scale = D ** -0.5 if scale is None else scale
     idx = indices.contiguous() if indices is not None else None
     dq = torch.empty(B, H, n, D, dtype=rows.dtype, device=dev)
     with torch.cuda.device(dev):
-        rc = lib().lh_attn_bwd_dq(*rows.args(), _ptr(idx), B, H, n, D, scale, _ptr(dout.contiguous()),
-                                  _ptr(lse), _ptr(delta), _ptr(dq), rows.dtype_code, _stream(dev))
+        rc = lib().lh_attn_bwd_ex(2, *rows.args(), _ptr(idx), B, H, n, D, scale, _ptr(dout.contiguous()),
+                                  _ptr(lse), _ptr(delta), _ptr(dq), None, None, rows.dtype_code, int(shaped),
+                                  _stream(dev))
     _check(rc, "lh_attn_bwd_dq")
     _check_queues(dev, "lh_attn_bwd_dq")
     return dq
 
 
 def attn_bwd(rows: Rows, indices, B: int, H: int, n: int, dout, lse, delta, D: int = D_SUPPORTED,
-             scale: float | None = None):
-    """Gradients w.r.t. the gathered q, k, v rows: three [B, H, n, D] of the rows' dtype."""
+             scale: float | None = None, shaped: bool = False):
+    """Gradients w.r.t. the gathered q, k, v rows: three [B, H, n, D] of the rows' dtype.
+    ``shaped`` as in ``attn_fwd``."""
     _bwd_args_check(rows, indices, dout, lse, delta)
     dev = rows.q.device
     scale = D ** -0.5 if scale is None else scale
@@ -520,8 +532,8 @@ def attn_bwd(rows: Rows, indices, B: int, H: int, n: int, dout, lse, delta, D: i
     dout = dout.contiguous()
     dq, dk, dv = (torch.empty(B, H, n, D, dtype=rows.dtype, device=dev) for _ in range(3))
     with torch.cuda.device(dev):
-        rc = lib().lh_attn_bwd(*rows.args(), _ptr(idx), B, H, n, D, scale, _ptr(dout), _ptr(lse), _ptr(delta),
-                               _ptr(dq), _ptr(dk), _ptr(dv), rows.dtype_code, _stream(dev))
+        rc = lib().lh_attn_bwd_ex(3, *rows.args(), _ptr(idx), B, H, n, D, scale, _ptr(dout), _ptr(lse), _ptr(delta),
+                                  _ptr(dq), _ptr(dk), _ptr(dv), rows.dtype_code, int(shaped), _stream(dev))
     _check(rc, "lh_attn_bwd")
     _check_queues(dev, "lh_attn_bwd")
     return dq, dk, dv

@@ -49,6 +49,7 @@ namespace {
 
 constexpr int BMK = 128;  // keys per workgroup of the key-stationary kernel: 4 waves x 32
 constexpr int QW = 8;     // waves per workgroup of the query-stationary kernels (32 queries each)
+constexpr int HB = 128;   // queries per workgroup of the half-block kernels (two waves per 32 queries)
 constexpr int BN = 64;   // rows per LDS tile
 constexpr float RESCALE_LOG2 = 8.0f;
 constexpr int FWD_AHEAD = 4;  // forward: LDS operands read this many MFMAs ahead
@@ -731,6 +732,114 @@ __device__ __forceinline__ void fwd_block(const AttnArgs& a, int bh, int qb, bf1
   }
 }
 
+// One query block of HB = 128 rows: waves w and w + 4 own the same 32 queries,
+// waves 0-3 take the even key tiles and waves 4-7 the odd ones, and the two
+// halves' states are joined through LDS at the end.  KV: 8 tiles, ML: 2 KB.
+//
+// Bound by the chain of one block's tiles, which it halves: a step of two tiles
+// takes about 1.3 times a step of one (twice the K/V copies for half the
+// queries), so it is for launches whose heaviest block outlasts the chip's
+// share of the work (half_blocks).  Forward / dQ, one box: 8 heads of 1152 rows
+// 35 / 43 -> 26 / 33 us, of 2048 59 / 73 -> 40 / 49, of 4608 119 / 149 -> 84 /
+// 104, of 7000 180 / 220 -> 126 / 164, 12 of 4780 124 / 157 -> 97 / 123; but 32
+// of 4608 184 / 240 -> 222 / 283 and 8 of 18432 646 / 847 -> 747 / 961.
+template <typename T>
+__device__ __forceinline__ void fwd_half_block(const AttnArgs& a, int bh, int qb, bf16_t* KV, float* ML) {
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), grp = wave >> 2, w4 = wave & 3;
+  const int n = a.n;
+  const BhRows m = bh_rows(a, bh);
+  const int q0 = qb * HB, qw = q0 + w4 * 32, my_q = qw + l32;
+
+  u32x4 qf[8];
+  {
+    bool pooled;
+    const uint32_t o = row_off(m, my_q, pooled) + 8 * hh;
+    const bf16_t* p = (pooled ? m.qp : m.q) + o;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) qf[c] = ldg16(p + 16 * c);
+  }
+
+  const int kend = min(q0 + HB, n);
+  const int nt = (kend + BN - 1) / BN, ns = (nt + 1) >> 1;  // key tiles, steps of two
+  // step j: tile 2 j + grp, in buffer j & 1 of this group
+  bf16_t *K0 = KV + grp * 4 * TILE, *V0 = K0 + TILE, *K1 = K0 + 2 * TILE, *V1 = K0 + 3 * TILE;
+  int rr[4];
+  load_rows<4>(rr, m, grp * BN, w4, lane);
+  issue_rows<4>(K0, m.k, m.kp, V0, m.v, m.vp, m, rr, w4, lane);
+  load_rows<4>(rr, m, (2 + grp) * BN, w4, lane);
+  wait_loads();
+  __syncthreads();
+
+  FwdState st;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) st.o[d] = floatx16{};
+  st.m = -INFINITY;
+  st.l = 0.f;
+  const int nfull = min((qw + 1) / BN, n / BN);
+
+  auto step = [&](int j, const bf16_t* Ks, const bf16_t* Vs, bf16_t* Kn, bf16_t* Vn) {
+    const int t = 2 * j + grp;
+    if (t + 2 < nt) issue_rows<4>(Kn, m.k, m.kp, Vn, m.v, m.vp, m, rr, w4, lane);
+    if (t + 4 < nt) load_rows<4>(rr, m, (t + 4) * BN, w4, lane);
+    if (t < nt && t * BN <= qw + 31) fwd_tile<T>(st, qf, Ks, Vs, t * BN, my_q, n, lane, a.sl2, t >= nfull);
+    wait_loads();
+    __syncthreads();
+  };
+  for (int j = 0; j < ns; j += 2) {
+    step(j, K0, V0, K1, V1);
+    step(j + 1, K1, V1, K0, V0);
+  }
+
+  // the odd tiles' state -> LDS (register order) -> the even tiles' waves
+  float4* ox = reinterpret_cast<float4*>(KV) + w4 * 1024 + lane;
+  if (grp) {
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        ox[(4 * d + g) * 64] = float4{st.o[d][4 * g], st.o[d][4 * g + 1], st.o[d][4 * g + 2], st.o[d][4 * g + 3]};
+    ML[w4 * 128 + lane] = st.m;
+    ML[w4 * 128 + 64 + lane] = st.l;
+  }
+  __syncthreads();
+  if (grp || my_q >= n) return;
+  const float m1 = ML[w4 * 128 + lane], l1 = ML[w4 * 128 + 64 + lane];
+  const float mx = fmaxf(st.m, m1);
+  // -inf: none of the half's keys is visible, or all their scores are -inf
+  const float f0 = st.m == -INFINITY ? 0.f : ex2((st.m - mx) * a.sl2);
+  const float f1 = m1 == -INFINITY ? 0.f : ex2((m1 - mx) * a.sl2);
+  float l = fmaf(f0, st.l, f1 * l1);
+  l += __shfl_xor(l, 32);
+  const float inv_l = l > 0.f ? 1.0f / l : 0.f;
+#pragma unroll
+  for (int d = 0; d < 4; ++d)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float4 x = ox[(4 * d + g) * 64];
+      st.o[d][4 * g + 0] = fmaf(f0, st.o[d][4 * g + 0], f1 * x.x);
+      st.o[d][4 * g + 1] = fmaf(f0, st.o[d][4 * g + 1], f1 * x.y);
+      st.o[d][4 * g + 2] = fmaf(f0, st.o[d][4 * g + 2], f1 * x.z);
+      st.o[d][4 * g + 3] = fmaf(f0, st.o[d][4 * g + 3], f1 * x.w);
+    }
+  store_rows<T>(a.out + ((int64_t)bh * n + my_q) * LH_D, st.o, inv_l, hh);
+  if (hh == 0) a.lse[(int64_t)bh * n + my_q] = l > 0.f ? mx * a.sl2 + __log2f(l) : -INFINITY;
+}
+
+template <typename T>
+__global__ __launch_bounds__(64 * QW, 8 / QW) void attn_fwd_half_kernel(const AttnArgs a, const WorkQ q) {
+  __shared__ __attribute__((aligned(1024))) bf16_t KV[8 * TILE];
+  __shared__ float ML[4 * 128];
+  __shared__ int wq_s[2];
+  int bh, qb;
+  bool have = wq_first(q, a.nq, a.BH, true, bh, qb);
+  if (!have && q.ctr) have = wq_next(q, a.nq, a.BH, true, -1, 0, bh, qb, wq_s);
+  for (int k = 1; have; ++k) {
+    fwd_half_block<T>(a, bh, qb, KV, ML);
+    have = q.ctr && wq_next(q, a.nq, a.BH, true, -1, k, bh, qb, wq_s);
+  }
+}
+
 template <typename T, int EPI>
 __global__ __launch_bounds__(64 * QW, 8 / QW) void attn_fwd_kernel(const AttnArgs a, const QPlan p, const WorkQ q) {
   __shared__ __attribute__((aligned(1024))) bf16_t K0[TILE];
@@ -860,17 +969,22 @@ __device__ __forceinline__ void dq_tile(floatx16 (&acc)[4], float& rsum, const u
 // over the sample (|c| above a quarter of the keys' spread about it); N(0, 1)
 // keys (|c|^2 about 2 against 126) skip it and give the uncentred result.
 // Every wave forms the same sums in the same order, so the choice is uniform.
-template <typename T>
-__device__ __forceinline__ void dq_block(const AttnArgs& a, int bh, int qb, bf16_t* K0, bf16_t* K1, bf16_t* V0,
-                                         bf16_t* V1, float* kc) {
-  constexpr int BM = 32 * QW;
+// HALF: a block of HB rows, the key tiles shared out as in fwd_half_block and
+// the two halves' sums joined through LDS.
+template <typename T, bool HALF>
+__device__ __forceinline__ void dq_block(const AttnArgs& a, int bh, int qb, bf16_t* KV, float* kc) {
+  constexpr int BM = HALF ? HB : 32 * QW;
+  constexpr int G = HALF ? 2 : 1;    // key groups
+  constexpr int NW = QW / G;         // waves that fill a tile
   int tid = threadIdx.x;  // opaque, as in dkdv_block
   asm volatile("" : "+v"(tid));
   const int lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = wave / NW, wl = wave % NW;
+  bf16_t *K0 = KV + grp * 4 * TILE, *V0 = K0 + TILE, *K1 = K0 + 2 * TILE, *V1 = K0 + 3 * TILE;
   const int n = a.n;
   const BhRows m = bh_rows(a, bh);
-  const int q0 = qb * BM, qw = q0 + wave * 32, my_q = qw + l32;
+  const int q0 = qb * BM, qw = q0 + wl * 32, my_q = qw + l32;
   const int qc = min(my_q, n - 1);
 
   u32x4 qf[8], df[8];
@@ -894,10 +1008,10 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, int bh, int qb, bf16
 
   const int kend = min(q0 + BM, n);
   const int nt = (kend + BN - 1) / BN;
-  int rr[16 / QW];
-  load_rows<QW>(rr, m, 0, wave, lane);
-  issue_rows<QW>(K0, m.k, m.kp, V0, m.v, m.vp, m, rr, wave, lane);
-  load_rows<QW>(rr, m, BN, wave, lane);
+  int rr[16 / NW];
+  load_rows<NW>(rr, m, grp * BN, wl, lane);
+  issue_rows<NW>(K0, m.k, m.kp, V0, m.v, m.vp, m, rr, wl, lane);
+  load_rows<NW>(rr, m, (G + grp) * BN, wl, lane);
   // key sample for the centre: thread t reads 16 bytes (dims 8 (t % 16) ..) of
   // sample rows t / 16 and t / 16 + 32, sample s at key (s kend) / 64
   u32x4 ks0, ks1;
@@ -969,27 +1083,53 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, int bh, int qb, bf16
   float rsum = 0.f;
   const int nfull = min((qw + 1) / BN, n / BN);
 
+  // step j: key tile G j + grp
   auto step = [&](auto C, int j, const bf16_t* Ks, const bf16_t* Vs, bf16_t* Kn, bf16_t* Vn) {
-    const int k0 = j * BN;
-    if (j + 1 < nt) issue_rows<QW>(Kn, m.k, m.kp, Vn, m.v, m.vp, m, rr, wave, lane);
-    if (j + 2 < nt) load_rows<QW>(rr, m, k0 + 2 * BN, wave, lane);
-    if (j < nt && k0 <= qw + 31)
-      dq_tile<T, decltype(C)::value>(acc, rsum, qf, df, Ks, Vs, k0, my_q, n, lane, a.sl2, nlse, dlt, j >= nfull);
+    const int t = G * j + grp, k0 = t * BN;
+    if (t + G < nt) issue_rows<NW>(Kn, m.k, m.kp, Vn, m.v, m.vp, m, rr, wl, lane);
+    if (t + 2 * G < nt) load_rows<NW>(rr, m, k0 + 2 * G * BN, wl, lane);
+    if (t < nt && k0 <= qw + 31)
+      dq_tile<T, decltype(C)::value>(acc, rsum, qf, df, Ks, Vs, k0, my_q, n, lane, a.sl2, nlse, dlt, t >= nfull);
     wait_loads();
     __syncthreads();
   };
+  const int ns = (nt + G - 1) / G;
   if (ctr) {
-    for (int j = 0; j < nt; j += 2) {
+    for (int j = 0; j < ns; j += 2) {
       step(std::true_type{}, j, K0, V0, K1, V1);
       step(std::true_type{}, j + 1, K1, V1, K0, V0);
     }
   } else {
-    for (int j = 0; j < nt; j += 2) {
+    for (int j = 0; j < ns; j += 2) {
       step(std::false_type{}, j, K0, V0, K1, V1);
       step(std::false_type{}, j + 1, K1, V1, K0, V0);
     }
   }
 
+  if (HALF) {  // the odd tiles' sums -> LDS (register order) -> the even tiles' waves
+    float4* ax = reinterpret_cast<float4*>(KV) + wl * 1024 + ln;
+    if (grp) {
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          ax[(4 * d + g) * 64] = float4{acc[d][4 * g], acc[d][4 * g + 1], acc[d][4 * g + 2], acc[d][4 * g + 3]};
+      kcp[wl * 64 + ln] = rsum;
+    }
+    __syncthreads();
+    if (grp) return;
+    rsum += kcp[wl * 64 + ln];
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float4 x = ax[(4 * d + g) * 64];
+        acc[d][4 * g + 0] += x.x;
+        acc[d][4 * g + 1] += x.y;
+        acc[d][4 * g + 2] += x.z;
+        acc[d][4 * g + 3] += x.w;
+      }
+  }
   // the two lane halves hold the two halves of each row's keys
   rsum += __shfl_xor(rsum, 32);
   if (my_q >= n) return;
@@ -1014,10 +1154,7 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, int bh, int qb, bf16
 
 template <typename T>
 __global__ __launch_bounds__(64 * QW, 8 / QW) void attn_bwd_dq_kernel(const AttnArgs a, const QPlan p, const WorkQ q) {
-  __shared__ __attribute__((aligned(1024))) bf16_t K0[TILE];
-  __shared__ __attribute__((aligned(1024))) bf16_t K1[TILE];
-  __shared__ __attribute__((aligned(1024))) bf16_t V0[TILE];
-  __shared__ __attribute__((aligned(1024))) bf16_t V1[TILE];
+  __shared__ __attribute__((aligned(1024))) bf16_t KV[4 * TILE];
   __shared__ __attribute__((aligned(16))) float KC[128 + QW * 132];  // key centre + per-wave partial sums
   __shared__ int wq_s[2];
   int bh, qb, bin = 0;
@@ -1030,12 +1167,26 @@ __global__ __launch_bounds__(64 * QW, 8 / QW) void attn_bwd_dq_kernel(const Attn
     if (!have && q.ctr) have = wq_next(q, a.nq, a.BH, true, -1, 0, bh, qb, wq_s);
   }
   for (int k = 1; have; ++k) {
-    dq_block<T>(a, bh, qb, K0, K1, V0, V1, KC);
+    dq_block<T, false>(a, bh, qb, KV, KC);
     // the next block starts after this one's last tile reads
     if (p.bph)
       have = plan_next(p, bin, k, qb);
     else
       have = q.ctr && wq_next(q, a.nq, a.BH, true, -1, k, bh, qb, wq_s);
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(64 * QW, 8 / QW) void attn_bwd_dq_half_kernel(const AttnArgs a, const WorkQ q) {
+  __shared__ __attribute__((aligned(1024))) bf16_t KV[8 * TILE];
+  __shared__ __attribute__((aligned(16))) float KC[128 + QW * 132];
+  __shared__ int wq_s[2];
+  int bh, qb;
+  bool have = wq_first(q, a.nq, a.BH, true, bh, qb);
+  if (!have && q.ctr) have = wq_next(q, a.nq, a.BH, true, -1, 0, bh, qb, wq_s);
+  for (int k = 1; have; ++k) {
+    dq_block<T, true>(a, bh, qb, KV, KC);
+    have = q.ctr && wq_next(q, a.nq, a.BH, true, -1, k, bh, qb, wq_s);
   }
 }
 
@@ -2037,6 +2188,26 @@ int wq_grid(int nblk, int BH, hipStream_t st, WorkQ& q) {
   return cus;
 }
 
+// Whether a query-stationary launch over BH (b, h) of length n runs half blocks
+// (fwd_half_block).  Both ways are estimated in units of 10 ns, with measured
+// constants: a step costs 1.57 us (one tile of 256 queries) or 2.07 us (two of
+// 128) while most of the chip idles, which bounds a launch by its heaviest
+// block, and 2.25 or 2.55 us when all CUs run, plus 7 us for each block of a CU
+// in turn, which bounds it by its share of the whole work.  Half blocks are
+// taken when they are estimated 5% shorter; the estimate is within 10% of the
+// measured time on both sides for 8 to 36 heads of 1152 to 18432 rows.
+bool half_blocks(int BH, int n) {
+  const int cus = cu_count();
+  if (cus <= 0) return false;
+  auto est = [&](int rows, int tiles_per_step, int chain, int load) {
+    const long long nb = (n + rows - 1) / rows, per = (long long)rows / BN / tiles_per_step;
+    const long long heavy = ((n + BN - 1) / BN + tiles_per_step - 1) / tiles_per_step;
+    const long long steps = per * nb * (nb - 1) / 2 + heavy;
+    return std::max(heavy * chain + 700, BH * (steps * load + nb * 700) / cus);
+  };
+  return est(HB, 2, 207, 255) * 105 < est(32 * QW, 1, 157, 225) * 100;
+}
+
 // Grid of a query-stationary launch: a packed plan where one applies, else as wq_grid.
 int query_grid(int BH, int n, hipStream_t st, QPlan& p, WorkQ& q) {
   const int grid = make_plan(BH, n, p);
@@ -2047,33 +2218,41 @@ int query_grid(int BH, int n, hipStream_t st, QPlan& p, WorkQ& q) {
 
 }  // namespace
 
-extern "C" int lh_attn_fwd(const void* q, const void* k, const void* v, int64_t sb, int64_t ss, int64_t sh,
-                           const void* qp, const void* kp, const void* vp, int64_t pb, int64_t ps, int64_t ph,
-                           int split, const int32_t* indices, int B, int H, int n, int D, float scale, void* out,
-                           float* lse, int dtype, void* stream) {
+namespace {
+int attn_fwd_impl(const void* q, const void* k, const void* v, int64_t sb, int64_t ss, int64_t sh, const void* qp,
+                  const void* kp, const void* vp, int64_t pb, int64_t ps, int64_t ph, int split,
+                  const int32_t* indices, int B, int H, int n, int D, float scale, void* out, float* lse, int dtype,
+                  int flags, void* stream) {
   AttnArgs a{};
   int rc = fill_rows(a, q, k, v, sb, ss, sh, qp, kp, vp, pb, ps, ph, split, indices, B, H, n, D, scale);
   if (rc) return rc;
-  if (!out || !lse || !al16(out) || !valid_dtype(dtype)) return LH_ERR_INVALID_ARG;
+  if (!out || !lse || !al16(out) || !valid_dtype(dtype) || (flags & ~LH_ATTN_SHAPED)) return LH_ERR_INVALID_ARG;
   a.out = (bf16_t*)out; a.lse = lse;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   QPlan p;
   WorkQ wq;
-  const int grid = query_grid(a.BH, a.n, st, p, wq);
-  LH_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((attn_fwd_kernel<T, 0>), dim3(grid), dim3(64 * QW), 0, st, a, p, wq));
+  if ((flags & LH_ATTN_SHAPED) && half_blocks(a.BH, n)) {
+    a.nq = (n + HB - 1) / HB;
+    const int grid = wq_grid(a.nq, a.BH, st, wq);
+    LH_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL(attn_fwd_half_kernel<T>, dim3(grid), dim3(64 * QW), 0, st, a, wq));
+  } else {
+    const int grid = query_grid(a.BH, a.n, st, p, wq);
+    LH_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((attn_fwd_kernel<T, 0>), dim3(grid), dim3(64 * QW), 0, st, a, p, wq));
+  }
   LH_CHECK_LAUNCH();
   return LH_OK;
 }
 
-namespace {
 // parts: bit 0 = dK/dV kernel, bit 1 = dQ kernel
 int attn_bwd_parts(int parts, const void* q, const void* k, const void* v, int64_t sb, int64_t ss, int64_t sh,
                    const void* qp, const void* kp, const void* vp, int64_t pb, int64_t ps, int64_t ph, int split,
                    const int32_t* indices, int B, int H, int n, int D, float scale, const void* dout,
-                   const float* lse, const float* delta, void* dq, void* dk, void* dv, int dtype, void* stream) {
+                   const float* lse, const float* delta, void* dq, void* dk, void* dv, int dtype, int flags,
+                   void* stream) {
   AttnArgs a{};
   int rc = fill_rows(a, q, k, v, sb, ss, sh, qp, kp, vp, pb, ps, ph, split, indices, B, H, n, D, scale);
   if (rc) return rc;
+  if (parts < 1 || parts > 3 || (flags & ~LH_ATTN_SHAPED)) return LH_ERR_INVALID_ARG;
   if (!dout || !lse || !delta || !al16(dout) || !valid_dtype(dtype)) return LH_ERR_INVALID_ARG;
   if (indices && n < 8) return LH_ERR_UNSUPPORTED;  // gathered rows are indexed 8 at a time
   if ((parts & 1) && (!dk || !dv || !al16(dk) || !al16(dv))) return LH_ERR_INVALID_ARG;
@@ -2095,30 +2274,62 @@ int attn_bwd_parts(int parts, const void* q, const void* k, const void* v, int64
   if (parts & 2) {
     QPlan p;
     WorkQ wq;
-    const int grid = query_grid(a.BH, a.n, st, p, wq);
-    LH_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL(attn_bwd_dq_kernel<T>, dim3(grid), dim3(64 * QW), 0, st, a, p, wq));
+    if ((flags & LH_ATTN_SHAPED) && half_blocks(a.BH, n)) {
+      a.nq = (n + HB - 1) / HB;
+      const int grid = wq_grid(a.nq, a.BH, st, wq);
+      LH_DISPATCH_DTYPE(dtype,
+                        hipLaunchKernelGGL(attn_bwd_dq_half_kernel<T>, dim3(grid), dim3(64 * QW), 0, st, a, wq));
+    } else {
+      const int grid = query_grid(a.BH, a.n, st, p, wq);
+      LH_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL(attn_bwd_dq_kernel<T>, dim3(grid), dim3(64 * QW), 0, st, a, p, wq));
+    }
     LH_CHECK_LAUNCH();
   }
   return LH_OK;
 }
 }  // namespace
 
+extern "C" int lh_attn_fwd(const void* q, const void* k, const void* v, int64_t sb, int64_t ss, int64_t sh,
+                           const void* qp, const void* kp, const void* vp, int64_t pb, int64_t ps, int64_t ph,
+                           int split, const int32_t* indices, int B, int H, int n, int D, float scale, void* out,
+                           float* lse, int dtype, void* stream) {
+  return attn_fwd_impl(q, k, v, sb, ss, sh, qp, kp, vp, pb, ps, ph, split, indices, B, H, n, D, scale, out, lse, dtype,
+                       0, stream);
+}
+
+extern "C" int lh_attn_fwd_ex(const void* q, const void* k, const void* v, int64_t sb, int64_t ss, int64_t sh,
+                              const void* qp, const void* kp, const void* vp, int64_t pb, int64_t ps, int64_t ph,
+                              int split, const int32_t* indices, int B, int H, int n, int D, float scale, void* out,
+                              float* lse, int dtype, int flags, void* stream) {
+  return attn_fwd_impl(q, k, v, sb, ss, sh, qp, kp, vp, pb, ps, ph, split, indices, B, H, n, D, scale, out, lse, dtype,
+                       flags, stream);
+}
+
 extern "C" int lh_attn_bwd(const void* q, const void* k, const void* v, int64_t sb, int64_t ss, int64_t sh,
                            const void* qp, const void* kp, const void* vp, int64_t pb, int64_t ps, int64_t ph,
-                           int split, const int32_t* indices, int B, int H, int n, int D, float scale,
-                           const void* dout, const float* lse, const float* delta, void* dq, void* dk, void* dv,
-                           int dtype, void* stream) {
-  return attn_bwd_parts(3, q, k, v, sb, ss, sh, qp, kp, vp, pb, ps, ph, split, indices, B, H, n, D, scale, dout,
-                        lse, delta, dq, dk, dv, dtype, stream);
+                           int split, const int32_t* indices, int B, int H, int n, int D, float scale, const void* dout,
+                           const float* lse, const float* delta, void* dq, void* dk, void* dv, int dtype,
+                           void* stream) {
+  return attn_bwd_parts(3, q, k, v, sb, ss, sh, qp, kp, vp, pb, ps, ph, split, indices, B, H, n, D, scale, dout, lse,
+                        delta, dq, dk, dv, dtype, 0, stream);
+}
+
+extern "C" int lh_attn_bwd_ex(int parts, const void* q, const void* k, const void* v, int64_t sb, int64_t ss,
+                              int64_t sh, const void* qp, const void* kp, const void* vp, int64_t pb, int64_t ps,
+                              int64_t ph, int split, const int32_t* indices, int B, int H, int n, int D, float scale,
+                              const void* dout, const float* lse, const float* delta, void* dq, void* dk, void* dv,
+                              int dtype, int flags, void* stream) {
+  return attn_bwd_parts(parts, q, k, v, sb, ss, sh, qp, kp, vp, pb, ps, ph, split, indices, B, H, n, D, scale, dout,
+                        lse, delta, dq, dk, dv, dtype, flags, stream);
 }
 
 extern "C" int lh_attn_bwd_dkdv(const void* q, const void* k, const void* v, int64_t sb, int64_t ss, int64_t sh,
                                 const void* qp, const void* kp, const void* vp, int64_t pb, int64_t ps, int64_t ph,
                                 int split, const int32_t* indices, int B, int H, int n, int D, float scale,
-                                const void* dout, const float* lse, const float* delta, void* dk, void* dv,
-                                int dtype, void* stream) {
-  return attn_bwd_parts(1, q, k, v, sb, ss, sh, qp, kp, vp, pb, ps, ph, split, indices, B, H, n, D, scale, dout,
-                        lse, delta, nullptr, dk, dv, dtype, stream);
+                                const void* dout, const float* lse, const float* delta, void* dk, void* dv, int dtype,
+                                void* stream) {
+  return attn_bwd_parts(1, q, k, v, sb, ss, sh, qp, kp, vp, pb, ps, ph, split, indices, B, H, n, D, scale, dout, lse,
+                        delta, nullptr, dk, dv, dtype, 0, stream);
 }
 
 extern "C" int lh_attn_bwd_dq(const void* q, const void* k, const void* v, int64_t sb, int64_t ss, int64_t sh,
@@ -2126,8 +2337,8 @@ extern "C" int lh_attn_bwd_dq(const void* q, const void* k, const void* v, int64
                               int split, const int32_t* indices, int B, int H, int n, int D, float scale,
                               const void* dout, const float* lse, const float* delta, void* dq, int dtype,
                               void* stream) {
-  return attn_bwd_parts(2, q, k, v, sb, ss, sh, qp, kp, vp, pb, ps, ph, split, indices, B, H, n, D, scale, dout,
-                        lse, delta, dq, nullptr, nullptr, dtype, stream);
+  return attn_bwd_parts(2, q, k, v, sb, ss, sh, qp, kp, vp, pb, ps, ph, split, indices, B, H, n, D, scale, dout, lse,
+                        delta, dq, nullptr, nullptr, dtype, 0, stream);
 }
 
 extern "C" int lh_attn_status(int* faults) {

@@ -36,7 +36,7 @@ class _DenseCausalFn(torch.autograd.Function):
     def forward(ctx, q, k, v, scale):
         B, H, S, D = q.shape
         _mark("dense_fwd_start")
-        o, lse = N.attn_fwd(_rows(q, k, v), None, B, H, S, D, scale)
+        o, lse = N.attn_fwd(_rows(q, k, v), None, B, H, S, D, scale, shaped=True)
         _mark("dense_attn_fwd")
         ctx.save_for_backward(q, k, v, o, lse)
         ctx.scale = scale
@@ -50,7 +50,7 @@ class _DenseCausalFn(torch.autograd.Function):
         # softmax-backward row term delta = rowsum(dO * O), accumulated in fp32
         delta = torch.linalg.vecdot(do.float(), o.float())
         _mark("dense_bwd_start")
-        dq, dk, dv = N.attn_bwd(_rows(q, k, v), None, B, H, S, do, lse, delta, D, ctx.scale)
+        dq, dk, dv = N.attn_bwd(_rows(q, k, v), None, B, H, S, do, lse, delta, D, ctx.scale, shaped=True)
         _mark("dense_attn_bwd")
         return dq, dk, dv, None
 

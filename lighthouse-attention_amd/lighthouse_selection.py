@@ -145,7 +145,7 @@ def _layer_fwd(xq, xk, xv, L, p, topk, tie, strict, dilation, seq_major, gk=None
     idx, inv = N.select_topk(sqk, skq, S, L, p, topk, tie=tie, strict=strict)
     _mark("select")
     rows = _base_rows(xq, xk, xv, pq, pk, pv)
-    o, lse = N.attn_fwd(rows, idx, B, H, S_sel, D, scale)
+    o, lse = N.attn_fwd(rows, idx, B, H, S_sel, D, scale, shaped=True)
     _mark("attn_fwd")
     out = N.scatter_fwd(o, inv, S, S, L, p, seq_major=seq_major)
     _mark("scatter_fwd")
@@ -172,7 +172,7 @@ def _attn_bwd_pair(rows, idx, B, H, S_sel, dattn, lse, delta, D, scale=None):
     if _bwd_streams < 2 or torch.compiler.is_compiling():
         dks, dvs = N.attn_bwd_dkdv(rows, idx, B, H, S_sel, dattn, lse, delta, D, scale)
         _mark("attn_bwd_dkdv")
-        dqs = N.attn_bwd_dq(rows, idx, B, H, S_sel, dattn, lse, delta, D, scale)
+        dqs = N.attn_bwd_dq(rows, idx, B, H, S_sel, dattn, lse, delta, D, scale, shaped=True)
         _mark("attn_bwd_dq")
         return dqs, dks, dvs
     dev = dattn.device
@@ -183,7 +183,7 @@ def _attn_bwd_pair(rows, idx, B, H, S_sel, dattn, lse, delta, D, scale=None):
     side.wait_stream(main)  # dattn, delta (and everything before) are ready
     with torch.cuda.stream(side):
         _mark("side_start")
-        dqs = N.attn_bwd_dq(rows, idx, B, H, S_sel, dattn, lse, delta, D, scale)
+        dqs = N.attn_bwd_dq(rows, idx, B, H, S_sel, dattn, lse, delta, D, scale, shaped=True)
         _mark("attn_bwd_dq")
     dks, dvs = N.attn_bwd_dkdv(rows, idx, B, H, S_sel, dattn, lse, delta, D, scale)
     _mark("attn_bwd_dkdv")
@@ -298,7 +298,7 @@ def _rope_layer_fwd(xqkv, freqs, H, L, p, topk, tie, strict, seq_major):
     idx, inv = N.select_topk(sqk, skq, S, L, p, topk, tie=tie, strict=strict)
     _mark("select")
     rows = _rope_rows(xqkv, xr, H, D, pq, pk, pv)
-    o, lse = N.attn_fwd(rows, idx, B, H, S_sel, D)
+    o, lse = N.attn_fwd(rows, idx, B, H, S_sel, D, shaped=True)
     _mark("attn_fwd")
     out = N.scatter_fwd(o, inv, S, S, L, p, seq_major=seq_major)
     _mark("scatter_fwd")
@@ -557,7 +557,7 @@ class _GatheredAttnFn(torch.autograd.Function):
         D = q_cat.shape[-1]
         rows = _GatheredAttnFn._rows(q_cat, k_cat, v_cat)
         n = idx.shape[-1]
-        o, lse = N.attn_fwd(rows, idx, B, H, n, D, scale)
+        o, lse = N.attn_fwd(rows, idx, B, H, n, D, scale, shaped=True)
         ctx.save_for_backward(q_cat, k_cat, v_cat, idx, o, lse)
         ctx.geo = (D0, scale)
         return o[..., :D0] if D0 < D else o
@@ -573,7 +573,7 @@ class _GatheredAttnFn(torch.autograd.Function):
         if D0 < D:
             do = torch.nn.functional.pad(do, (0, D - D0))
         delta = (do.float() * o.float()).sum(-1)
-        dqs, dks, dvs = N.attn_bwd(rows, idx, B, H, n, do, lse, delta, D, scale)
+        dqs, dks, dvs = N.attn_bwd(rows, idx, B, H, n, do, lse, delta, D, scale, shaped=True)
         inv = N.build_inverse(idx, S_tot)
         # one-level pyramid over S_tot rows: row r receives dsel[inv[r]] (or 0)
         dq, dk, dv = N.pyramid_bwd(dqs, dks, dvs, inv, B, S_tot, H, 1, 2, D)
