@@ -10,7 +10,7 @@
  *   - returns LH_OK (0) or an LH_ERR_* code (lh_strerror() names it); argument
  *     errors are detected on the host before any launch.
  *
- * Layouts (B batch, S base length, H heads, D = 128 head dim, p pooling
+ * Layouts (B batch, S base length, H heads, D head dim, p pooling
  * factor, L levels, S_tot = sum_l S/p^(l-1), Sp = S_tot - S, n = selected
  * length):
  *   base rows     bf16 [B, S, H, D]   (the model's xq/xk/xv, post-RoPE)
@@ -20,6 +20,10 @@
  *   inverse       int32 [B, H, S_tot] position in the selected sequence or -1
  *   selected rows bf16 [B, H, n, D];  lse / delta fp32 [B, H, n]
  *   layer output  bf16 [B, H, S, D]
+ * D, a multiple of 8: 8..96 and 128 in the attention and dilated-scorer entry
+ * points, 8..128 in the pyramid, fan-out and their adjoints, 128 in the GLA
+ * scorer and the entry points with a rotary embedding (other head dims there
+ * run zero-padded by the caller with the scale of their own width).
  *
  * Citations are to the reference repository (ighoshsubho/lighthouse-attention).
  */
@@ -36,7 +40,7 @@ extern "C" {
 #define LH_ERR_INVALID_ARG 1  /* bad size, null pointer or unsupported shape */
 #define LH_ERR_DOMAIN 2       /* geometry the reference asserts on or overruns (strict mode) */
 #define LH_ERR_LAUNCH 3       /* the HIP runtime refused a launch */
-#define LH_ERR_UNSUPPORTED 4  /* shape beyond this build's limits (e.g. D != 128) */
+#define LH_ERR_UNSUPPORTED 4  /* shape beyond this build's limits (see D below) */
 #define LH_ERR_RUNTIME 5      /* a HIP runtime call (synchronize, copy, symbol lookup) failed */
 
 /* The ABI this header declares; lh_abi_version() of a matching library returns it. */

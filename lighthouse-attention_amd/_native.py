@@ -21,6 +21,33 @@ LIB_PATH = os.path.join(_HERE, "liblighthouse_hip.so")
 CSRC = os.path.join(_HERE, "csrc")
 D_SUPPORTED = 128
 
+
+def padded_dim(D: int) -> int:
+    """Width a head dim D (a multiple of 8, at most 128) runs at: its own up to 96, else
+    128 with zero columns (no attention layout between the two)."""
+    return D if D <= 96 else D_SUPPORTED
+
+
+def own_rows(x):
+    """``x`` contiguous and, for head dims below 128, on a 16-byte boundary (copied if
+    it is not; 128-wide rows off the boundary are refused by the library)."""
+    x = x.contiguous()
+    return x.clone() if x.shape[-1] < D_SUPPORTED and x.data_ptr() % 16 else x
+
+
+def shared_rows(q, k, v):
+    """``q, k, v`` [B, H, S, D] as the attention kernels read them: with D < 128 each is
+    copied unless all three share strides that are multiples of 8 elements (D
+    contiguous, row offsets within 32 bits) and start on 16-byte boundaries.  128-wide
+    rows pass as they are; their misfits are refused."""
+    D = q.shape[-1]
+    if D == D_SUPPORTED:
+        return q, k, v
+    st = q.stride()
+    fit = st[3] == 1 and st[2] > 0 and not any(s % 8 for s in st[:3]) and q.shape[2] * st[2] + D_SUPPORTED < 2 ** 31 \
+        and all(x.stride() == st and x.data_ptr() % 16 == 0 for x in (q, k, v))
+    return (q, k, v) if fit else tuple(own_rows(x) for x in (q, k, v))
+
 TIE_MODES = {"reference": 0, "lower_index": 1}
 
 _lib = None
@@ -572,7 +599,7 @@ def scatter_bwd(dout, indices, o, S: int, L: int, p: int):
     if _check_mode():
         check_indices(indices, 0, pyramid_lengths(S, L, p)[2], unique=True, what="scatter_bwd indices")
     if dout.stride(3) != 1 or any(st % 8 for st in dout.stride()[:3]) or dout.data_ptr() % 16:
-        dout = dout.contiguous()
+        dout = own_rows(dout)
     B, H, S_out, D = dout.shape
     n = indices.shape[-1]
     dattn = torch.empty(B, H, n, D, dtype=dout.dtype, device=dout.device)

@@ -6,7 +6,7 @@
 
 #include "../../include/lighthouse_hip.h"
 
-#define LH_D 128  // head dimension supported by every kernel in this library
+#define LH_D 128  // widest head dimension; D below it: see Lanes
 
 typedef uint16_t bf16_t;  // bfloat16 storage
 typedef __bf16 bf16x8 __attribute__((__vector_size__(8 * sizeof(__bf16))));
@@ -87,6 +87,31 @@ __device__ __forceinline__ uint4 pack8_t(const float* f) {
   v.z = T::pack2(f[4], f[5]); v.w = T::pack2(f[6], f[7]);
   return v;
 }
+
+// Lanes of the streaming row kernels: LPR lanes own a row, 8 elements each.  A
+// head dim D up to 64 takes 8 lanes, a wider one 16; FULL: D is exactly 8 LPR,
+// otherwise the lanes past D hold zeros and store nothing.
+template <int LPR_, bool FULL_>
+struct Lanes {
+  static constexpr int LPR = LPR_;
+  static constexpr bool FULL = FULL_;
+  static constexpr int ROWS = 256 / LPR;  // rows of a 256-thread block
+  __device__ static __forceinline__ bool in(int l, int D) { return FULL || 8 * l < D; }
+};
+#define LH_DISPATCH_LANES(D, ...)      \
+  do {                                 \
+    if ((D) == LH_D) {                 \
+      using Ln = Lanes<16, true>;      \
+      __VA_ARGS__;                     \
+    } else if ((D) > 64) {             \
+      using Ln = Lanes<16, false>;     \
+      __VA_ARGS__;                     \
+    } else {                           \
+      using Ln = Lanes<8, false>;      \
+      __VA_ARGS__;                     \
+    }                                  \
+  } while (0)
+static inline bool lanes_supported(int D) { return D > 0 && D <= LH_D && D % 8 == 0; }
 
 // Launch helper: F(tag) for the element type named by a dtype code.
 #define LH_DISPATCH_DTYPE(dtype, ...)                         \

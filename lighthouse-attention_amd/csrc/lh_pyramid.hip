@@ -6,7 +6,7 @@
 // rows; level j = 1..L-1 rows are
 // the means of p^j consecutive base rows (fp32 sum, one rounding), and level-j
 // scores are maxima of the base scores over the same span.  One pass streams
-// xq/xk/xv once: 16 lanes own one (b, span, head) unit, 8 bf16 each, and walk
+// xq/xk/xv once: 16 lanes (8 for D <= 64) own one (b, span, head) unit, 8 bf16 each, and walk
 // the p^(L-1) base tokens of the span.  Base rows are never copied: pooled rows
 // go to a separate [B, Sp, H, D] buffer.
 //
@@ -27,7 +27,7 @@ struct PyrArgs {
   const float* fs;   // rotary (cos, sin) table [>= S, D/2, 2] (ROPE)
   bf16_t *rq, *rk;   // rotated base rows out (ROPE)
   int64_t rb, rs, rh;
-  int B, S, H, L, shift, S_tot, nspan, cmax, units;
+  int B, S, H, D, L, shift, S_tot, nspan, cmax, units;
   int off[9], len[9];
 };
 
@@ -38,9 +38,9 @@ constexpr int PYR_CHUNK = 4;  // base tokens whose loads are issued together
 // One base token t of (b, h): unpack the 16-byte slices of its q, k, v rows,
 // rotate q and k (ROPE: rounded to bf16 and stored to rq / rk, the rounded
 // values kept), and make its base scores: the bf16-rounded L2 norms of q and k
-// (every lane of the 16-lane group gets them), or the given ones (GIVEN: sq, sk
+// (every lane of the row's group gets them), or the given ones (GIVEN: sq, sk
 // on entry).
-template <typename T, bool GIVEN, bool ROPE>
+template <typename T, typename Ln, bool GIVEN, bool ROPE>
 __device__ __forceinline__ void pyr_token(const PyrArgs& a, int b, int h, int l16, size_t srow, int t,
                                           const uint4 xq, const uint4 xk, const uint4 xv, float* fq, float* fk,
                                           float* fv, float& sq, float& sk) {
@@ -64,7 +64,7 @@ __device__ __forceinline__ void pyr_token(const PyrArgs& a, int b, int h, int l1
 #pragma unroll
     for (int e = 0; e < 8; ++e) { pq = fmaf(fq[e], fq[e], pq); pk = fmaf(fk[e], fk[e], pk); }
 #pragma unroll
-    for (int m = 1; m < 16; m <<= 1) { pq += __shfl_xor(pq, m, 16); pk += __shfl_xor(pk, m, 16); }
+    for (int m = 1; m < Ln::LPR; m <<= 1) { pq += __shfl_xor(pq, m, Ln::LPR); pk += __shfl_xor(pk, m, Ln::LPR); }
     sq = round_to<T>(sqrtf(pq));
     sk = round_to<T>(sqrtf(pk));
   }
@@ -74,11 +74,12 @@ __device__ __forceinline__ void pyr_token(const PyrArgs& a, int b, int h, int l1
 // position's angles, rounded to bf16 and written to rq / rk, and the norms and
 // means below are taken of those rounded rows, exactly as if the rotated rows
 // had been stored first and read back.
-template <typename T, int NL, bool GIVEN, bool ROPE>
+template <typename T, typename Ln, int NL, bool GIVEN, bool ROPE>
 __global__ __launch_bounds__(256) void pyramid_fwd_kernel(const PyrArgs a) {
   const int tid = threadIdx.x;
-  const int u = blockIdx.x * 16 + (tid >> 4);
-  const int l16 = tid & 15;
+  const int u = blockIdx.x * Ln::ROWS + tid / Ln::LPR;
+  const int l16 = tid % Ln::LPR;
+  const bool in = Ln::in(l16, a.D);
   if (u >= a.units) return;
   const int h = u % a.H;
   const int rest = u / a.H;
@@ -102,13 +103,13 @@ __global__ __launch_bounds__(256) void pyramid_fwd_kernel(const PyrArgs a) {
   auto token = [&](int t, const uint4 xq, const uint4 xk, const uint4 xv, float sq, float sk)
       __attribute__((always_inline)) {
     float fq[8], fk[8], fv[8];
-    pyr_token<T, GIVEN, ROPE>(a, b, h, l16, srow, t, xq, xk, xv, fq, fk, fv, sq, sk);
+    pyr_token<T, Ln, GIVEN, ROPE>(a, b, h, l16, srow, t, xq, xk, xv, fq, fk, fv, sq, sk);
     if (!GIVEN) {
-      // base scores leave 16 tokens at a time: lane j keeps token t0 + 16 i + j,
-      // and the group stores them as one contiguous 64-byte run per tensor
-      const int j = (t - t0) & 15;
+      // base scores leave LPR tokens at a time: lane j keeps token t0 + LPR i + j,
+      // and the group stores them as one contiguous run per tensor
+      const int j = (t - t0) & (Ln::LPR - 1);
       if (l16 == j) { bq = sq; bk = sk; }
-      if ((j == 15 || t == t1 - 1) && l16 <= j) {
+      if ((j == Ln::LPR - 1 || t == t1 - 1) && l16 <= j) {
         a.sqk[srow + t - j + l16] = bq;
         a.skq[srow + t - j + l16] = bk;
       }
@@ -128,13 +129,13 @@ __global__ __launch_bounds__(256) void pyramid_fwd_kernel(const PyrArgs a) {
         const int64_t prow = (int64_t)b * a.pb + (int64_t)(a.off[lvl] - a.S + node) * a.ps + (int64_t)h * a.ph + 8 * l16;
 #pragma unroll
         for (int e = 0; e < 8; ++e) mo[e] = accq[l][e] * inv_c;
-        *reinterpret_cast<uint4*>(a.pq + prow) = pack8_t<T>(mo);
+        if (in) *reinterpret_cast<uint4*>(a.pq + prow) = pack8_t<T>(mo);
 #pragma unroll
         for (int e = 0; e < 8; ++e) mo[e] = acck[l][e] * inv_c;
-        *reinterpret_cast<uint4*>(a.pk + prow) = pack8_t<T>(mo);
+        if (in) *reinterpret_cast<uint4*>(a.pk + prow) = pack8_t<T>(mo);
 #pragma unroll
         for (int e = 0; e < 8; ++e) mo[e] = accv[l][e] * inv_c;
-        *reinterpret_cast<uint4*>(a.pv + prow) = pack8_t<T>(mo);
+        if (in) *reinterpret_cast<uint4*>(a.pv + prow) = pack8_t<T>(mo);
         if (l16 == 0) {
           a.sqk[srow + a.off[lvl] + node] = mq[l];
           a.skq[srow + a.off[lvl] + node] = mk[l];
@@ -148,6 +149,7 @@ __global__ __launch_bounds__(256) void pyramid_fwd_kernel(const PyrArgs a) {
   // Tokens in chunks of PYR_CHUNK with every load of a chunk issued before the
   // first is used, so a wave keeps PYR_CHUNK rows per tensor in flight instead
   // of one; tokens are still summed in order.
+  const uint4 zero = make_uint4(0, 0, 0, 0);
   int t = t0;
   for (; t + PYR_CHUNK <= t1; t += PYR_CHUNK) {
     uint4 cq[PYR_CHUNK], ck[PYR_CHUNK], cv[PYR_CHUNK];
@@ -155,9 +157,9 @@ __global__ __launch_bounds__(256) void pyramid_fwd_kernel(const PyrArgs a) {
 #pragma unroll
     for (int i = 0; i < PYR_CHUNK; ++i) {
       const int64_t o = xoff + (int64_t)(t + i) * a.ss;
-      cq[i] = ld16(a.xq + o);
-      ck[i] = ld16(a.xk + o);
-      cv[i] = ld16(a.xv + o);
+      cq[i] = in ? ld16(a.xq + o) : zero;
+      ck[i] = in ? ld16(a.xk + o) : zero;
+      cv[i] = in ? ld16(a.xv + o) : zero;
       gq[i] = GIVEN ? a.sqk[srow + t + i] : 0.f;
       gk[i] = GIVEN ? a.skq[srow + t + i] : 0.f;
     }
@@ -166,7 +168,7 @@ __global__ __launch_bounds__(256) void pyramid_fwd_kernel(const PyrArgs a) {
   }
   for (; t < t1; ++t) {
     const int64_t o = xoff + (int64_t)t * a.ss;
-    token(t, ld16(a.xq + o), ld16(a.xk + o), ld16(a.xv + o), GIVEN ? a.sqk[srow + t] : 0.f,
+    token(t, in ? ld16(a.xq + o) : zero, in ? ld16(a.xk + o) : zero, in ? ld16(a.xv + o) : zero, GIVEN ? a.sqk[srow + t] : 0.f,
           GIVEN ? a.skq[srow + t] : 0.f);
   }
 }
@@ -178,14 +180,14 @@ struct PyrBwdArgs {
   bf16_t *dq, *dk, *dv;
   int64_t ob, os, oh;  // strides of the three outputs (element units)
   const float* fs;     // ROPE: (cos, sin) table; dq, dk are rotated back by -theta
-  int B, S, H, L, shift, S_tot;
+  int B, S, H, D, L, shift, S_tot;
   int off[9], len[9];
   long long rows;
-  int chunks;  // 16-token chunks per (b, h)
+  int chunks;  // chunks of 16 (D <= 64: 32) tokens per (b, h)
 };
 
 // One 16-lane group per (b, t, h) row, 8 d each; a block covers 16 consecutive
-// tokens of one (b, h), so the rows of a pooled node spanning up to 16 tokens
+// tokens of one (b, h) (D <= 64: 8 lanes, 32 tokens), so the rows of a pooled node spanning up to 16 tokens
 // are read by one block (the wave or block coalesces the repeats instead of
 // several blocks fetching the row through L2), and runs of 32 consecutive
 // chunks of a head stay on one XCD (`xcd_run`; one whole head per XCD left the
@@ -195,14 +197,14 @@ struct PyrBwdArgs {
 // memory round trips instead of two per level.  ROPE: the q and k sums are
 // the gradients of rotated rows; they are rotated back (the adjoint of the
 // forward rotation) in fp32 before the one rounding.
-template <typename T, int NL, bool ROPE>
+template <typename T, typename Ln, int NL, bool ROPE>
 __global__ __launch_bounds__(256) void pyramid_bwd_kernel(const PyrBwdArgs a) {
   const int tid = threadIdx.x;
   const long long blk = xcd_run(blockIdx.x, gridDim.x, 32);
   const long long bh = blk / a.chunks;
-  const int t = (int)(blk - bh * a.chunks) * 16 + (tid >> 4);
-  const int l16 = tid & 15;
-  if (t >= a.S) return;
+  const int t = (int)(blk - bh * a.chunks) * Ln::ROWS + tid / Ln::LPR;
+  const int l16 = tid % Ln::LPR;
+  if (t >= a.S || !Ln::in(l16, a.D)) return;
   const int h = (int)(bh % a.H);
   const int b = (int)(bh / a.H);
   const size_t irow = (size_t)(b * a.H + h) * a.S_tot;
@@ -252,13 +254,19 @@ __global__ __launch_bounds__(256) void pyramid_bwd_kernel(const PyrBwdArgs a) {
 
 template <typename T, int NL>
 int launch_fwd(const PyrArgs& a, bool given, hipStream_t st) {
-  const int blocks = (a.units + 15) / 16;
-  if (a.fs)
-    hipLaunchKernelGGL((pyramid_fwd_kernel<BF16, NL, false, true>), dim3(blocks), dim3(256), 0, st, a);
-  else if (given)
-    hipLaunchKernelGGL((pyramid_fwd_kernel<T, NL, true, false>), dim3(blocks), dim3(256), 0, st, a);
-  else
-    hipLaunchKernelGGL((pyramid_fwd_kernel<T, NL, false, false>), dim3(blocks), dim3(256), 0, st, a);
+  if (a.fs) {  // D == LH_D
+    using Ln = Lanes<16, true>;
+    hipLaunchKernelGGL((pyramid_fwd_kernel<BF16, Ln, NL, false, true>), dim3((a.units + Ln::ROWS - 1) / Ln::ROWS),
+                       dim3(256), 0, st, a);
+  } else {
+    LH_DISPATCH_LANES(a.D, {
+      const dim3 grid((a.units + Ln::ROWS - 1) / Ln::ROWS);
+      if (given)
+        hipLaunchKernelGGL((pyramid_fwd_kernel<T, Ln, NL, true, false>), grid, dim3(256), 0, st, a);
+      else
+        hipLaunchKernelGGL((pyramid_fwd_kernel<T, Ln, NL, false, false>), grid, dim3(256), 0, st, a);
+    });
+  }
   LH_CHECK_LAUNCH();
   return LH_OK;
 }
@@ -274,7 +282,7 @@ int pyramid_fwd_impl(const void* xq, const void* xk, const void* xv, int64_t sb,
                      void* pq, void* pk, void* pv, int64_t pb, int64_t ps, int64_t ph,
                      float* scores_qk, float* scores_kq, int B, int S, int H, int D, int L, int p,
                      bool given, int dtype, void* stream) {
-  if (D != LH_D) return LH_ERR_UNSUPPORTED;
+  if (!lanes_supported(D) || (freqs && D != LH_D)) return LH_ERR_UNSUPPORTED;
   if (!valid_dtype(dtype) || (freqs && dtype != LH_DTYPE_BF16)) return LH_ERR_INVALID_ARG;
   if (!xq || !xk || !xv || !scores_qk || !scores_kq || B <= 0 || H <= 0 || S <= 0) return LH_ERR_INVALID_ARG;
   const int shift = ilog2_exact(p);
@@ -296,7 +304,7 @@ int pyramid_fwd_impl(const void* xq, const void* xk, const void* xv, int64_t sb,
   a.sqk = scores_qk; a.skq = scores_kq;
   a.fs = freqs; a.rq = (bf16_t*)rq; a.rk = (bf16_t*)rk;
   a.rb = rb; a.rs = rs; a.rh = rh;
-  a.B = B; a.S = S; a.H = H; a.L = L; a.shift = shift; a.S_tot = g.total;
+  a.B = B; a.S = S; a.H = H; a.D = D; a.L = L; a.shift = shift; a.S_tot = g.total;
   a.cmax = ipow(p, L - 1);
   if (a.cmax > 4096) return LH_ERR_UNSUPPORTED;
   a.nspan = (S + a.cmax - 1) / a.cmax;
@@ -317,25 +325,25 @@ int pyramid_fwd_impl(const void* xq, const void* xk, const void* xv, int64_t sb,
   return rc;
 }
 
-template <typename T, bool ROPE>
+template <typename T, typename Ln, bool ROPE>
 void launch_bwd(const PyrBwdArgs& a, dim3 grid, hipStream_t st) {
   const dim3 blk(256);
   switch (a.L) {
-    case 1: hipLaunchKernelGGL((pyramid_bwd_kernel<T, 1, ROPE>), grid, blk, 0, st, a); break;
-    case 2: hipLaunchKernelGGL((pyramid_bwd_kernel<T, 2, ROPE>), grid, blk, 0, st, a); break;
-    case 3: hipLaunchKernelGGL((pyramid_bwd_kernel<T, 3, ROPE>), grid, blk, 0, st, a); break;
-    case 4: hipLaunchKernelGGL((pyramid_bwd_kernel<T, 4, ROPE>), grid, blk, 0, st, a); break;
-    case 5: hipLaunchKernelGGL((pyramid_bwd_kernel<T, 5, ROPE>), grid, blk, 0, st, a); break;
-    case 6: hipLaunchKernelGGL((pyramid_bwd_kernel<T, 6, ROPE>), grid, blk, 0, st, a); break;
-    case 7: hipLaunchKernelGGL((pyramid_bwd_kernel<T, 7, ROPE>), grid, blk, 0, st, a); break;
-    default: hipLaunchKernelGGL((pyramid_bwd_kernel<T, 8, ROPE>), grid, blk, 0, st, a); break;
+    case 1: hipLaunchKernelGGL((pyramid_bwd_kernel<T, Ln, 1, ROPE>), grid, blk, 0, st, a); break;
+    case 2: hipLaunchKernelGGL((pyramid_bwd_kernel<T, Ln, 2, ROPE>), grid, blk, 0, st, a); break;
+    case 3: hipLaunchKernelGGL((pyramid_bwd_kernel<T, Ln, 3, ROPE>), grid, blk, 0, st, a); break;
+    case 4: hipLaunchKernelGGL((pyramid_bwd_kernel<T, Ln, 4, ROPE>), grid, blk, 0, st, a); break;
+    case 5: hipLaunchKernelGGL((pyramid_bwd_kernel<T, Ln, 5, ROPE>), grid, blk, 0, st, a); break;
+    case 6: hipLaunchKernelGGL((pyramid_bwd_kernel<T, Ln, 6, ROPE>), grid, blk, 0, st, a); break;
+    case 7: hipLaunchKernelGGL((pyramid_bwd_kernel<T, Ln, 7, ROPE>), grid, blk, 0, st, a); break;
+    default: hipLaunchKernelGGL((pyramid_bwd_kernel<T, Ln, 8, ROPE>), grid, blk, 0, st, a); break;
   }
 }
 
 int pyramid_bwd_impl(const void* gq, const void* gk, const void* gv, int64_t gb, int64_t gh, int64_t gs,
                      const int32_t* inverse, const float* freqs, void* dxq, void* dxk, void* dxv, int64_t ob,
                      int64_t os, int64_t oh, int B, int S, int H, int D, int L, int p, int dtype, void* stream) {
-  if (D != LH_D) return LH_ERR_UNSUPPORTED;
+  if (!lanes_supported(D) || (freqs && D != LH_D)) return LH_ERR_UNSUPPORTED;
   if (B <= 0 || H <= 0 || S <= 0 || L < 1 || L > 8) return LH_ERR_INVALID_ARG;
   if (!valid_dtype(dtype) || (freqs && dtype != LH_DTYPE_BF16)) return LH_ERR_INVALID_ARG;
   const int shift = ilog2_exact(p);
@@ -353,17 +361,18 @@ int pyramid_bwd_impl(const void* gq, const void* gk, const void* gv, int64_t gb,
   a.gb = gb; a.gh = gh; a.gs = gs; a.inv = inverse;
   a.dq = (bf16_t*)dxq; a.dk = (bf16_t*)dxk; a.dv = (bf16_t*)dxv;
   a.ob = ob; a.os = os; a.oh = oh; a.fs = freqs;
-  a.B = B; a.S = S; a.H = H; a.L = L; a.shift = shift; a.S_tot = g.total;
+  a.B = B; a.S = S; a.H = H; a.D = D; a.L = L; a.shift = shift; a.S_tot = g.total;
   for (int l = 1; l <= L; ++l) { a.off[l] = g.off[l]; a.len[l] = g.len[l]; }
   a.rows = (long long)B * S * H;
-  a.chunks = (S + 15) / 16;
+  const int rows = D <= 64 ? 32 : 16;
+  a.chunks = (S + rows - 1) / rows;
   const long long blocks = (long long)B * H * a.chunks;
   if (blocks > 2147483647LL) return LH_ERR_UNSUPPORTED;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (freqs)
-    launch_bwd<BF16, true>(a, dim3((unsigned)blocks), st);
+    launch_bwd<BF16, Lanes<16, true>, true>(a, dim3((unsigned)blocks), st);
   else
-    LH_DISPATCH_DTYPE(dtype, launch_bwd<T, false>(a, dim3((unsigned)blocks), st));
+    LH_DISPATCH_DTYPE(dtype, LH_DISPATCH_LANES(D, (launch_bwd<T, Ln, false>(a, dim3((unsigned)blocks), st))));
   LH_CHECK_LAUNCH();
   return LH_OK;
 }

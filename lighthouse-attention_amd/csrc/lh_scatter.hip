@@ -22,7 +22,7 @@ struct ScatArgs {
   bf16_t* dst;             // fwd: out, [b, h, t] at b*sb + h*sh + t*st;  bwd: dattn [BH, n, D]
   float* delta;            // bwd: [BH, n] (optional)
   int64_t sb, sh, st;      // element strides of the base-sequence tensor (D contiguous)
-  int H, S, S_out, n, L, shift, S_tot;
+  int H, D, S, S_out, n, L, shift, S_tot;
   int off[9], len[9];
   long long rows;
 };
@@ -38,20 +38,23 @@ __device__ __forceinline__ uint4 ld16(const bf16_t* p) { return *reinterpret_cas
 // span lengths (the adjoint's work) differ from head to head.
 constexpr int SCAT_RUN = 16;
 //
-// Forward: each 16-lane group owns SF_ROWS output rows (16 apart); all their
+// Forward: each 16-lane group (8 lanes for D <= 64) owns SF_ROWS output rows (a
+// block's groups apart); all their
 // levels' inverse lookups are issued first, then all row loads, so a group
 // has SF_ROWS * NL loads in flight across two dependent round trips.
 constexpr int SF_ROWS = 2;
-template <typename T, int NL, int R>
+template <typename T, typename Ln, int NL, int R>
 __global__ __launch_bounds__(256) void scatter_fwd_kernel(const ScatArgs a) {
   const int tid = threadIdx.x;
-  const int l16 = tid & 15;
-  const long long row0 = xcd_run(blockIdx.x, gridDim.x, SCAT_RUN) * (16 * R) + (tid >> 4);
+  const int l16 = tid % Ln::LPR;
+  const long long row0 = xcd_run(blockIdx.x, gridDim.x, SCAT_RUN) * (Ln::ROWS * R) + tid / Ln::LPR;
+  if (!Ln::in(l16, a.D)) return;
+  const int D = Ln::FULL ? 8 * Ln::LPR : a.D;
   int s[R][NL], tr[R];
   long long bhr[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const long long row = row0 + 16 * r;
+    const long long row = row0 + Ln::ROWS * r;
     const bool ok = row < a.rows;
     const long long bh = ok ? row / a.S_out : 0;
     const int t = ok ? (int)(row - bh * a.S_out) : 0;
@@ -67,10 +70,10 @@ __global__ __launch_bounds__(256) void scatter_fwd_kernel(const ScatArgs a) {
   uint4 v[R][NL];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const bf16_t* src = a.src + (size_t)bhr[r] * a.n * LH_D + 8 * l16;
+    const bf16_t* src = a.src + (size_t)bhr[r] * a.n * D + 8 * l16;
 #pragma unroll
     for (int l = 0; l < NL; ++l)
-      v[r][l] = s[r][l] >= 0 ? ld16(src + (size_t)s[r][l] * LH_D) : make_uint4(0, 0, 0, 0);
+      v[r][l] = s[r][l] >= 0 ? ld16(src + (size_t)s[r][l] * D) : make_uint4(0, 0, 0, 0);
   }
 #pragma unroll
   for (int r = 0; r < R; ++r) {
@@ -91,20 +94,22 @@ __global__ __launch_bounds__(256) void scatter_fwd_kernel(const ScatArgs a) {
 
 // Backward: the span's dout rows are loaded eight at a time (independent
 // loads), and the attention-output row for delta is loaded up front.  A block
-// is one wave (4 rows; spans of 1 to p^(L-1) rows make waves finish at
+// is one wave (4 rows, or 8 for D <= 64; spans of 1 to p^(L-1) rows make waves finish at
 // different times, and one-wave blocks free their slots soonest); XCD runs
 // stay 256 rows long.
-constexpr int SB_ROWS = 4;
-template <typename T>
-__global__ __launch_bounds__(16 * SB_ROWS) void scatter_bwd_kernel(const ScatArgs a) {
+template <typename T, typename Ln>
+__global__ __launch_bounds__(64) void scatter_bwd_kernel(const ScatArgs a) {
   const int tid = threadIdx.x;
-  const long long row = xcd_run(blockIdx.x, gridDim.x, SCAT_RUN * 16 / SB_ROWS) * SB_ROWS + (tid >> 4);
-  const int l16 = tid & 15;
-  if (row >= a.rows) return;  // all 16 lanes of a row leave together
+  constexpr int ROWS = 64 / Ln::LPR;
+  const long long row = xcd_run(blockIdx.x, gridDim.x, SCAT_RUN * 16 / ROWS) * ROWS + tid / Ln::LPR;
+  const int l16 = tid % Ln::LPR;
+  const int D = Ln::FULL ? 8 * Ln::LPR : a.D;
+  const bool in = Ln::in(l16, D);
+  if (row >= a.rows) return;  // all lanes of a row leave together
   const long long bh = row / a.n;
   const int r = a.map[row];
   uint4 ov = make_uint4(0, 0, 0, 0);
-  if (a.delta) ov = ld16(a.o + (size_t)row * LH_D + 8 * l16);
+  if (a.delta && in) ov = ld16(a.o + (size_t)row * D + 8 * l16);
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   if (r >= 0 && r < a.S_tot) {
     int lvl = 1;
@@ -119,7 +124,7 @@ __global__ __launch_bounds__(16 * SB_ROWS) void scatter_bwd_kernel(const ScatArg
     for (int t = start; t < stop; t += 8) {
       uint4 v[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = t + u < stop ? ld16(src + (t + u) * a.st) : make_uint4(0, 0, 0, 0);
+      for (int u = 0; u < 8; ++u) v[u] = in && t + u < stop ? ld16(src + (t + u) * a.st) : make_uint4(0, 0, 0, 0);
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         if (t + u >= stop) break;  // same left-to-right fp32 sum as one row at a time
@@ -131,7 +136,7 @@ __global__ __launch_bounds__(16 * SB_ROWS) void scatter_bwd_kernel(const ScatArg
     }
   }
   const uint4 packed = pack8_t<T>(acc);
-  *reinterpret_cast<uint4*>(a.dst + (size_t)row * LH_D + 8 * l16) = packed;
+  if (in) *reinterpret_cast<uint4*>(a.dst + (size_t)row * D + 8 * l16) = packed;
   if (a.delta) {
     float g[8], o[8];
     unpack8_t<T>(packed, g);
@@ -140,18 +145,19 @@ __global__ __launch_bounds__(16 * SB_ROWS) void scatter_bwd_kernel(const ScatArg
 #pragma unroll
     for (int e = 0; e < 8; ++e) d = fmaf(g[e], o[e], d);
 #pragma unroll
-    for (int m = 1; m < 16; m <<= 1) d += __shfl_xor(d, m, 16);
+    for (int m = 1; m < Ln::LPR; m <<= 1) d += __shfl_xor(d, m, Ln::LPR);
     if (l16 == 0) a.delta[row] = d;
   }
 }
 
-int fill(ScatArgs& a, int S, int S_out, int n, int L, int p, int B, int H, int64_t sb, int64_t sh, int64_t st) {
+int fill(ScatArgs& a, int D, int S, int S_out, int n, int L, int p, int B, int H, int64_t sb, int64_t sh, int64_t st) {
   const int shift = ilog2_exact(p);
   if (shift <= 0 || L < 1 || L > 8 || S <= 0 || S_out <= 0 || n < 0 || B <= 0 || H <= 0) return LH_ERR_INVALID_ARG;
   if ((sb | sh | st) % 8 || sb < 0 || sh < 0 || st <= 0) return LH_ERR_INVALID_ARG;
   Pyramid g;
   if (!make_pyramid(S, L, p, &g)) return LH_ERR_INVALID_ARG;
   a.sb = sb; a.sh = sh; a.st = st; a.H = H;
+  a.D = D;
   a.S = S; a.S_out = S_out; a.n = n; a.L = L; a.shift = shift; a.S_tot = g.total;
   for (int l = 1; l <= L; ++l) { a.off[l] = g.off[l]; a.len[l] = g.len[l]; }
   return LH_OK;
@@ -162,27 +168,28 @@ int fill(ScatArgs& a, int S, int S_out, int n, int L, int p, int B, int H, int64
 extern "C" int lh_scatter_fwd(const void* attn, const int32_t* inverse, void* out, int64_t ob, int64_t oh,
                               int64_t os, int B, int H, int S, int S_out, int n, int D, int L, int p, int dtype,
                               void* stream) {
-  if (D != LH_D) return LH_ERR_UNSUPPORTED;
+  if (!lanes_supported(D)) return LH_ERR_UNSUPPORTED;
   if (!attn || !inverse || !out || ((uintptr_t)out & 15) || !valid_dtype(dtype)) return LH_ERR_INVALID_ARG;
   ScatArgs a{};
-  int rc = fill(a, S, S_out, n, L, p, B, H, ob, oh, os);
+  int rc = fill(a, D, S, S_out, n, L, p, B, H, ob, oh, os);
   if (rc) return rc;
   a.src = (const bf16_t*)attn; a.map = inverse; a.dst = (bf16_t*)out;
   a.rows = (long long)B * H * S_out;
-  const long long blocks = (a.rows + 16 * SF_ROWS - 1) / (16 * SF_ROWS);
+  const int per = (D <= 64 ? 32 : 16) * SF_ROWS;
+  const long long blocks = (a.rows + per - 1) / per;
   if (blocks > 2147483647LL) return LH_ERR_UNSUPPORTED;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)blocks), blk(256);
-  LH_DISPATCH_DTYPE(dtype, switch (L) {
-    case 1: hipLaunchKernelGGL((scatter_fwd_kernel<T, 1, SF_ROWS>), grid, blk, 0, st, a); break;
-    case 2: hipLaunchKernelGGL((scatter_fwd_kernel<T, 2, SF_ROWS>), grid, blk, 0, st, a); break;
-    case 3: hipLaunchKernelGGL((scatter_fwd_kernel<T, 3, SF_ROWS>), grid, blk, 0, st, a); break;
-    case 4: hipLaunchKernelGGL((scatter_fwd_kernel<T, 4, SF_ROWS>), grid, blk, 0, st, a); break;
-    case 5: hipLaunchKernelGGL((scatter_fwd_kernel<T, 5, SF_ROWS>), grid, blk, 0, st, a); break;
-    case 6: hipLaunchKernelGGL((scatter_fwd_kernel<T, 6, SF_ROWS>), grid, blk, 0, st, a); break;
-    case 7: hipLaunchKernelGGL((scatter_fwd_kernel<T, 7, SF_ROWS>), grid, blk, 0, st, a); break;
-    default: hipLaunchKernelGGL((scatter_fwd_kernel<T, 8, SF_ROWS>), grid, blk, 0, st, a); break;
-  });
+  LH_DISPATCH_DTYPE(dtype, LH_DISPATCH_LANES(D, switch (L) {
+    case 1: hipLaunchKernelGGL((scatter_fwd_kernel<T, Ln, 1, SF_ROWS>), grid, blk, 0, st, a); break;
+    case 2: hipLaunchKernelGGL((scatter_fwd_kernel<T, Ln, 2, SF_ROWS>), grid, blk, 0, st, a); break;
+    case 3: hipLaunchKernelGGL((scatter_fwd_kernel<T, Ln, 3, SF_ROWS>), grid, blk, 0, st, a); break;
+    case 4: hipLaunchKernelGGL((scatter_fwd_kernel<T, Ln, 4, SF_ROWS>), grid, blk, 0, st, a); break;
+    case 5: hipLaunchKernelGGL((scatter_fwd_kernel<T, Ln, 5, SF_ROWS>), grid, blk, 0, st, a); break;
+    case 6: hipLaunchKernelGGL((scatter_fwd_kernel<T, Ln, 6, SF_ROWS>), grid, blk, 0, st, a); break;
+    case 7: hipLaunchKernelGGL((scatter_fwd_kernel<T, Ln, 7, SF_ROWS>), grid, blk, 0, st, a); break;
+    default: hipLaunchKernelGGL((scatter_fwd_kernel<T, Ln, 8, SF_ROWS>), grid, blk, 0, st, a); break;
+  }));
   LH_CHECK_LAUNCH();
   return LH_OK;
 }
@@ -190,20 +197,22 @@ extern "C" int lh_scatter_fwd(const void* attn, const int32_t* inverse, void* ou
 extern "C" int lh_scatter_bwd(const void* dout, int64_t db, int64_t dh, int64_t ds, const int32_t* indices,
                               const void* o, void* dattn, float* delta, int B, int H, int S, int S_out, int n, int D,
                               int L, int p, int dtype, void* stream) {
-  if (D != LH_D) return LH_ERR_UNSUPPORTED;
+  if (!lanes_supported(D)) return LH_ERR_UNSUPPORTED;
   if (!dout || !indices || !dattn || ((o == nullptr) != (delta == nullptr)) || ((uintptr_t)dout & 15) ||
       !valid_dtype(dtype))
     return LH_ERR_INVALID_ARG;
   ScatArgs a{};
-  int rc = fill(a, S, S_out, n, L, p, B, H, db, dh, ds);
+  int rc = fill(a, D, S, S_out, n, L, p, B, H, db, dh, ds);
   if (rc) return rc;
   a.src = (const bf16_t*)dout; a.map = indices; a.o = (const bf16_t*)o; a.dst = (bf16_t*)dattn; a.delta = delta;
   a.rows = (long long)B * H * n;
   if (a.rows == 0) return LH_OK;
-  const long long blocks = (a.rows + SB_ROWS - 1) / SB_ROWS;
+  const int per = D <= 64 ? 8 : 4;
+  const long long blocks = (a.rows + per - 1) / per;
   if (blocks > 2147483647LL) return LH_ERR_UNSUPPORTED;
-  LH_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL(scatter_bwd_kernel<T>, dim3((unsigned)blocks), dim3(16 * SB_ROWS), 0,
-                                              reinterpret_cast<hipStream_t>(stream), a));
+  LH_DISPATCH_DTYPE(dtype, LH_DISPATCH_LANES(D, hipLaunchKernelGGL((scatter_bwd_kernel<T, Ln>),
+                                                                  dim3((unsigned)blocks), dim3(64), 0,
+                                                                  reinterpret_cast<hipStream_t>(stream), a)));
   LH_CHECK_LAUNCH();
   return LH_OK;
 }

@@ -35,6 +35,7 @@ class _DenseCausalFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, scale):
         B, H, S, D = q.shape
+        q, k, v = N.shared_rows(q, k, v)
         _mark("dense_fwd_start")
         o, lse = N.attn_fwd(_rows(q, k, v), None, B, H, S, D, scale, shaped=True)
         _mark("dense_attn_fwd")
@@ -46,7 +47,7 @@ class _DenseCausalFn(torch.autograd.Function):
     def backward(ctx, do):
         q, k, v, o, lse = ctx.saved_tensors
         B, H, S, D = q.shape
-        do = do.contiguous()
+        do = N.own_rows(do)
         # softmax-backward row term delta = rowsum(dO * O), accumulated in fp32
         delta = torch.linalg.vecdot(do.float(), o.float())
         _mark("dense_bwd_start")
@@ -58,8 +59,8 @@ class _DenseCausalFn(torch.autograd.Function):
 @graph_break
 def dense_causal_attention(q, k, v):
     """Causal softmax attention, scale 1/sqrt(D): ``q, k, v`` bf16 or fp16 ``[B, H, S, D]``
-    (any batch/head/seq strides, D contiguous) -> ``[B, H, S, D]``.  D < 128 (a
-    multiple of 8) runs zero-padded to the kernels' 128 with scale 1/sqrt(D)."""
+    (any batch/head/seq strides, D contiguous) -> ``[B, H, S, D]``.  D is a multiple
+    of 8, at most 128; 104 to 120 run zero-padded to 128 with scale 1/sqrt(D)."""
     D = q.shape[-1]
     if D > N.D_SUPPORTED or D % 8:
         raise ValueError(f"head_dim must be a multiple of 8 and at most {N.D_SUPPORTED}, got {D}")
@@ -69,8 +70,9 @@ def dense_causal_attention(q, k, v):
         if t.dtype not in N.ROW_DTYPES or t.dtype != q.dtype:
             raise TypeError("the native attention computes in bfloat16 or float16 (one dtype for q, k, v); got "
                             + ", ".join(str(x.dtype) for x in (q, k, v)))
-    if D < N.D_SUPPORTED:
-        q, k, v = (torch.nn.functional.pad(x, (0, N.D_SUPPORTED - D)) for x in (q, k, v))
+    W = N.padded_dim(D)
+    if D < W:
+        q, k, v = (torch.nn.functional.pad(x, (0, W - D)) for x in (q, k, v))
         return _DenseCausalFn.apply(q, k, v, D ** -0.5)[..., :D]
     return _DenseCausalFn.apply(q, k, v, None)
 

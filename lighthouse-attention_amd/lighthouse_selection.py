@@ -120,6 +120,13 @@ def _mark(name):
         _op_hook(name)
 
 
+def _gla_rows(*xs):
+    """Rows as the GLA scorer takes them: contiguous, zero-padded to 128 columns (zero
+    columns change no product, so the scores are the D-wide rows')."""
+    pad = N.D_SUPPORTED - xs[0].shape[-1]
+    return tuple(torch.nn.functional.pad(x, (0, pad)) if pad else x.contiguous() for x in xs)
+
+
 def _layer_fwd(xq, xk, xv, L, p, topk, tie, strict, dilation, seq_major, gk=None, scale=None):
     """Forward of the whole layer on contiguous bf16 [B, S, H, D] inputs:
     pyramid -> selection -> gathered causal attention -> fan-out.  The scorer is
@@ -132,7 +139,7 @@ def _layer_fwd(xq, xk, xv, L, p, topk, tie, strict, dilation, seq_major, gk=None
     _, _, _, S_sel = N.geometry(S, L, p, topk, strict)
     _mark("fwd_start")
     if gk is not None:
-        scores = N.gla_scores(xq, xk, xv, gk, dilation, S_tot, scale)
+        scores = N.gla_scores(*_gla_rows(xq, xk, xv), gk, dilation, S_tot, D ** -0.5 if scale is None else scale)
         _mark("gla_scores")
         pq, pk, pv, sqk, skq = N.pyramid_fwd(xq, xk, xv, L, p, scores=scores)
     elif dilation:
@@ -213,7 +220,7 @@ class _LighthouseLayerFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, xq, xk, xv, L, p, topk, tie, strict, dilation, seq_major, gk, scale):
-        xq, xk, xv = xq.contiguous(), xk.contiguous(), xv.contiguous()
+        xq, xk, xv = N.own_rows(xq), N.own_rows(xk), N.own_rows(xv)
         out, idx, (pq, pk, pv, inv, o, lse) = _layer_fwd(xq, xk, xv, L, p, topk, tie, strict, dilation,
                                                          seq_major, gk, scale)
         ctx.save_for_backward(xq, xk, xv, pq, pk, pv, idx, inv, o, lse)
@@ -257,10 +264,10 @@ def lighthouse_layer(xq, xk, xv, num_levels: int = 3, pooling_factor: int = 4, t
     ``torch.compile`` the layer is one registered custom op (traced without a
     graph break); eagerly it is an ``autograd.Function``; both run the same kernels.
 
-    The kernels work on 128-wide heads.  A head dim D < 128 (a multiple of 8, e.g.
-    the 64 and 72 of the patch's ablation flavors) runs zero-padded to 128 with the
-    scale 1/sqrt(D): zero columns change no dot product, norm or mean, so the
-    results are the D-wide layer's, at 128/D times the work."""
+    The head dim D is a multiple of 8, at most 128.  Up to 96 (e.g. the 64 and 72 of
+    the patch's ablation flavors) and at 128 the kernels read the D-wide rows; 104 to
+    120 run zero-padded to 128 with the scale 1/sqrt(D): zero columns change no dot
+    product, norm or mean, so the results are the D-wide layer's."""
     D = xq.shape[-1]
     if D > N.D_SUPPORTED or D % 8:
         raise ValueError(f"head_dim must be a multiple of 8 and at most {N.D_SUPPORTED}, got {D}")
@@ -274,16 +281,17 @@ def lighthouse_layer(xq, xk, xv, num_levels: int = 3, pooling_factor: int = 4, t
             raise ValueError("the GLA scorer needs dilation >= 1")
         gk = gk.detach()
     scale = None
-    if D < N.D_SUPPORTED:
+    W = N.padded_dim(D)
+    if D < W:
         scale = D ** -0.5
-        xq, xk, xv = (torch.nn.functional.pad(x, (0, N.D_SUPPORTED - D)) for x in (xq, xk, xv))
+        xq, xk, xv = (torch.nn.functional.pad(x, (0, W - D)) for x in (xq, xk, xv))
     if torch.compiler.is_compiling():
         out, idx = _compiled_ops.layer_fwd(xq, xk, xv, num_levels, pooling_factor, topk, tie_break, bool(strict),
                                            int(dilation), bool(seq_major), gk, scale)[:2]
     else:
         out, idx = _LighthouseLayerFn.apply(xq, xk, xv, num_levels, pooling_factor, topk, tie_break, strict,
                                             int(dilation), bool(seq_major), gk, scale)
-    return (out[..., :D] if D < N.D_SUPPORTED else out), idx
+    return (out[..., :D] if D < W else out), idx
 
 
 def _rope_layer_fwd(xqkv, freqs, H, L, p, topk, tie, strict, seq_major):
@@ -404,7 +412,7 @@ class _CompiledOps:
             "bool seq_major, Tensor? gk, float? scale) -> "
             "(Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)"))
         def layer_fwd(xq, xk, xv, L, p, topk, tie, strict, dilation, seq_major, gk, scale):
-            xq, xk, xv = xq.contiguous(), xk.contiguous(), xv.contiguous()
+            xq, xk, xv = N.own_rows(xq), N.own_rows(xk), N.own_rows(xv)
             out, idx, saved = _layer_fwd(xq, xk, xv, L, p, topk, tie, strict, dilation, seq_major, gk, scale)
             return (out, idx) + saved
 
@@ -423,7 +431,7 @@ class _CompiledOps:
             "(Tensor dout, Tensor xq, Tensor xk, Tensor xv, Tensor pq, Tensor pk, Tensor pv, Tensor idx, "
             "Tensor inv, Tensor o, Tensor lse, int L, int p, float? scale) -> (Tensor, Tensor, Tensor)"))
         def layer_bwd(dout, xq, xk, xv, pq, pk, pv, idx, inv, o, lse, L, p, scale):
-            xq, xk, xv = xq.contiguous(), xk.contiguous(), xv.contiguous()
+            xq, xk, xv = N.own_rows(xq), N.own_rows(xk), N.own_rows(xv)
             return _layer_bwd(dout, xq, xk, xv, pq, pk, pv, idx, inv, o, lse, L, p, scale)
 
         @layer_bwd.register_fake
@@ -495,15 +503,15 @@ _compiled_ops = _CompiledOps()
 class _PyramidCatFn(torch.autograd.Function):
     """The reference scorer's 5-tuple from the native pyramid; backward through the
     dense pyramid adjoint (``g[pyramid row]`` gathered onto base rows).  Head dims
-    below 128 run zero-padded (the padded columns of the returned rows are cut off)."""
+    from 104 to 120 run zero-padded (the padded columns of the returned rows are cut off)."""
 
     @staticmethod
     def forward(ctx, xq, xk, xv, L, p, dilation, base_qk=None, base_kq=None):
         B, S, H, D0 = xq.shape
-        xq, xk, xv = xq.contiguous(), xk.contiguous(), xv.contiguous()
-        if D0 < N.D_SUPPORTED:
-            xq, xk, xv = (torch.nn.functional.pad(x, (0, N.D_SUPPORTED - D0)) for x in (xq, xk, xv))
-        D = xq.shape[-1]
+        D = N.padded_dim(D0)
+        if D0 < D:
+            xq, xk, xv = (torch.nn.functional.pad(x, (0, D - D0)) for x in (xq, xk, xv))
+        xq, xk, xv = N.own_rows(xq), N.own_rows(xk), N.own_rows(xv)
         _, _, S_tot = N.pyramid_lengths(S, L, p)
         cats = [torch.empty(B, S_tot, H, D, dtype=xq.dtype, device=xq.device) for _ in range(3)]
         for c, x in zip(cats, (xq, xk, xv)):
@@ -527,9 +535,10 @@ class _PyramidCatFn(torch.autograd.Function):
         ref = next((g for g in gs if g is not None), None)
         if ref is None:
             return None, None, None, None, None, None, None, None
-        gs = [g.contiguous() if g is not None else torch.zeros_like(ref) for g in gs]
+        gs = [g if g is not None else torch.zeros_like(ref) for g in gs]
         if D0 < D:
             gs = [torch.nn.functional.pad(g, (0, D - D0)) for g in gs]
+        gs = [N.own_rows(g) for g in gs]
         dx = N.pyramid_bwd(*gs, None, B, S, H, L, p, D)
         return dx[0][..., :D0], dx[1][..., :D0], dx[2][..., :D0], None, None, None, None, None
 
@@ -551,10 +560,11 @@ class _GatheredAttnFn(torch.autograd.Function):
     def forward(ctx, q_cat, k_cat, v_cat, idx):
         B, H, S_tot, D0 = q_cat.shape
         scale = None
-        if D0 < N.D_SUPPORTED:  # zero-padded head dim, scale 1/sqrt(D0)
-            q_cat, k_cat, v_cat = (torch.nn.functional.pad(x, (0, N.D_SUPPORTED - D0)) for x in (q_cat, k_cat, v_cat))
+        D = N.padded_dim(D0)
+        if D0 < D:  # zero-padded head dim, scale 1/sqrt(D0)
+            q_cat, k_cat, v_cat = (torch.nn.functional.pad(x, (0, D - D0)) for x in (q_cat, k_cat, v_cat))
             scale = D0 ** -0.5
-        D = q_cat.shape[-1]
+        q_cat, k_cat, v_cat = N.shared_rows(q_cat, k_cat, v_cat)
         rows = _GatheredAttnFn._rows(q_cat, k_cat, v_cat)
         n = idx.shape[-1]
         o, lse = N.attn_fwd(rows, idx, B, H, n, D, scale, shaped=True)
@@ -569,9 +579,9 @@ class _GatheredAttnFn(torch.autograd.Function):
         B, H, S_tot, D = q_cat.shape
         rows = _GatheredAttnFn._rows(q_cat, k_cat, v_cat)
         n = idx.shape[-1]
-        do = do.contiguous()
         if D0 < D:
             do = torch.nn.functional.pad(do, (0, D - D0))
+        do = N.own_rows(do)
         delta = (do.float() * o.float()).sum(-1)
         dqs, dks, dvs = N.attn_bwd(rows, idx, B, H, n, do, lse, delta, D, scale, shaped=True)
         inv = N.build_inverse(idx, S_tot)
@@ -593,21 +603,23 @@ class _ScatterToBaseFn(torch.autograd.Function):
             N.check_indices(idx, -1, S_tot, unique=True, what="scatter_to_base_sequence indices")
         inv = N.build_inverse(idx, S_tot)
         D0 = attn_out.shape[-1]
-        if D0 < N.D_SUPPORTED:  # the kernels move 128-wide rows: zero-pad, then cut the columns off
-            attn_out = torch.nn.functional.pad(attn_out, (0, N.D_SUPPORTED - D0))
-        out = N.scatter_fwd(attn_out, inv, N_shard, N_total, num_levels, pooling_factor)
+        pad = -D0 % 8  # the kernels move rows of whole 16-byte chunks: zero-pad, then cut the columns off
+        if pad:
+            attn_out = torch.nn.functional.pad(attn_out, (0, pad))
+        out = N.scatter_fwd(N.own_rows(attn_out), inv, N_shard, N_total, num_levels, pooling_factor)
         ctx.save_for_backward(idx)
         ctx.geo = (N_shard, num_levels, pooling_factor, D0)
-        return out[..., :D0] if D0 < N.D_SUPPORTED else out
+        return out[..., :D0] if pad else out
 
     @staticmethod
     def backward(ctx, grad_output):
         (idx,) = ctx.saved_tensors
         S, L, p, D0 = ctx.geo
-        if D0 < N.D_SUPPORTED:
-            grad_output = torch.nn.functional.pad(grad_output, (0, N.D_SUPPORTED - D0))
+        pad = -D0 % 8
+        if pad:
+            grad_output = torch.nn.functional.pad(grad_output, (0, pad))
         dattn, _ = N.scatter_bwd(grad_output, idx, None, S, L, p)
-        return (dattn[..., :D0] if D0 < N.D_SUPPORTED else dattn), None, None, None, None, None, None
+        return (dattn[..., :D0] if pad else dattn), None, None, None, None, None, None
 
 
 def scatter_to_base_sequence(attn_out, indices_hp, rank_ids_hp, N_shard: int, N_total: int,
@@ -704,10 +716,7 @@ class DilatedLighthouseGLAScorer(nn.Module):
         b, s, h, d = xq.shape
         _, _, S_tot = N.pyramid_lengths(s, self.levels, self.pooling_factor)
         with torch.no_grad():
-            q, k, v = (x.contiguous() for x in (xq, xk, xv))
-            if d < N.D_SUPPORTED:  # zero-padded head dim, as the native layer runs it
-                q, k, v = (torch.nn.functional.pad(x, (0, N.D_SUPPORTED - d)) for x in (q, k, v))
-            sqk, skq = N.gla_scores(q, k, v, gk.detach(), self.dilation, S_tot, self.scaling)
+            sqk, skq = N.gla_scores(*_gla_rows(xq, xk, xv), gk.detach(), self.dilation, S_tot, self.scaling)
         return _PyramidCatFn.apply(xq, xk, xv, self.levels, self.pooling_factor, 0, sqk[..., :s], skq[..., :s])
 
 

@@ -2,8 +2,7 @@
 lighthouse-attention.patch:78-89,514-526; the reference path takes any D through
 BLOCK_D = next_power_of_2(D), src/lighthouse_selection.py:532,566).
 
-The kernels move 128-wide rows; a D-wide head runs zero-padded with the softmax
-scale 1/sqrt(D).  Checked against the fp32 oracle at the original width:
+The softmax scale is 1/sqrt(D).  Checked against the fp32 oracle at the original width:
 selection bit-exact on the device's scores, outputs and gradients within the
 bf16 tolerance."""
 import dataclasses

@@ -1,0 +1,127 @@
+"""Head dims below 128 on their own row width (lh_attn.hip, struct Head; the row
+kernels' struct Lanes): both LDS layouts at their edges and with zero tails,
+against fp32 attention, and the inputs that are copied first because the kernels
+cannot read them in place."""
+import pytest
+import torch
+
+from conftest import assert_close
+from oracle import lh_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+# 8, 40, 56: zero tails in 64-column rows (40: half a k-slice); 64: exact; 72, 88:
+# zero tails in 96 columns (72: half a k-slice); 96: exact; 104: padded to 128.
+# n = 300: whole query blocks of a low-level call, half blocks of the module's
+@pytest.mark.parametrize("D", [8, 40, 56, 64, 72, 88, 96, 104])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_dense_narrow(pkg, dev, D, dtype):
+    N = pkg._native
+    n, H = 300, 3
+    print(f"dense D={D} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(D)
+    xs = [torch.randn(2, n, H, D, generator=g).to(dtype) for _ in range(3)]
+    do = torch.randn(2, H, n, D, generator=g).to(dtype)
+    xg = [x.to(dev).transpose(1, 2).requires_grad_() for x in xs]
+    out = pkg.dense_attention.dense_causal_attention(*xg)
+    grads = torch.autograd.grad(out, xg, do.to(dev))
+    xc = [x.float().transpose(1, 2).contiguous().requires_grad_() for x in xs]
+    ref = O.sdpa_causal(*xc)
+    ref.backward(do.float())
+    assert_close(out, ref, f"D={D} out")
+    for name, a, c in zip(("dq", "dk", "dv"), grads, xc):
+        assert_close(a, c.grad, f"D={D} {name}")
+    if N.padded_dim(D) == D:
+        xd = [x.to(dev) for x in xs]
+        rows = N.Rows(*xd, xd[0].stride()[:3])
+        o, lse = N.attn_fwd(rows, None, 2, H, n, D)
+        delta = (do.to(dev).float() * o.float()).sum(-1)
+        got = (o,) + N.attn_bwd(rows, None, 2, H, n, do.to(dev), lse, delta, D)
+        for name, a, r in zip(("o", "dq", "dk", "dv"), got, [ref] + [c.grad for c in xc]):
+            assert_close(a, r, f"D={D} whole blocks {name}")
+
+
+@pytest.mark.parametrize("D,L,p,strict", [(64, 3, 4, True), (40, 2, 2, False), (96, 3, 2, False), (72, 4, 2, False)])
+def test_row_kernels_narrow(pkg, dev, D, L, p, strict):
+    """Pyramid, fan-out, its adjoint and the pyramid backward give the first D columns
+    of what the zero-padded 128-wide rows give, bit for bit (the sums run over the same
+    values in the same order; the norms add zeros)."""
+    N = pkg._native
+    B, S, H, k = 2, 2048 if strict else 1999, 3, 128
+    print(f"row kernels D={D} L={L} p={p}", flush=True)
+    g = torch.Generator().manual_seed(D + L)
+    xs = [torch.randn(B, S, H, D, generator=g).bfloat16().to(dev) for _ in range(3)]
+    wide = [torch.nn.functional.pad(x, (0, 128 - D)) for x in xs]
+    a, b = N.pyramid_fwd(*xs, L, p), N.pyramid_fwd(*wide, L, p)
+    for x, y in zip(a[:3], b[:3]):
+        assert torch.equal(x, y[..., :D])
+    for x, y in zip(a[3:], b[3:]):  # norms: the tree over 8 or 16 lanes differs, one bf16 ulp at most
+        assert_close(x, y, "scores", max_abs=4e-3, rel_l2=1e-3)
+    idx, inv = N.select_topk(b[3], b[4], S, L, p, k, strict=strict)
+    n = idx.shape[-1]
+    att = torch.randn(B, H, n, D, generator=g).bfloat16().to(dev)
+    attw = torch.nn.functional.pad(att, (0, 128 - D))
+    assert torch.equal(N.scatter_fwd(att, inv, S, S, L, p), N.scatter_fwd(attw, inv, S, S, L, p)[..., :D])
+    do = torch.randn(B, H, S, D, generator=g).bfloat16().to(dev)
+    dow = torch.nn.functional.pad(do, (0, 128 - D))
+    (d1, e1), (d2, e2) = N.scatter_bwd(do, idx, att, S, L, p), N.scatter_bwd(dow, idx, attw, S, L, p)
+    assert torch.equal(d1, d2[..., :D])
+    assert_close(e1, e2, "delta", max_abs=1e-5, rel_l2=1e-6)  # fp32 sums of 8 or 16 lanes
+    gs = [torch.randn(B, H, n, D, generator=g).bfloat16().to(dev) for _ in range(3)]
+    got = N.pyramid_bwd(*gs, inv, B, S, H, L, p, D)
+    want = N.pyramid_bwd(*[torch.nn.functional.pad(x, (0, 128 - D)) for x in gs], inv, B, S, H, L, p, 128)
+    for x, y in zip(got, want):
+        assert torch.equal(x, y[..., :D])
+
+
+def _off(x):
+    """x at an address 2 bytes past a 16-byte boundary."""
+    buf = torch.empty(x.numel() + 1, dtype=x.dtype, device=x.device)[1:]
+    return buf.view(x.shape).copy_(x)
+
+
+def test_narrow_inputs_that_are_copied(pkg, dev):
+    """Strides that differ, a strided head dim, odd strides and odd addresses: accepted
+    for head dims below 128 and equal to the contiguous call."""
+    n, H, D, S = 200, 2, 64, 2048
+    g = torch.Generator().manual_seed(1)
+    q, k, v, do = (torch.randn(1, H, n, D, generator=g).bfloat16().to(dev) for _ in range(4))
+    dense = pkg.dense_attention.dense_causal_attention
+
+    def run(q, k, v, do):
+        xs = [x.detach().requires_grad_() for x in (q, k, v)]
+        o = dense(*xs)
+        return (o,) + torch.autograd.grad(o, xs, do)
+
+    want = run(q, k, v, do)
+    odd = torch.empty(1, H, n, D + 1, dtype=q.dtype, device=dev)[..., :D]
+    forms = [(q.transpose(1, 2).contiguous().transpose(1, 2), k, v, do), (_off(q), _off(k), _off(v), _off(do)),
+             (q.transpose(2, 3).contiguous().transpose(2, 3), k, v, do.transpose(2, 3).contiguous().transpose(2, 3)),
+             (odd.copy_(q), odd.clone().copy_(k), v, do)]
+    for i, f in enumerate(forms):
+        for name, x, y in zip(("o", "dq", "dk", "dv"), run(*f), want):
+            assert torch.equal(x, y), f"form {i}: {name}"
+
+    xs = [torch.randn(1, S, H, D, generator=g).bfloat16().to(dev) for _ in range(3)]
+    dl = torch.randn(1, H, S, D, generator=g).bfloat16().to(dev)
+
+    def layer(xs, dl):
+        xs = [x.detach().requires_grad_() for x in xs]
+        o, idx = pkg.lighthouse_layer(*xs, 3, 4, 128)
+        return (o, idx) + torch.autograd.grad(o, xs, dl)
+
+    for x, y in zip(layer([_off(x) for x in xs], _off(dl)), layer(xs, dl)):
+        assert torch.equal(x, y)
+
+
+def test_fan_out_any_width(pkg, dev):
+    """scatter_to_base_sequence takes row widths that are no multiple of 8."""
+    S, H, L, p = 512, 2, 2, 2
+    att = torch.randn(1, H, 300, 36, generator=torch.Generator().manual_seed(2)).bfloat16().to(dev).requires_grad_()
+    idx = torch.stack([torch.randperm(S + S // p)[:300] for _ in range(H)])[None].int().to(dev)
+    out = pkg.scatter_to_base_sequence(att, idx, None, S, S, L, p)
+    ref = O.scatter_fwd(att.detach().float().cpu(), idx.cpu().long(), S, L, p)
+    assert_close(out, ref, "fan-out of 36 columns")
+    out.backward(torch.ones_like(out))
+    assert att.grad.shape == att.shape
