@@ -20,10 +20,9 @@
  *   inverse       int32 [B, H, S_tot] position in the selected sequence or -1
  *   selected rows bf16 [B, H, n, D];  lse / delta fp32 [B, H, n]
  *   layer output  bf16 [B, H, S, D]
- * D, a multiple of 8: 8..96 and 128 in the attention and dilated-scorer entry
- * points, 8..128 in the pyramid, fan-out and their adjoints, 128 in the GLA
- * scorer and the entry points with a rotary embedding (other head dims there
- * run zero-padded by the caller with the scale of their own width).
+ * D is 128, except in the entry points that say so (lh_attn_*_ex, lh_*_nd: D a
+ * multiple of 8, below 128 too); elsewhere narrower heads run zero-padded by the
+ * caller with the scale of their own width.
  *
  * Citations are to the reference repository (ighoshsubho/lighthouse-attention).
  */
@@ -277,7 +276,8 @@ int lh_attn_bwd_dq(const void *q, const void *k, const void *v, int64_t sb, int6
  * 128 queries whose keys two halves of a workgroup share, where the heaviest
  * 256-query block would outlast the rest); the last bits of its results then
  * depend on them, while with flags = 0 a (b, h) has the same bits alone and
- * beside others.  Unknown bits give LH_ERR_INVALID_ARG.
+ * beside others.  Unknown bits give LH_ERR_INVALID_ARG.  D: 8..96 in steps of 8,
+ * or 128.
  */
 #define LH_ATTN_SHAPED 1
 int lh_attn_fwd_ex(const void *q, const void *k, const void *v, int64_t sb, int64_t ss, int64_t sh,
@@ -289,6 +289,24 @@ int lh_attn_bwd_ex(int parts, const void *q, const void *k, const void *v, int64
                    int split, const int32_t *indices, int B, int H, int n, int D, float scale,
                    const void *dout, const float *lse, const float *delta,
                    void *dq, void *dk, void *dv, int dtype, int flags, void *stream);
+
+/*
+ * The entry points of the same names without _nd, for narrow heads as well: rows
+ * of D elements, D a multiple of 8 up to 128 (lh_dilated_scores_nd: 8..96 or 128).
+ */
+int lh_pyramid_fwd_nd(const void *xq, const void *xk, const void *xv, int64_t sb, int64_t ss, int64_t sh, void *pq,
+                      void *pk, void *pv, int64_t pb, int64_t ps, int64_t ph, float *scores_qk, float *scores_kq,
+                      int B, int S, int H, int D, int L, int p, int base_scores_given, int dtype, void *stream);
+int lh_dilated_scores_nd(const void *xq, const void *xk, const void *xv, float *scores_qk, float *scores_kq, int B,
+                         int S, int H, int D, int dilation, int S_tot, float scale, int dtype, void *stream);
+int lh_scatter_fwd_nd(const void *attn, const int32_t *inverse, void *out, int64_t ob, int64_t oh, int64_t os, int B,
+                      int H, int S, int S_out, int n, int D, int L, int p, int dtype, void *stream);
+int lh_scatter_bwd_nd(const void *dout, int64_t db, int64_t dh, int64_t ds, const int32_t *indices, const void *o,
+                      void *dattn, float *delta, int B, int H, int S, int S_out, int n, int D, int L, int p,
+                      int dtype, void *stream);
+int lh_pyramid_bwd_nd(const void *gq, const void *gk, const void *gv, int64_t gb, int64_t gh, int64_t gs,
+                      const int32_t *inverse, void *dxq, void *dxk, void *dxv, int B, int S, int H, int D, int L,
+                      int p, int dtype, void *stream);
 
 /*
  * Work-queue faults of the persistent attention launches (lh_attn_fwd,

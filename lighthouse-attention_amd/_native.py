@@ -103,6 +103,8 @@ _SIGS = {
     "lh_swiglu_bwd": (_I, [_P, _P, _P, _L, _I, _P]),
     "lh_splitk_sum": (_I, [_P, _P, _I, _L, _P]),
 }
+for _n in ("lh_pyramid_fwd", "lh_dilated_scores", "lh_scatter_fwd", "lh_scatter_bwd", "lh_pyramid_bwd"):
+    _SIGS[_n + "_nd"] = _SIGS[_n]
 EXPORTED = tuple(_SIGS)
 
 
@@ -277,7 +279,7 @@ def pyramid_fwd(xq, xk, xv, L: int, p: int, scores=None, pooled_out=None):
     sb, ss, sh, _ = xq.stride()
     pb, ps, ph, _ = pq.stride()
     with torch.cuda.device(dev):
-        rc = lib().lh_pyramid_fwd(_ptr(xq), _ptr(xk), _ptr(xv), sb, ss, sh, _ptr(pq), _ptr(pk), _ptr(pv),
+        rc = lib().lh_pyramid_fwd_nd(_ptr(xq), _ptr(xk), _ptr(xv), sb, ss, sh, _ptr(pq), _ptr(pk), _ptr(pv),
                                   pb, ps, ph, _ptr(sqk), _ptr(skq), B, S, H, D, L, p, given, dt, _stream(dev))
     _check(rc, "lh_pyramid_fwd")
     return pq, pk, pv, sqk, skq
@@ -332,7 +334,7 @@ def dilated_scores(xq, xk, xv, dilation: int, S_tot: int, scale: float | None = 
     sqk = torch.empty(B, H, S_tot, dtype=torch.float32, device=dev)
     skq = torch.empty_like(sqk)
     with torch.cuda.device(dev):
-        rc = lib().lh_dilated_scores(_ptr(xq), _ptr(xk), _ptr(xv), _ptr(sqk), _ptr(skq), B, S, H, D, dilation,
+        rc = lib().lh_dilated_scores_nd(_ptr(xq), _ptr(xk), _ptr(xv), _ptr(sqk), _ptr(skq), B, S, H, D, dilation,
                                      S_tot, float(scale or 0.0), dt, _stream(dev))
     _check(rc, "lh_dilated_scores")
     _check_queues(dev, "lh_dilated_scores")
@@ -584,7 +586,7 @@ def scatter_fwd(attn, inverse, S: int, S_out: int, L: int, p: int, seq_major: bo
         out = torch.empty(B, H, S_out, D, dtype=attn.dtype, device=attn.device)
     ob, oh, os_, od = out.stride()
     with torch.cuda.device(attn.device):
-        rc = lib().lh_scatter_fwd(_ptr(attn), _ptr(inverse), _ptr(out), ob, oh, os_, B, H, S, S_out, n, D, L, p,
+        rc = lib().lh_scatter_fwd_nd(_ptr(attn), _ptr(inverse), _ptr(out), ob, oh, os_, B, H, S, S_out, n, D, L, p,
                                   dt, _stream(attn.device))
     _check(rc, "lh_scatter_fwd")
     return out
@@ -607,7 +609,7 @@ def scatter_bwd(dout, indices, o, S: int, L: int, p: int):
     oc = o.contiguous() if o is not None else None
     db, dh, ds, _ = dout.stride()
     with torch.cuda.device(dout.device):
-        rc = lib().lh_scatter_bwd(_ptr(dout), db, dh, ds, _ptr(indices.contiguous()), _ptr(oc), _ptr(dattn),
+        rc = lib().lh_scatter_bwd_nd(_ptr(dout), db, dh, ds, _ptr(indices.contiguous()), _ptr(oc), _ptr(dattn),
                                   _ptr(delta), B, H, S, S_out, n, D, L, p, dt, _stream(dout.device))
     _check(rc, "lh_scatter_bwd")
     return dattn, delta
@@ -629,7 +631,7 @@ def pyramid_bwd(gq, gk, gv, inverse, B: int, S: int, H: int, L: int, p: int, D: 
     for g in (gq, gk, gv):
         assert g is None or tuple(g.stride()) == (gb, gh, gs, 1), "selected grads must share strides"
     with torch.cuda.device(dev):
-        rc = lib().lh_pyramid_bwd(_ptr(gq), _ptr(gk), _ptr(gv), gb, gh, gs, _ptr(inverse),
+        rc = lib().lh_pyramid_bwd_nd(_ptr(gq), _ptr(gk), _ptr(gv), gb, gh, gs, _ptr(inverse),
                                   _ptr(outs[0]), _ptr(outs[1]), _ptr(outs[2]), B, S, H, D, L, p, dt, _stream(dev))
     _check(rc, "lh_pyramid_bwd")
     return tuple(outs)

@@ -2386,6 +2386,7 @@ extern "C" int lh_attn_fwd(const void* q, const void* k, const void* v, int64_t 
                            const void* qp, const void* kp, const void* vp, int64_t pb, int64_t ps, int64_t ph,
                            int split, const int32_t* indices, int B, int H, int n, int D, float scale, void* out,
                            float* lse, int dtype, void* stream) {
+  if (D != LH_D) return LH_ERR_UNSUPPORTED;
   return attn_fwd_impl(q, k, v, sb, ss, sh, qp, kp, vp, pb, ps, ph, split, indices, B, H, n, D, scale, out, lse, dtype,
                        0, stream);
 }
@@ -2403,6 +2404,7 @@ extern "C" int lh_attn_bwd(const void* q, const void* k, const void* v, int64_t 
                            int split, const int32_t* indices, int B, int H, int n, int D, float scale, const void* dout,
                            const float* lse, const float* delta, void* dq, void* dk, void* dv, int dtype,
                            void* stream) {
+  if (D != LH_D) return LH_ERR_UNSUPPORTED;
   return attn_bwd_parts(3, q, k, v, sb, ss, sh, qp, kp, vp, pb, ps, ph, split, indices, B, H, n, D, scale, dout, lse,
                         delta, dq, dk, dv, dtype, 0, stream);
 }
@@ -2421,6 +2423,7 @@ extern "C" int lh_attn_bwd_dkdv(const void* q, const void* k, const void* v, int
                                 int split, const int32_t* indices, int B, int H, int n, int D, float scale,
                                 const void* dout, const float* lse, const float* delta, void* dk, void* dv, int dtype,
                                 void* stream) {
+  if (D != LH_D) return LH_ERR_UNSUPPORTED;
   return attn_bwd_parts(1, q, k, v, sb, ss, sh, qp, kp, vp, pb, ps, ph, split, indices, B, H, n, D, scale, dout, lse,
                         delta, nullptr, dk, dv, dtype, 0, stream);
 }
@@ -2430,6 +2433,7 @@ extern "C" int lh_attn_bwd_dq(const void* q, const void* k, const void* v, int64
                               int split, const int32_t* indices, int B, int H, int n, int D, float scale,
                               const void* dout, const float* lse, const float* delta, void* dq, int dtype,
                               void* stream) {
+  if (D != LH_D) return LH_ERR_UNSUPPORTED;
   return attn_bwd_parts(2, q, k, v, sb, ss, sh, qp, kp, vp, pb, ps, ph, split, indices, B, H, n, D, scale, dout, lse,
                         delta, dq, nullptr, nullptr, dtype, 0, stream);
 }
@@ -2481,9 +2485,9 @@ extern "C" int lh_attn_queue_slot(void* stream, void** slot) {
   return *slot ? LH_OK : LH_ERR_UNSUPPORTED;
 }
 
-extern "C" int lh_dilated_scores(const void* xq, const void* xk, const void* xv, float* scores_qk, float* scores_kq,
-                                 int B, int S, int H, int D, int dilation, int S_tot, float scale, int dtype,
-                                 void* stream) {
+extern "C" int lh_dilated_scores_nd(const void* xq, const void* xk, const void* xv, float* scores_qk,
+                                    float* scores_kq, int B, int S, int H, int D, int dilation, int S_tot,
+                                    float scale, int dtype, void* stream) {
   if (!head_supported(D)) return LH_ERR_UNSUPPORTED;
   if (!valid_dtype(dtype)) return LH_ERR_INVALID_ARG;
   if (!xq || !xk || !xv || !scores_qk || !scores_kq || dilation <= 0 || S <= 0 || S % dilation || S_tot < S)
@@ -2508,6 +2512,13 @@ extern "C" int lh_dilated_scores(const void* xq, const void* xk, const void* xv,
     LH_CHECK_LAUNCH();
   }
   return LH_OK;
+}
+
+extern "C" int lh_dilated_scores(const void* xq, const void* xk, const void* xv, float* scores_qk, float* scores_kq,
+                                 int B, int S, int H, int D, int dilation, int S_tot, float scale, int dtype,
+                                 void* stream) {
+  if (D != LH_D) return LH_ERR_UNSUPPORTED;
+  return lh_dilated_scores_nd(xq, xk, xv, scores_qk, scores_kq, B, S, H, D, dilation, S_tot, scale, dtype, stream);
 }
 
 namespace {

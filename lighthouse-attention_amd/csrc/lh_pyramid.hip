@@ -379,12 +379,21 @@ int pyramid_bwd_impl(const void* gq, const void* gk, const void* gv, int64_t gb,
 
 }  // namespace
 
-extern "C" int lh_pyramid_fwd(const void* xq, const void* xk, const void* xv, int64_t sb, int64_t ss, int64_t sh,
-                              void* pq, void* pk, void* pv, int64_t pb, int64_t ps, int64_t ph,
-                              float* scores_qk, float* scores_kq, int B, int S, int H, int D, int L, int p,
-                              int base_scores_given, int dtype, void* stream) {
+extern "C" int lh_pyramid_fwd_nd(const void* xq, const void* xk, const void* xv, int64_t sb, int64_t ss, int64_t sh,
+                                 void* pq, void* pk, void* pv, int64_t pb, int64_t ps, int64_t ph, float* scores_qk,
+                                 float* scores_kq, int B, int S, int H, int D, int L, int p, int base_scores_given,
+                                 int dtype, void* stream) {
   return pyramid_fwd_impl(xq, xk, xv, sb, ss, sh, nullptr, nullptr, nullptr, 0, 0, 0, pq, pk, pv, pb, ps, ph,
                           scores_qk, scores_kq, B, S, H, D, L, p, base_scores_given != 0, dtype, stream);
+}
+
+extern "C" int lh_pyramid_fwd(const void* xq, const void* xk, const void* xv, int64_t sb, int64_t ss, int64_t sh,
+                              void* pq, void* pk, void* pv, int64_t pb, int64_t ps, int64_t ph, float* scores_qk,
+                              float* scores_kq, int B, int S, int H, int D, int L, int p, int base_scores_given,
+                              int dtype, void* stream) {
+  if (D != LH_D) return LH_ERR_UNSUPPORTED;
+  return lh_pyramid_fwd_nd(xq, xk, xv, sb, ss, sh, pq, pk, pv, pb, ps, ph, scores_qk, scores_kq, B, S, H, D, L, p,
+                           base_scores_given, dtype, stream);
 }
 
 extern "C" int lh_rope_pyramid_fwd(const void* xq, const void* xk, const void* xv, int64_t sb, int64_t ss,
@@ -397,12 +406,19 @@ extern "C" int lh_rope_pyramid_fwd(const void* xq, const void* xk, const void* x
                           scores_kq, B, S, H, D, L, p, false, LH_DTYPE_BF16, stream);
 }
 
-extern "C" int lh_pyramid_bwd(const void* gq, const void* gk, const void* gv, int64_t gb, int64_t gh, int64_t gs,
-                              const int32_t* inverse, void* dxq, void* dxk, void* dxv, int B, int S, int H, int D,
-                              int L, int p, int dtype, void* stream) {
+extern "C" int lh_pyramid_bwd_nd(const void* gq, const void* gk, const void* gv, int64_t gb, int64_t gh, int64_t gs,
+                                 const int32_t* inverse, void* dxq, void* dxk, void* dxv, int B, int S, int H, int D,
+                                 int L, int p, int dtype, void* stream) {
   const int64_t oh = D, os = (int64_t)H * D, ob = (int64_t)S * os;
   return pyramid_bwd_impl(gq, gk, gv, gb, gh, gs, inverse, nullptr, dxq, dxk, dxv, ob, os, oh, B, S, H, D, L, p,
                           dtype, stream);
+}
+
+extern "C" int lh_pyramid_bwd(const void* gq, const void* gk, const void* gv, int64_t gb, int64_t gh, int64_t gs,
+                              const int32_t* inverse, void* dxq, void* dxk, void* dxv, int B, int S, int H, int D,
+                              int L, int p, int dtype, void* stream) {
+  if (D != LH_D) return LH_ERR_UNSUPPORTED;
+  return lh_pyramid_bwd_nd(gq, gk, gv, gb, gh, gs, inverse, dxq, dxk, dxv, B, S, H, D, L, p, dtype, stream);
 }
 
 extern "C" int lh_pyramid_rope_bwd(const void* gq, const void* gk, const void* gv, int64_t gb, int64_t gh,

@@ -165,9 +165,9 @@ int fill(ScatArgs& a, int D, int S, int S_out, int n, int L, int p, int B, int H
 
 }  // namespace
 
-extern "C" int lh_scatter_fwd(const void* attn, const int32_t* inverse, void* out, int64_t ob, int64_t oh,
-                              int64_t os, int B, int H, int S, int S_out, int n, int D, int L, int p, int dtype,
-                              void* stream) {
+extern "C" int lh_scatter_fwd_nd(const void* attn, const int32_t* inverse, void* out, int64_t ob, int64_t oh,
+                                 int64_t os, int B, int H, int S, int S_out, int n, int D, int L, int p, int dtype,
+                                 void* stream) {
   if (!lanes_supported(D)) return LH_ERR_UNSUPPORTED;
   if (!attn || !inverse || !out || ((uintptr_t)out & 15) || !valid_dtype(dtype)) return LH_ERR_INVALID_ARG;
   ScatArgs a{};
@@ -194,9 +194,15 @@ extern "C" int lh_scatter_fwd(const void* attn, const int32_t* inverse, void* ou
   return LH_OK;
 }
 
-extern "C" int lh_scatter_bwd(const void* dout, int64_t db, int64_t dh, int64_t ds, const int32_t* indices,
-                              const void* o, void* dattn, float* delta, int B, int H, int S, int S_out, int n, int D,
-                              int L, int p, int dtype, void* stream) {
+extern "C" int lh_scatter_fwd(const void* attn, const int32_t* inverse, void* out, int64_t ob, int64_t oh, int64_t os,
+                              int B, int H, int S, int S_out, int n, int D, int L, int p, int dtype, void* stream) {
+  if (D != LH_D) return LH_ERR_UNSUPPORTED;
+  return lh_scatter_fwd_nd(attn, inverse, out, ob, oh, os, B, H, S, S_out, n, D, L, p, dtype, stream);
+}
+
+extern "C" int lh_scatter_bwd_nd(const void* dout, int64_t db, int64_t dh, int64_t ds, const int32_t* indices,
+                                 const void* o, void* dattn, float* delta, int B, int H, int S, int S_out, int n,
+                                 int D, int L, int p, int dtype, void* stream) {
   if (!lanes_supported(D)) return LH_ERR_UNSUPPORTED;
   if (!dout || !indices || !dattn || ((o == nullptr) != (delta == nullptr)) || ((uintptr_t)dout & 15) ||
       !valid_dtype(dtype))
@@ -215,4 +221,11 @@ extern "C" int lh_scatter_bwd(const void* dout, int64_t db, int64_t dh, int64_t 
                                                                   reinterpret_cast<hipStream_t>(stream), a)));
   LH_CHECK_LAUNCH();
   return LH_OK;
+}
+
+extern "C" int lh_scatter_bwd(const void* dout, int64_t db, int64_t dh, int64_t ds, const int32_t* indices,
+                              const void* o, void* dattn, float* delta, int B, int H, int S, int S_out, int n, int D,
+                              int L, int p, int dtype, void* stream) {
+  if (D != LH_D) return LH_ERR_UNSUPPORTED;
+  return lh_scatter_bwd_nd(dout, db, dh, ds, indices, o, dattn, delta, B, H, S, S_out, n, D, L, p, dtype, stream);
 }
