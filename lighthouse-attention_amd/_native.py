@@ -525,8 +525,9 @@ def attn_bwd_dkdv(rows: Rows, indices, B: int, H: int, n: int, dout, lse, delta,
     idx = indices.contiguous() if indices is not None else None
     dk, dv = (torch.empty(B, H, n, D, dtype=rows.dtype, device=dev) for _ in range(2))
     with torch.cuda.device(dev):
-        rc = lib().lh_attn_bwd_dkdv(*rows.args(), _ptr(idx), B, H, n, D, scale, _ptr(dout.contiguous()),
-                                    _ptr(lse), _ptr(delta), _ptr(dk), _ptr(dv), rows.dtype_code, _stream(dev))
+        rc = lib().lh_attn_bwd_ex(1, *rows.args(), _ptr(idx), B, H, n, D, scale, _ptr(dout.contiguous()),
+                                  _ptr(lse), _ptr(delta), None, _ptr(dk), _ptr(dv), rows.dtype_code, 0,
+                                  _stream(dev))
     _check(rc, "lh_attn_bwd_dkdv")
     _check_queues(dev, "lh_attn_bwd_dkdv")
     return dk, dv
