@@ -309,6 +309,16 @@ int lh_pyramid_bwd_nd(const void *gq, const void *gk, const void *gv, int64_t gb
                       int p, int dtype, void *stream);
 
 /*
+ * The softmax backward's row term of an attention without a fan-out:
+ * delta fp32 [B, H, n] = rowsum(dout * o), fp32 sums.  dout is [B, H, n, D] with
+ * element strides (db, dh, ds), each a multiple of 8, D contiguous; o is
+ * contiguous.  copy, if not NULL, receives dout as contiguous rows.  D: a
+ * multiple of 8 up to 128.  (The reference's SDPA forms it inside its backward.)
+ */
+int lh_attn_delta(const void *dout, int64_t db, int64_t dh, int64_t ds, const void *o, void *copy, float *delta,
+                  int B, int H, int n, int D, int dtype, void *stream);
+
+/*
  * Work-queue faults of the persistent attention launches (lh_attn_fwd,
  * lh_attn_bwd*, lh_dilated_scores) on the current device since the last call.
  * Waits for the device to go idle (hipDeviceSynchronize), then counts the

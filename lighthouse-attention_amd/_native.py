@@ -83,6 +83,7 @@ _SIGS = {
                             _I, _I, _I, _I, _F, _P, _P, _I, _I, _P]),
     "lh_attn_bwd_ex": (_I, [_I, _P, _P, _P, _L, _L, _L, _P, _P, _P, _L, _L, _L, _I, _P,
                             _I, _I, _I, _I, _F, _P, _P, _P, _P, _P, _P, _I, _I, _P]),
+    "lh_attn_delta": (_I, [_P, _L, _L, _L, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     "lh_attn_status": (_I, [_P]),
     "lh_attn_queue_slot": (_I, [_P, _P]),
     "lh_attn_set_schedule": (_I, [_I, _P]),
@@ -567,6 +568,27 @@ def attn_bwd(rows: Rows, indices, B: int, H: int, n: int, dout, lse, delta, D: i
     _check(rc, "lh_attn_bwd")
     _check_queues(dev, "lh_attn_bwd")
     return dq, dk, dv
+
+
+def attn_delta(dout, o):
+    """``(dout contiguous, delta fp32 [B, H, n])`` with ``delta = rowsum(dout * o)``;
+    ``dout`` may have any strides (copied in the same pass if it is not contiguous),
+    ``o`` [B, H, n, D] is contiguous."""
+    dt = _need_rows("attn_delta", o)
+    _need_dtype("attention backward dout", o.dtype, dout)
+    _need_gpu(dout, o)
+    B, H, n, D = o.shape
+    assert dout.shape == o.shape and o.is_contiguous()
+    if dout.stride(3) != 1 or any(st % 8 for st in dout.stride()[:3]) or dout.data_ptr() % 16:
+        dout = own_rows(dout)
+    st = [s if size > 1 else 0 for s, size in zip(dout.stride(), dout.shape)]
+    rows = dout if dout.is_contiguous() else torch.empty(dout.shape, dtype=dout.dtype, device=dout.device)
+    delta = torch.empty(B, H, n, dtype=torch.float32, device=dout.device)
+    with torch.cuda.device(dout.device):
+        rc = lib().lh_attn_delta(_ptr(dout), *st[:3], _ptr(o), None if rows is dout else _ptr(rows), _ptr(delta),
+                                 B, H, n, D, dt, _stream(dout.device))
+    _check(rc, "lh_attn_delta")
+    return rows, delta
 
 
 def scatter_fwd(attn, inverse, S: int, S_out: int, L: int, p: int, seq_major: bool = False):

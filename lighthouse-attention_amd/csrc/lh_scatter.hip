@@ -150,6 +150,43 @@ __global__ __launch_bounds__(64) void scatter_bwd_kernel(const ScatArgs a) {
   }
 }
 
+// delta = rowsum(dout * o) of the attention backward outside the fan-out (dense
+// causal attention), and dout copied to contiguous rows on the way where its
+// strides ask for it: one pass over both tensors.  Bound by memory; as torch
+// operations (two widening casts, a product, a sum and the copy) it took 115 us
+// at 8 heads of 16384, in one pass 20 us.
+struct DeltaArgs {
+  const bf16_t *dout, *o;
+  bf16_t* copy;  // [BH, n, D] or null
+  float* delta;
+  int64_t sb, sh, ss;
+  int H, n, D;
+  int chunks;  // blocks per (b, h)
+};
+
+template <typename T, typename Ln>
+__global__ __launch_bounds__(256) void attn_delta_kernel(const DeltaArgs a) {
+  const int bh = blockIdx.x / a.chunks, b = bh / a.H, h = bh - b * a.H;
+  const int s = (blockIdx.x - bh * a.chunks) * Ln::ROWS + threadIdx.x / Ln::LPR;
+  const int l = threadIdx.x % Ln::LPR;
+  if (s >= a.n) return;
+  const int64_t row = (int64_t)bh * a.n + s;
+  float d = 0.f;
+  if (Ln::in(l, a.D)) {
+    const uint4 gv = ld16(a.dout + b * a.sb + h * a.sh + s * a.ss + 8 * l);
+    const uint4 ov = ld16(a.o + row * a.D + 8 * l);
+    if (a.copy) *reinterpret_cast<uint4*>(a.copy + row * a.D + 8 * l) = gv;
+    float g[8], o[8];
+    unpack8_t<T>(gv, g);
+    unpack8_t<T>(ov, o);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) d = fmaf(g[e], o[e], d);
+  }
+#pragma unroll
+  for (int m = 1; m < Ln::LPR; m <<= 1) d += __shfl_xor(d, m, Ln::LPR);
+  if (l == 0) a.delta[row] = d;
+}
+
 int fill(ScatArgs& a, int D, int S, int S_out, int n, int L, int p, int B, int H, int64_t sb, int64_t sh, int64_t st) {
   const int shift = ilog2_exact(p);
   if (shift <= 0 || L < 1 || L > 8 || S <= 0 || S_out <= 0 || n < 0 || B <= 0 || H <= 0) return LH_ERR_INVALID_ARG;
@@ -228,4 +265,20 @@ extern "C" int lh_scatter_bwd(const void* dout, int64_t db, int64_t dh, int64_t 
                               int L, int p, int dtype, void* stream) {
   if (D != LH_D) return LH_ERR_UNSUPPORTED;
   return lh_scatter_bwd_nd(dout, db, dh, ds, indices, o, dattn, delta, B, H, S, S_out, n, D, L, p, dtype, stream);
+}
+
+extern "C" int lh_attn_delta(const void* dout, int64_t db, int64_t dh, int64_t ds, const void* o, void* copy,
+                             float* delta, int B, int H, int n, int D, int dtype, void* stream) {
+  if (!lanes_supported(D)) return LH_ERR_UNSUPPORTED;
+  if (!dout || !o || !delta || B <= 0 || H <= 0 || n <= 0 || !valid_dtype(dtype)) return LH_ERR_INVALID_ARG;
+  if (((uintptr_t)dout | (uintptr_t)o | (uintptr_t)copy) & 15 || (db | dh | ds) % 8) return LH_ERR_INVALID_ARG;
+  const int per = D <= 64 ? 32 : 16;
+  DeltaArgs a{(const bf16_t*)dout, (const bf16_t*)o, (bf16_t*)copy, delta, db, dh, ds, H, n, D, (n - 1) / per + 1};
+  const long long blocks = (long long)B * H * a.chunks;
+  if (blocks > 2147483647LL) return LH_ERR_UNSUPPORTED;
+  LH_DISPATCH_DTYPE(dtype, LH_DISPATCH_LANES(D, hipLaunchKernelGGL((attn_delta_kernel<T, Ln>), dim3((unsigned)blocks),
+                                                                  dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
+                                                                  a)));
+  LH_CHECK_LAUNCH();
+  return LH_OK;
 }

@@ -47,9 +47,8 @@ class _DenseCausalFn(torch.autograd.Function):
     def backward(ctx, do):
         q, k, v, o, lse = ctx.saved_tensors
         B, H, S, D = q.shape
-        do = N.own_rows(do)
         # softmax-backward row term delta = rowsum(dO * O), accumulated in fp32
-        delta = torch.linalg.vecdot(do.float(), o.float())
+        do, delta = N.attn_delta(do, o)
         _mark("dense_bwd_start")
         dq, dk, dv = N.attn_bwd(_rows(q, k, v), None, B, H, S, do, lse, delta, D, ctx.scale, shaped=True)
         _mark("dense_attn_bwd")

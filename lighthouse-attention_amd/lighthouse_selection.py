@@ -581,8 +581,7 @@ class _GatheredAttnFn(torch.autograd.Function):
         n = idx.shape[-1]
         if D0 < D:
             do = torch.nn.functional.pad(do, (0, D - D0))
-        do = N.own_rows(do)
-        delta = (do.float() * o.float()).sum(-1)
+        do, delta = N.attn_delta(do, o)
         dqs, dks, dvs = N.attn_bwd(rows, idx, B, H, n, do, lse, delta, D, scale, shaped=True)
         inv = N.build_inverse(idx, S_tot)
         # one-level pyramid over S_tot rows: row r receives dsel[inv[r]] (or 0)

@@ -125,3 +125,24 @@ def test_fan_out_any_width(pkg, dev):
     assert_close(out, ref, "fan-out of 36 columns")
     out.backward(torch.ones_like(out))
     assert att.grad.shape == att.shape
+
+
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (72, torch.float16), (64, torch.bfloat16), (8, torch.bfloat16)])
+def test_attn_delta(pkg, dev, D, dtype):
+    """Row sums of dO * O and the contiguous dO, for contiguous, transposed, expanded
+    and unaligned upstream gradients; 33 rows: two blocks, the second nearly empty."""
+    N = pkg._native
+    B, H, n = 2, 3, 33
+    g = torch.Generator().manual_seed(D)
+    o = torch.randn(B, H, n, D, generator=g).to(dtype).to(dev)
+    do = torch.randn(B, n, H, D, generator=g).to(dtype).to(dev)
+    forms = [do.transpose(1, 2).contiguous(), do.transpose(1, 2), do[:1, :, :1].expand(B, n, H, D).transpose(1, 2)]
+    if D < 128:
+        forms.append(_off(do.transpose(1, 2).contiguous()))
+    for i, f in enumerate(forms):
+        rows, delta = N.attn_delta(f, o)
+        assert rows.is_contiguous() and torch.equal(rows, f), f"form {i}"
+        ref = (f.double() * o.double()).sum(-1)
+        # fp32 sums of D products of 16-bit values: D roundings at most
+        bound = D * 2.0 ** -24 * (f.double() * o.double()).abs().sum(-1)
+        assert bool(((delta.double() - ref).abs() <= bound).all()), f"form {i}"
