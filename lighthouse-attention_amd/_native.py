@@ -13,6 +13,7 @@ import ctypes
 import os
 import subprocess
 import threading
+from functools import lru_cache
 
 import torch
 
@@ -147,11 +148,32 @@ def _check(rc: int, what: str):
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+# The current stream's handle and the current device, without the Python objects
+# around them (a call made 4 us of such objects and of a device guard otherwise).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+if _raw_stream is None:
+    def _raw_stream(index):
+        return torch.cuda.current_stream(index).cuda_stream
 
 
 def _stream(dev):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    return torch.cuda.current_stream(dev).cuda_stream
+
+
+def _run(name: str, dev, *args):
+    """The library function ``name`` with ``args`` and the current stream of ``dev``
+    (its last argument), on that device; raises on an error code."""
+    f = getattr(_lib or lib(), name)
+    if torch.cuda.current_device() == dev.index:
+        rc = f(*args, _raw_stream(dev.index))
+    else:
+        with torch.cuda.device(dev):
+            rc = f(*args, _raw_stream(dev.index))
+    if rc:
+        _check(rc, name)
 
 
 def _need_gpu(*ts):
@@ -216,9 +238,7 @@ def check_indices(indices, lo: int, hi: int, unique: bool = True, what: str = "i
     dev = idx.device
     counts = torch.empty(2, dtype=torch.int32, device=dev)
     marks = torch.empty(B, H, hi - lo, dtype=torch.int32, device=dev) if unique else None
-    with torch.cuda.device(dev):
-        rc = lib().lh_check_indices(_ptr(idx), B, H, n, lo, hi, _ptr(marks), _ptr(counts), _stream(dev))
-    _check(rc, "lh_check_indices")
+    _run("lh_check_indices", dev, _ptr(idx), B, H, n, lo, hi, _ptr(marks), _ptr(counts))
     bad, dup = (int(c) for c in counts.cpu())
     if bad:
         raise IndexError(f"{what}: {bad} entries outside [{lo}, {hi})")
@@ -226,6 +246,7 @@ def check_indices(indices, lo: int, hi: int, unique: bool = True, what: str = "i
         raise IndexError(f"{what}: {dup} duplicate entries (indices must be unique per (batch, head))")
 
 
+@lru_cache(maxsize=256)
 def geometry(S: int, L: int, p: int, topk: int, strict: bool = True):
     """``(num_tiles, nodes_per_tile, per_tile, S_sel)``; raises like the reference outside
     its domain when ``strict``."""
@@ -238,6 +259,11 @@ def geometry(S: int, L: int, p: int, topk: int, strict: bool = True):
             "divide the coarsest level); pass strict=False for per-tile compaction")
     _check(rc, "lh_select_geometry")
     return tuple(o.value for o in out)
+
+
+@lru_cache(maxsize=256)
+def pyramid_total(S: int, L: int, p: int) -> int:
+    return pyramid_lengths(S, L, p)[2]
 
 
 def pyramid_lengths(S: int, L: int, p: int):
@@ -262,7 +288,7 @@ def pyramid_fwd(xq, xk, xv, L: int, p: int, scores=None, pooled_out=None):
     B, S, H, D = xq.shape
     assert xk.shape == xq.shape and xv.shape == xq.shape
     assert xq.stride() == xk.stride() == xv.stride(), "q/k/v must share strides"
-    lens, offs, S_tot = pyramid_lengths(S, L, p)
+    S_tot = pyramid_total(S, L, p)
     Sp = S_tot - S
     dev = xq.device
     if pooled_out is None:
@@ -279,10 +305,8 @@ def pyramid_fwd(xq, xk, xv, L: int, p: int, scores=None, pooled_out=None):
         given = 1
     sb, ss, sh, _ = xq.stride()
     pb, ps, ph, _ = pq.stride()
-    with torch.cuda.device(dev):
-        rc = lib().lh_pyramid_fwd_nd(_ptr(xq), _ptr(xk), _ptr(xv), sb, ss, sh, _ptr(pq), _ptr(pk), _ptr(pv),
-                                  pb, ps, ph, _ptr(sqk), _ptr(skq), B, S, H, D, L, p, given, dt, _stream(dev))
-    _check(rc, "lh_pyramid_fwd")
+    _run("lh_pyramid_fwd_nd", dev, _ptr(xq), _ptr(xk), _ptr(xv), sb, ss, sh, _ptr(pq), _ptr(pk), _ptr(pv), pb, ps, ph,
+         _ptr(sqk), _ptr(skq), B, S, H, D, L, p, given, dt)
     return pq, pk, pv, sqk, skq
 
 
@@ -306,7 +330,7 @@ def rope_pyramid_fwd(xqkv, freqs, H: int, L: int, p: int, D: int = D_SUPPORTED):
     assert W == 3 * H * D, "xqkv must hold [q | k | v] heads"
     assert xqkv.stride(2) == 1 and xqkv.stride(0) == S * xqkv.stride(1), "rows of xqkv must be evenly strided"
     _check_freqs(freqs, S, D)
-    lens, offs, S_tot = pyramid_lengths(S, L, p)
+    S_tot = pyramid_total(S, L, p)
     dev = xqkv.device
     xr = torch.empty_strided(xqkv.shape, xqkv.stride(), dtype=torch.bfloat16, device=dev)
     pq, pk, pv = (torch.empty(B, S_tot - S, H, D, dtype=torch.bfloat16, device=dev) for _ in range(3))
@@ -315,12 +339,9 @@ def rope_pyramid_fwd(xqkv, freqs, H: int, L: int, p: int, D: int = D_SUPPORTED):
     rs = xqkv.stride(1)
     base = xqkv.data_ptr()
     e = xqkv.element_size()
-    with torch.cuda.device(dev):
-        rc = lib().lh_rope_pyramid_fwd(base, base + H * D * e, base + 2 * H * D * e, S * rs, rs, D,
-                                       _ptr(freqs), xr.data_ptr(), xr.data_ptr() + H * D * e, S * rs, rs, D,
-                                       _ptr(pq), _ptr(pk), _ptr(pv), *pq.stride()[:3], _ptr(sqk), _ptr(skq),
-                                       B, S, H, D, L, p, _stream(dev))
-    _check(rc, "lh_rope_pyramid_fwd")
+    _run("lh_rope_pyramid_fwd", dev, base, base + H * D * e, base + 2 * H * D * e, S * rs, rs, D, _ptr(freqs),
+         xr.data_ptr(), xr.data_ptr() + H * D * e, S * rs, rs, D, _ptr(pq), _ptr(pk), _ptr(pv), *pq.stride()[:3],
+         _ptr(sqk), _ptr(skq), B, S, H, D, L, p)
     return xr, pq, pk, pv, sqk, skq
 
 
@@ -334,10 +355,8 @@ def dilated_scores(xq, xk, xv, dilation: int, S_tot: int, scale: float | None = 
     dev = xq.device
     sqk = torch.empty(B, H, S_tot, dtype=torch.float32, device=dev)
     skq = torch.empty_like(sqk)
-    with torch.cuda.device(dev):
-        rc = lib().lh_dilated_scores_nd(_ptr(xq), _ptr(xk), _ptr(xv), _ptr(sqk), _ptr(skq), B, S, H, D, dilation,
-                                     S_tot, float(scale or 0.0), dt, _stream(dev))
-    _check(rc, "lh_dilated_scores")
+    _run("lh_dilated_scores_nd", dev, _ptr(xq), _ptr(xk), _ptr(xv), _ptr(sqk), _ptr(skq), B, S, H, D, dilation, S_tot,
+         float(scale or 0.0), dt)
     _check_queues(dev, "lh_dilated_scores")
     return sqk, skq
 
@@ -364,11 +383,8 @@ def gla_scores(xq, xk, xv, gk, dilation: int, S_tot: int, scale: float | None = 
     if nbytes < 0:
         raise ValueError(f"gla_scores: invalid geometry B={B} S={S} H={H} D={D} dilation={dilation}")
     ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev) if nbytes else None
-    with torch.cuda.device(dev):
-        rc = lib().lh_gla_scores(_ptr(xq), _ptr(xk), _ptr(xv), _ptr(g), _ptr(sqk), _ptr(skq), B, S, H, D, dilation,
-                                 S_tot, float(scale), int(segments), _ptr(ws), nbytes, dt,
-                                 _stream(dev))
-    _check(rc, "lh_gla_scores")
+    _run("lh_gla_scores", dev, _ptr(xq), _ptr(xk), _ptr(xv), _ptr(g), _ptr(sqk), _ptr(skq), B, S, H, D, dilation,
+         S_tot, float(scale), int(segments), _ptr(ws), nbytes, dt)
     return sqk, skq
 
 
@@ -381,7 +397,7 @@ def select_topk(scores_qk, scores_kq, S: int, L: int, p: int, topk: int, tie: st
     if tie not in TIE_MODES:
         raise ValueError(f"tie_break must be one of {sorted(TIE_MODES)}, got {tie!r}")
     B, H, S_tot = scores_qk.shape
-    _, _, S_tot_expected = pyramid_lengths(S, L, p)
+    S_tot_expected = pyramid_total(S, L, p)
     assert S_tot >= S_tot_expected, "scores are shorter than the pyramid"
     sqk = scores_qk.contiguous()
     skq = scores_kq.contiguous()
@@ -391,10 +407,8 @@ def select_topk(scores_qk, scores_kq, S: int, L: int, p: int, topk: int, tie: st
     inv = torch.empty(B, H, S_tot, dtype=torch.int32, device=dev) if with_inverse else None
     if with_inverse and S_tot != S_tot_expected:
         raise AssertionError("inverse map needs scores of exactly the pyramid length")
-    with torch.cuda.device(dev):
-        rc = lib().lh_select_topk(_ptr(sqk), _ptr(skq), _ptr(idx), _ptr(inv), B, H, S, L, p, topk,
-                                  TIE_MODES[tie], int(bool(strict)), _stream(dev))
-    _check(rc, "lh_select_topk")
+    _run("lh_select_topk", dev, _ptr(sqk), _ptr(skq), _ptr(idx), _ptr(inv), B, H, S, L, p, topk, TIE_MODES[tie],
+         int(bool(strict)))
     return idx, inv
 
 
@@ -409,9 +423,7 @@ def build_inverse(indices, S_tot: int, validate: bool = False):
     idx = indices.contiguous()
     B, H, n = idx.shape
     inv = torch.empty(B, H, S_tot, dtype=torch.int32, device=idx.device)
-    with torch.cuda.device(idx.device):
-        rc = lib().lh_build_inverse(_ptr(idx), n, _ptr(inv), S_tot, B, H, _stream(idx.device))
-    _check(rc, "lh_build_inverse")
+    _run("lh_build_inverse", idx.device, _ptr(idx), n, _ptr(inv), S_tot, B, H)
     return inv
 
 
@@ -509,10 +521,8 @@ def attn_fwd(rows: Rows, indices, B: int, H: int, n: int, D: int = D_SUPPORTED, 
     idx = indices.contiguous() if indices is not None else None
     out = torch.empty(B, H, n, D, dtype=rows.dtype, device=dev)
     lse = torch.empty(B, H, n, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        rc = lib().lh_attn_fwd_ex(*rows.args(), _ptr(idx), B, H, n, D, scale, _ptr(out), _ptr(lse), rows.dtype_code,
-                                  int(shaped), _stream(dev))
-    _check(rc, "lh_attn_fwd")
+    _run("lh_attn_fwd_ex", dev, *rows.args(), _ptr(idx), B, H, n, D, scale, _ptr(out), _ptr(lse), rows.dtype_code,
+         int(shaped))
     _check_queues(dev, "lh_attn_fwd")
     return out, lse
 
@@ -525,11 +535,8 @@ def attn_bwd_dkdv(rows: Rows, indices, B: int, H: int, n: int, dout, lse, delta,
     scale = D ** -0.5 if scale is None else scale
     idx = indices.contiguous() if indices is not None else None
     dk, dv = (torch.empty(B, H, n, D, dtype=rows.dtype, device=dev) for _ in range(2))
-    with torch.cuda.device(dev):
-        rc = lib().lh_attn_bwd_ex(1, *rows.args(), _ptr(idx), B, H, n, D, scale, _ptr(dout.contiguous()),
-                                  _ptr(lse), _ptr(delta), None, _ptr(dk), _ptr(dv), rows.dtype_code, 0,
-                                  _stream(dev))
-    _check(rc, "lh_attn_bwd_dkdv")
+    _run("lh_attn_bwd_ex", dev, 1, *rows.args(), _ptr(idx), B, H, n, D, scale, _ptr(dout.contiguous()), _ptr(lse),
+         _ptr(delta), None, _ptr(dk), _ptr(dv), rows.dtype_code, 0)
     _check_queues(dev, "lh_attn_bwd_dkdv")
     return dk, dv
 
@@ -543,11 +550,8 @@ def attn_bwd_dq(rows: Rows, indices, B: int, H: int, n: int, dout, lse, delta, D
     scale = D ** -0.5 if scale is None else scale
     idx = indices.contiguous() if indices is not None else None
     dq = torch.empty(B, H, n, D, dtype=rows.dtype, device=dev)
-    with torch.cuda.device(dev):
-        rc = lib().lh_attn_bwd_ex(2, *rows.args(), _ptr(idx), B, H, n, D, scale, _ptr(dout.contiguous()),
-                                  _ptr(lse), _ptr(delta), _ptr(dq), None, None, rows.dtype_code, int(shaped),
-                                  _stream(dev))
-    _check(rc, "lh_attn_bwd_dq")
+    _run("lh_attn_bwd_ex", dev, 2, *rows.args(), _ptr(idx), B, H, n, D, scale, _ptr(dout.contiguous()), _ptr(lse),
+         _ptr(delta), _ptr(dq), None, None, rows.dtype_code, int(shaped))
     _check_queues(dev, "lh_attn_bwd_dq")
     return dq
 
@@ -562,10 +566,8 @@ def attn_bwd(rows: Rows, indices, B: int, H: int, n: int, dout, lse, delta, D: i
     idx = indices.contiguous() if indices is not None else None
     dout = dout.contiguous()
     dq, dk, dv = (torch.empty(B, H, n, D, dtype=rows.dtype, device=dev) for _ in range(3))
-    with torch.cuda.device(dev):
-        rc = lib().lh_attn_bwd_ex(3, *rows.args(), _ptr(idx), B, H, n, D, scale, _ptr(dout), _ptr(lse), _ptr(delta),
-                                  _ptr(dq), _ptr(dk), _ptr(dv), rows.dtype_code, int(shaped), _stream(dev))
-    _check(rc, "lh_attn_bwd")
+    _run("lh_attn_bwd_ex", dev, 3, *rows.args(), _ptr(idx), B, H, n, D, scale, _ptr(dout), _ptr(lse), _ptr(delta),
+         _ptr(dq), _ptr(dk), _ptr(dv), rows.dtype_code, int(shaped))
     _check_queues(dev, "lh_attn_bwd")
     return dq, dk, dv
 
@@ -584,10 +586,8 @@ def attn_delta(dout, o):
     st = [s if size > 1 else 0 for s, size in zip(dout.stride(), dout.shape)]
     rows = dout if dout.is_contiguous() else torch.empty(dout.shape, dtype=dout.dtype, device=dout.device)
     delta = torch.empty(B, H, n, dtype=torch.float32, device=dout.device)
-    with torch.cuda.device(dout.device):
-        rc = lib().lh_attn_delta(_ptr(dout), *st[:3], _ptr(o), None if rows is dout else _ptr(rows), _ptr(delta),
-                                 B, H, n, D, dt, _stream(dout.device))
-    _check(rc, "lh_attn_delta")
+    _run("lh_attn_delta", dout.device, _ptr(dout), *st[:3], _ptr(o), None if rows is dout else _ptr(rows),
+         _ptr(delta), B, H, n, D, dt)
     return rows, delta
 
 
@@ -608,10 +608,8 @@ def scatter_fwd(attn, inverse, S: int, S_out: int, L: int, p: int, seq_major: bo
     else:
         out = torch.empty(B, H, S_out, D, dtype=attn.dtype, device=attn.device)
     ob, oh, os_, od = out.stride()
-    with torch.cuda.device(attn.device):
-        rc = lib().lh_scatter_fwd_nd(_ptr(attn), _ptr(inverse), _ptr(out), ob, oh, os_, B, H, S, S_out, n, D, L, p,
-                                  dt, _stream(attn.device))
-    _check(rc, "lh_scatter_fwd")
+    _run("lh_scatter_fwd_nd", attn.device, _ptr(attn), _ptr(inverse), _ptr(out), ob, oh, os_, B, H, S, S_out, n, D, L,
+         p, dt)
     return out
 
 
@@ -622,7 +620,7 @@ def scatter_bwd(dout, indices, o, S: int, L: int, p: int):
     _need_dtype("scatter_bwd indices", torch.int32, indices)
     _need_gpu(dout, indices, o)
     if _check_mode():
-        check_indices(indices, 0, pyramid_lengths(S, L, p)[2], unique=True, what="scatter_bwd indices")
+        check_indices(indices, 0, pyramid_total(S, L, p), unique=True, what="scatter_bwd indices")
     if dout.stride(3) != 1 or any(st % 8 for st in dout.stride()[:3]) or dout.data_ptr() % 16:
         dout = own_rows(dout)
     B, H, S_out, D = dout.shape
@@ -631,10 +629,8 @@ def scatter_bwd(dout, indices, o, S: int, L: int, p: int):
     delta = torch.empty(B, H, n, dtype=torch.float32, device=dout.device) if o is not None else None
     oc = o.contiguous() if o is not None else None
     db, dh, ds, _ = dout.stride()
-    with torch.cuda.device(dout.device):
-        rc = lib().lh_scatter_bwd_nd(_ptr(dout), db, dh, ds, _ptr(indices.contiguous()), _ptr(oc), _ptr(dattn),
-                                  _ptr(delta), B, H, S, S_out, n, D, L, p, dt, _stream(dout.device))
-    _check(rc, "lh_scatter_bwd")
+    _run("lh_scatter_bwd_nd", dout.device, _ptr(dout), db, dh, ds, _ptr(indices.contiguous()), _ptr(oc), _ptr(dattn),
+         _ptr(delta), B, H, S, S_out, n, D, L, p, dt)
     return dattn, delta
 
 
@@ -653,10 +649,8 @@ def pyramid_bwd(gq, gk, gv, inverse, B: int, S: int, H: int, L: int, p: int, D: 
     gb, gh, gs, _ = ref.stride()
     for g in (gq, gk, gv):
         assert g is None or tuple(g.stride()) == (gb, gh, gs, 1), "selected grads must share strides"
-    with torch.cuda.device(dev):
-        rc = lib().lh_pyramid_bwd_nd(_ptr(gq), _ptr(gk), _ptr(gv), gb, gh, gs, _ptr(inverse),
-                                  _ptr(outs[0]), _ptr(outs[1]), _ptr(outs[2]), B, S, H, D, L, p, dt, _stream(dev))
-    _check(rc, "lh_pyramid_bwd")
+    _run("lh_pyramid_bwd_nd", dev, _ptr(gq), _ptr(gk), _ptr(gv), gb, gh, gs, _ptr(inverse), _ptr(outs[0]),
+         _ptr(outs[1]), _ptr(outs[2]), B, S, H, D, L, p, dt)
     return tuple(outs)
 
 
@@ -674,11 +668,8 @@ def pyramid_rope_bwd(gq, gk, gv, inverse, freqs, B: int, S: int, H: int, L: int,
     W = 3 * H * D
     dx = torch.empty(B, S, W, dtype=torch.bfloat16, device=dev)
     base, e = dx.data_ptr(), dx.element_size()
-    with torch.cuda.device(dev):
-        rc = lib().lh_pyramid_rope_bwd(_ptr(gq), _ptr(gk), _ptr(gv), gb, gh, gs, _ptr(inverse), _ptr(freqs),
-                                       base, base + H * D * e, base + 2 * H * D * e, S * W, W, D,
-                                       B, S, H, D, L, p, _stream(dev))
-    _check(rc, "lh_pyramid_rope_bwd")
+    _run("lh_pyramid_rope_bwd", dev, _ptr(gq), _ptr(gk), _ptr(gv), gb, gh, gs, _ptr(inverse), _ptr(freqs), base,
+         base + H * D * e, base + 2 * H * D * e, S * W, W, D, B, S, H, D, L, p)
     return dx
 
 
@@ -700,10 +691,7 @@ def rope_qkv_fwd(x, freqs, Hq: int, Hkv: int, D: int = D_SUPPORTED):
     q = torch.empty(B, S, Hq, D, dtype=torch.bfloat16, device=dev)
     k = torch.empty(B, S, Hkv, D, dtype=torch.bfloat16, device=dev)
     v = torch.empty(B, S, Hkv, D, dtype=torch.bfloat16, device=dev)
-    with torch.cuda.device(dev):
-        rc = lib().lh_rope_qkv_fwd(_ptr(x), x.stride(1), _ptr(freqs), _ptr(q), _ptr(k), _ptr(v), B, S, Hq, Hkv, D,
-                                   _stream(dev))
-    _check(rc, "lh_rope_qkv_fwd")
+    _run("lh_rope_qkv_fwd", dev, _ptr(x), x.stride(1), _ptr(freqs), _ptr(q), _ptr(k), _ptr(v), B, S, Hq, Hkv, D)
     return q, k, v
 
 
@@ -721,10 +709,8 @@ def rope_qkv_bwd(dq, dk, dv, freqs, Hq: int, Hkv: int, D: int = D_SUPPORTED):
     st = (ctypes.c_int64 * 9)(*[int(s) for g in (dq, dk, dv) for s in g.stride()[:3]])
     for g in (dq, dk, dv):
         assert g.stride(3) == 1, "head dimension must be contiguous"
-    with torch.cuda.device(dev):
-        rc = lib().lh_rope_qkv_bwd(_ptr(dq), _ptr(dk), _ptr(dv), ctypes.cast(st, _P), _ptr(freqs), _ptr(dx),
-                                   dx.stride(1), B, S, Hq, Hkv, D, _stream(dev))
-    _check(rc, "lh_rope_qkv_bwd")
+    _run("lh_rope_qkv_bwd", dev, _ptr(dq), _ptr(dk), _ptr(dv), ctypes.cast(st, _P), _ptr(freqs), _ptr(dx),
+         dx.stride(1), B, S, Hq, Hkv, D)
     return dx
 
 
@@ -738,9 +724,7 @@ def rmsnorm_fwd(x, w, eps: float):
     rows = x.numel() // dim
     y = torch.empty_like(x)
     rstd = torch.empty(x.shape[:-1], dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
-        rc = lib().lh_rmsnorm_fwd(_ptr(x), _ptr(w), _ptr(y), _ptr(rstd), rows, dim, float(eps), _stream(x.device))
-    _check(rc, "lh_rmsnorm_fwd")
+    _run("lh_rmsnorm_fwd", x.device, _ptr(x), _ptr(w), _ptr(y), _ptr(rstd), rows, dim, float(eps))
     return y, rstd
 
 
@@ -755,10 +739,8 @@ def add_rmsnorm_fwd(x, r, w, eps: float):
     h = torch.empty_like(x)
     y = torch.empty_like(x)
     rstd = torch.empty(x.shape[:-1], dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
-        rc = lib().lh_add_rmsnorm_fwd(_ptr(x), _ptr(r), _ptr(w), _ptr(h), _ptr(y), _ptr(rstd), rows, dim, float(eps),
-                                      _stream(x.device))
-    _check(rc, "lh_add_rmsnorm_fwd")
+    _run("lh_add_rmsnorm_fwd", x.device, _ptr(x), _ptr(r), _ptr(w), _ptr(h), _ptr(y), _ptr(rstd), rows, dim,
+         float(eps))
     return h, y, rstd
 
 
@@ -779,10 +761,8 @@ def rmsnorm_bwd(dy, x, w, rstd, dres=None):
     dw = torch.empty(w.shape, dtype=w.dtype, device=w.device)
     parts = min(RMSNORM_BWD_PARTS, rows)
     part = torch.empty(dim, parts, dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
-        rc = lib().lh_rmsnorm_bwd(_ptr(dy), _ptr(x), _ptr(w), _ptr(rstd), _ptr(dres), _ptr(dx), _ptr(dw),
-                                  _ptr(part), parts, rows, dim, _stream(x.device))
-    _check(rc, "lh_rmsnorm_bwd")
+    _run("lh_rmsnorm_bwd", x.device, _ptr(dy), _ptr(x), _ptr(w), _ptr(rstd), _ptr(dres), _ptr(dx), _ptr(dw),
+         _ptr(part), parts, rows, dim)
     return dx, dw
 
 
@@ -794,9 +774,7 @@ def swiglu_fwd(h):
     F2 = h.shape[-1]
     rows = h.numel() // F2
     a = torch.empty(*h.shape[:-1], F2 // 2, dtype=torch.bfloat16, device=h.device)
-    with torch.cuda.device(h.device):
-        rc = lib().lh_swiglu_fwd(_ptr(h), _ptr(a), rows, F2 // 2, _stream(h.device))
-    _check(rc, "lh_swiglu_fwd")
+    _run("lh_swiglu_fwd", h.device, _ptr(h), _ptr(a), rows, F2 // 2)
     return a
 
 
@@ -807,9 +785,7 @@ def swiglu_bwd(da, h):
     F2 = h.shape[-1]
     rows = h.numel() // F2
     dh = torch.empty(h.shape, dtype=h.dtype, device=h.device)
-    with torch.cuda.device(h.device):
-        rc = lib().lh_swiglu_bwd(_ptr(da), _ptr(h), _ptr(dh), rows, F2 // 2, _stream(h.device))
-    _check(rc, "lh_swiglu_bwd")
+    _run("lh_swiglu_bwd", h.device, _ptr(da), _ptr(h), _ptr(dh), rows, F2 // 2)
     return dh
 
 
@@ -818,7 +794,5 @@ def splitk_sum(part):
     _need_gpu(part)
     part = part.contiguous()
     out = torch.empty(part.shape[1:], dtype=torch.bfloat16, device=part.device)
-    with torch.cuda.device(part.device):
-        rc = lib().lh_splitk_sum(_ptr(part), _ptr(out), part.shape[0], out.numel(), _stream(part.device))
-    _check(rc, "lh_splitk_sum")
+    _run("lh_splitk_sum", part.device, _ptr(part), _ptr(out), part.shape[0], out.numel())
     return out

@@ -135,7 +135,7 @@ def _layer_fwd(xq, xk, xv, L, p, topk, tie, strict, dilation, seq_major, gk=None
     ``saved = (pq, pk, pv, inv, o, lse)``.  ``scale``: the attention (and scorer)
     scale, 1/sqrt(D) when None."""
     B, S, H, D = xq.shape
-    _, _, S_tot = N.pyramid_lengths(S, L, p)
+    S_tot = N.pyramid_total(S, L, p)
     _, _, _, S_sel = N.geometry(S, L, p, topk, strict)
     _mark("fwd_start")
     if gk is not None:
@@ -419,7 +419,7 @@ class _CompiledOps:
         @layer_fwd.register_fake
         def _(xq, xk, xv, L, p, topk, tie, strict, dilation, seq_major, gk, scale):
             B, S, H, D = xq.shape
-            _, _, S_tot = N.pyramid_lengths(S, L, p)
+            S_tot = N.pyramid_total(S, L, p)
             S_sel = N.geometry(S, L, p, topk, strict)[3]
             out = xq.new_empty(B, S, H, D).transpose(1, 2) if seq_major else xq.new_empty(B, H, S, D)
             pooled = [xq.new_empty(B, S_tot - S, H, D) for _ in range(3)]
@@ -463,7 +463,7 @@ class _CompiledOps:
         def _(xqkv, freqs, H, L, p, topk, tie, strict, seq_major):
             B, S, W = xqkv.shape
             D = W // (3 * H)
-            _, _, S_tot = N.pyramid_lengths(S, L, p)
+            S_tot = N.pyramid_total(S, L, p)
             S_sel = N.geometry(S, L, p, topk, strict)[3]
             e = xqkv.new_empty
             out = e(B, S, H, D).transpose(1, 2) if seq_major else e(B, H, S, D)
@@ -512,7 +512,7 @@ class _PyramidCatFn(torch.autograd.Function):
         if D0 < D:
             xq, xk, xv = (torch.nn.functional.pad(x, (0, D - D0)) for x in (xq, xk, xv))
         xq, xk, xv = N.own_rows(xq), N.own_rows(xk), N.own_rows(xv)
-        _, _, S_tot = N.pyramid_lengths(S, L, p)
+        S_tot = N.pyramid_total(S, L, p)
         cats = [torch.empty(B, S_tot, H, D, dtype=xq.dtype, device=xq.device) for _ in range(3)]
         for c, x in zip(cats, (xq, xk, xv)):
             c[:, :S].copy_(x)
