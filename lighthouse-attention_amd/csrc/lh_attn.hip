@@ -1837,21 +1837,27 @@ __device__ __forceinline__ void gla_state_update(floatx16 (&hs)[2], float el, co
       vt[e] = cvt2<T>(lo, hi);
     }
 #pragma unroll
-    for (int q = 0; q < 2; ++q) hs[q] = mfma<T>(vt, lds_tr(Kt, ll, 16 * kk, sib + q), hs[q]);
+    for (int q = 0; q < 2; ++q) hs[q] = mfma<T>(lds_tr(Kt, ll, 16 * kk, sib + q), vt, hs[q]);
   }
 }
 
-// Copy of this wave's state blocks, rounded to the element type, into the LDS operand H^T
+// Copy of this wave's state blocks, rounded to the element type, into the LDS
+// operand H^T.  A lane holds four consecutive i of one j per group of slots: one
+// 8-byte store (with the accumulators the other way round, j in the slots, these
+// were 32 two-byte stores per lane and chunk, a quarter of the chunk's time).
 template <typename T>
 __device__ __forceinline__ void gla_state_copy(bf16_t (*HT)[TILE], const floatx16 (&hs)[2], int sjb, int sib,
                                                int l32, int hh) {
+  const int j = 32 * sjb + l32;
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
-    const int i = 32 * (sib + q) + l32;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int j = 32 * sjb + slot_key(v, hh);
-      HT[j >> 6][tile_elem(j & 63, i)] = (bf16_t)(cvt2<T>(hs[q][v], 0.f) & 0xffffu);
+    for (int g = 0; g < 4; ++g) {
+      const int i = 32 * (sib + q) + 8 * g + 4 * hh;
+      u32x2 w;
+      w.x = cvt2<T>(hs[q][4 * g + 0], hs[q][4 * g + 1]);
+      w.y = cvt2<T>(hs[q][4 * g + 2], hs[q][4 * g + 3]);
+      *reinterpret_cast<u32x2*>(&HT[j >> 6][tile_elem(j & 63, i)]) = w;
     }
   }
 }
