@@ -309,6 +309,17 @@ int lh_pyramid_bwd_nd(const void *gq, const void *gk, const void *gv, int64_t gb
                       int p, int dtype, void *stream);
 
 /*
+ * lh_pyramid_fwd_nd with the outputs of the scorer modules
+ * (src/lighthouse_selection.py:610-616): cq, ck, cv [B, S_tot, H, D] (element
+ * strides cb, cs, ch) receive the base rows and behind them the pooled rows,
+ * row_qk and row_kq [B, H, S_tot] every score in the row type.  scores_* as there.
+ */
+int lh_pyramid_cat(const void *xq, const void *xk, const void *xv, int64_t sb, int64_t ss, int64_t sh,
+                   void *cq, void *ck, void *cv, int64_t cb, int64_t cs, int64_t ch, float *scores_qk,
+                   float *scores_kq, void *row_qk, void *row_kq, int B, int S, int H, int D, int L, int p,
+                   int base_scores_given, int dtype, void *stream);
+
+/*
  * The softmax backward's row term of an attention without a fan-out:
  * delta fp32 [B, H, n] = rowsum(dout * o), fp32 sums.  dout is [B, H, n, D] with
  * element strides (db, dh, ds), each a multiple of 8, D contiguous; o is

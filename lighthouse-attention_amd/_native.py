@@ -84,6 +84,8 @@ _SIGS = {
                             _I, _I, _I, _I, _F, _P, _P, _I, _I, _P]),
     "lh_attn_bwd_ex": (_I, [_I, _P, _P, _P, _L, _L, _L, _P, _P, _P, _L, _L, _L, _I, _P,
                             _I, _I, _I, _I, _F, _P, _P, _P, _P, _P, _P, _I, _I, _P]),
+    "lh_pyramid_cat": (_I, [_P, _P, _P, _L, _L, _L, _P, _P, _P, _L, _L, _L, _P, _P, _P, _P,
+                            _I, _I, _I, _I, _I, _I, _I, _I, _P]),
     "lh_attn_delta": (_I, [_P, _L, _L, _L, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     "lh_attn_status": (_I, [_P]),
     "lh_attn_queue_slot": (_I, [_P, _P]),
@@ -308,6 +310,28 @@ def pyramid_fwd(xq, xk, xv, L: int, p: int, scores=None, pooled_out=None):
     _run("lh_pyramid_fwd_nd", dev, _ptr(xq), _ptr(xk), _ptr(xv), sb, ss, sh, _ptr(pq), _ptr(pk), _ptr(pv), pb, ps, ph,
          _ptr(sqk), _ptr(skq), B, S, H, D, L, p, given, dt)
     return pq, pk, pv, sqk, skq
+
+
+def pyramid_cat(xq, xk, xv, L: int, p: int, scores=None):
+    """The pyramids as the scorer modules return them, in one pass over contiguous
+    ``xq/xk/xv`` [B, S, H, D]: ``(scores_qk, scores_kq [B, H, S_tot] in the row type, three
+    [B, S_tot, H, D] of base and pooled rows)``.  ``scores``: fp32 [B, H, S_tot] whose base
+    level is given and whose other levels are filled in."""
+    _need_gpu(xq, xk, xv)
+    dt = _need_rows("pyramid_cat", xq, xk, xv)
+    B, S, H, D = xq.shape
+    assert xq.is_contiguous() and xk.is_contiguous() and xv.is_contiguous()
+    S_tot = pyramid_total(S, L, p)
+    dev = xq.device
+    cats = [torch.empty(B, S_tot, H, D, dtype=xq.dtype, device=dev) for _ in range(3)]
+    rows = [torch.empty(B, H, S_tot, dtype=xq.dtype, device=dev) for _ in range(2)]
+    given = scores is not None
+    if not given:
+        scores = [torch.empty(B, H, S_tot, dtype=torch.float32, device=dev) for _ in range(2)]
+    HD = H * D
+    _run("lh_pyramid_cat", dev, _ptr(xq), _ptr(xk), _ptr(xv), S * HD, HD, D, *[_ptr(c) for c in cats], S_tot * HD, HD,
+         D, _ptr(scores[0]), _ptr(scores[1]), _ptr(rows[0]), _ptr(rows[1]), B, S, H, D, L, p, int(given), dt)
+    return (*rows, *cats)
 
 
 def _check_freqs(freqs, S: int, D: int):

@@ -27,6 +27,8 @@ struct PyrArgs {
   const float* fs;   // rotary (cos, sin) table [>= S, D/2, 2] (ROPE)
   bf16_t *rq, *rk;   // rotated base rows out (ROPE)
   int64_t rb, rs, rh;
+  bf16_t *cq, *ck, *cv;  // CAT: base rows out (strides pb, ps, ph)
+  bf16_t *hq, *hk;       // CAT: all levels' scores in the row type, [B, H, S_tot]
   int B, S, H, D, L, shift, S_tot, nspan, cmax, units;
   int off[9], len[9];
 };
@@ -74,7 +76,11 @@ __device__ __forceinline__ void pyr_token(const PyrArgs& a, int b, int h, int l1
 // position's angles, rounded to bf16 and written to rq / rk, and the norms and
 // means below are taken of those rounded rows, exactly as if the rotated rows
 // had been stored first and read back.
-template <typename T, typename Ln, int NL, bool GIVEN, bool ROPE>
+// CAT: the scorer modules' form, whose outputs are the concatenated pyramids: the
+// base rows are written out as they stream by (in front of the pooled rows, as
+// three separate copies they were read a second time: 71 us of a 285 us scorer
+// call at 8 x 32768 rows) and every score also in the row type.
+template <typename T, typename Ln, int NL, bool GIVEN, bool ROPE, bool CAT>
 __global__ __launch_bounds__(256) void pyramid_fwd_kernel(const PyrArgs a) {
   const int tid = threadIdx.x;
   const int u = blockIdx.x * Ln::ROWS + tid / Ln::LPR;
@@ -104,14 +110,26 @@ __global__ __launch_bounds__(256) void pyramid_fwd_kernel(const PyrArgs a) {
       __attribute__((always_inline)) {
     float fq[8], fk[8], fv[8];
     pyr_token<T, Ln, GIVEN, ROPE>(a, b, h, l16, srow, t, xq, xk, xv, fq, fk, fv, sq, sk);
-    if (!GIVEN) {
+    if (CAT && in) {
+      const int64_t co = (int64_t)b * a.pb + (int64_t)t * a.ps + (int64_t)h * a.ph + 8 * l16;
+      *reinterpret_cast<uint4*>(a.cq + co) = xq;
+      *reinterpret_cast<uint4*>(a.ck + co) = xk;
+      *reinterpret_cast<uint4*>(a.cv + co) = xv;
+    }
+    if (!GIVEN || CAT) {
       // base scores leave LPR tokens at a time: lane j keeps token t0 + LPR i + j,
       // and the group stores them as one contiguous run per tensor
       const int j = (t - t0) & (Ln::LPR - 1);
       if (l16 == j) { bq = sq; bk = sk; }
       if ((j == Ln::LPR - 1 || t == t1 - 1) && l16 <= j) {
-        a.sqk[srow + t - j + l16] = bq;
-        a.skq[srow + t - j + l16] = bk;
+        if (!GIVEN) {
+          a.sqk[srow + t - j + l16] = bq;
+          a.skq[srow + t - j + l16] = bk;
+        }
+        if (CAT) {
+          a.hq[srow + t - j + l16] = (bf16_t)(T::pack2(bq, 0.f) & 0xffffu);
+          a.hk[srow + t - j + l16] = (bf16_t)(T::pack2(bk, 0.f) & 0xffffu);
+        }
       }
     }
 #pragma unroll
@@ -139,6 +157,10 @@ __global__ __launch_bounds__(256) void pyramid_fwd_kernel(const PyrArgs a) {
         if (l16 == 0) {
           a.sqk[srow + a.off[lvl] + node] = mq[l];
           a.skq[srow + a.off[lvl] + node] = mk[l];
+          if (CAT) {
+            a.hq[srow + a.off[lvl] + node] = (bf16_t)(T::pack2(mq[l], 0.f) & 0xffffu);
+            a.hk[srow + a.off[lvl] + node] = (bf16_t)(T::pack2(mk[l], 0.f) & 0xffffu);
+          }
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) { accq[l][e] = 0.f; acck[l][e] = 0.f; accv[l][e] = 0.f; }
@@ -256,15 +278,19 @@ template <typename T, int NL>
 int launch_fwd(const PyrArgs& a, bool given, hipStream_t st) {
   if (a.fs) {  // D == LH_D
     using Ln = Lanes<16, true>;
-    hipLaunchKernelGGL((pyramid_fwd_kernel<BF16, Ln, NL, false, true>), dim3((a.units + Ln::ROWS - 1) / Ln::ROWS),
+    hipLaunchKernelGGL((pyramid_fwd_kernel<BF16, Ln, NL, false, true, false>), dim3((a.units + Ln::ROWS - 1) / Ln::ROWS),
                        dim3(256), 0, st, a);
   } else {
     LH_DISPATCH_LANES(a.D, {
       const dim3 grid((a.units + Ln::ROWS - 1) / Ln::ROWS);
-      if (given)
-        hipLaunchKernelGGL((pyramid_fwd_kernel<T, Ln, NL, true, false>), grid, dim3(256), 0, st, a);
+      if (a.cq && given)
+        hipLaunchKernelGGL((pyramid_fwd_kernel<T, Ln, NL, true, false, true>), grid, dim3(256), 0, st, a);
+      else if (a.cq)
+        hipLaunchKernelGGL((pyramid_fwd_kernel<T, Ln, NL, false, false, true>), grid, dim3(256), 0, st, a);
+      else if (given)
+        hipLaunchKernelGGL((pyramid_fwd_kernel<T, Ln, NL, true, false, false>), grid, dim3(256), 0, st, a);
       else
-        hipLaunchKernelGGL((pyramid_fwd_kernel<T, Ln, NL, false, false>), grid, dim3(256), 0, st, a);
+        hipLaunchKernelGGL((pyramid_fwd_kernel<T, Ln, NL, false, false, false>), grid, dim3(256), 0, st, a);
     });
   }
   LH_CHECK_LAUNCH();
@@ -281,7 +307,7 @@ int pyramid_fwd_impl(const void* xq, const void* xk, const void* xv, int64_t sb,
                      const float* freqs, void* rq, void* rk, int64_t rb, int64_t rs, int64_t rh,
                      void* pq, void* pk, void* pv, int64_t pb, int64_t ps, int64_t ph,
                      float* scores_qk, float* scores_kq, int B, int S, int H, int D, int L, int p,
-                     bool given, int dtype, void* stream) {
+                     bool given, int dtype, void* stream, void* const* cat = nullptr) {
   if (!lanes_supported(D) || (freqs && D != LH_D)) return LH_ERR_UNSUPPORTED;
   if (!valid_dtype(dtype) || (freqs && dtype != LH_DTYPE_BF16)) return LH_ERR_INVALID_ARG;
   if (!xq || !xk || !xv || !scores_qk || !scores_kq || B <= 0 || H <= 0 || S <= 0) return LH_ERR_INVALID_ARG;
@@ -304,6 +330,13 @@ int pyramid_fwd_impl(const void* xq, const void* xk, const void* xv, int64_t sb,
   a.sqk = scores_qk; a.skq = scores_kq;
   a.fs = freqs; a.rq = (bf16_t*)rq; a.rk = (bf16_t*)rk;
   a.rb = rb; a.rs = rs; a.rh = rh;
+  if (cat) {
+    for (int i = 0; i < 5; ++i)
+      if (!cat[i] || (i < 3 && !aligned16(cat[i]))) return LH_ERR_INVALID_ARG;
+    if ((pb | ps | ph) % 8) return LH_ERR_INVALID_ARG;
+    a.cq = (bf16_t*)cat[0]; a.ck = (bf16_t*)cat[1]; a.cv = (bf16_t*)cat[2];
+    a.hq = (bf16_t*)cat[3]; a.hk = (bf16_t*)cat[4];
+  }
   a.B = B; a.S = S; a.H = H; a.D = D; a.L = L; a.shift = shift; a.S_tot = g.total;
   a.cmax = ipow(p, L - 1);
   if (a.cmax > 4096) return LH_ERR_UNSUPPORTED;
@@ -394,6 +427,18 @@ extern "C" int lh_pyramid_fwd(const void* xq, const void* xk, const void* xv, in
   if (D != LH_D) return LH_ERR_UNSUPPORTED;
   return lh_pyramid_fwd_nd(xq, xk, xv, sb, ss, sh, pq, pk, pv, pb, ps, ph, scores_qk, scores_kq, B, S, H, D, L, p,
                            base_scores_given, dtype, stream);
+}
+
+extern "C" int lh_pyramid_cat(const void* xq, const void* xk, const void* xv, int64_t sb, int64_t ss, int64_t sh,
+                              void* cq, void* ck, void* cv, int64_t cb, int64_t cs, int64_t ch, float* scores_qk,
+                              float* scores_kq, void* row_qk, void* row_kq, int B, int S, int H, int D, int L, int p,
+                              int base_scores_given, int dtype, void* stream) {
+  if (!cq || !ck || !cv || S <= 0) return LH_ERR_INVALID_ARG;
+  void* const cat[5] = {cq, ck, cv, row_qk, row_kq};
+  bf16_t* pool[3];
+  for (int i = 0; i < 3; ++i) pool[i] = (bf16_t*)cat[i] + (int64_t)S * cs;  // the pooled rows follow the base rows
+  return pyramid_fwd_impl(xq, xk, xv, sb, ss, sh, nullptr, nullptr, nullptr, 0, 0, 0, pool[0], pool[1], pool[2], cb, cs,
+                          ch, scores_qk, scores_kq, B, S, H, D, L, p, base_scores_given != 0, dtype, stream, cat);
 }
 
 extern "C" int lh_rope_pyramid_fwd(const void* xq, const void* xk, const void* xv, int64_t sb, int64_t ss,

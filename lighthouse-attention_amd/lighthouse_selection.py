@@ -506,27 +506,25 @@ class _PyramidCatFn(torch.autograd.Function):
     from 104 to 120 run zero-padded (the padded columns of the returned rows are cut off)."""
 
     @staticmethod
-    def forward(ctx, xq, xk, xv, L, p, dilation, base_qk=None, base_kq=None):
+    def forward(ctx, xq, xk, xv, L, p, dilation, base_qk=None, base_kq=None, full=False):
         B, S, H, D0 = xq.shape
         D = N.padded_dim(D0)
         if D0 < D:
             xq, xk, xv = (torch.nn.functional.pad(x, (0, D - D0)) for x in (xq, xk, xv))
         xq, xk, xv = N.own_rows(xq), N.own_rows(xk), N.own_rows(xv)
         S_tot = N.pyramid_total(S, L, p)
-        cats = [torch.empty(B, S_tot, H, D, dtype=xq.dtype, device=xq.device) for _ in range(3)]
-        for c, x in zip(cats, (xq, xk, xv)):
-            c[:, :S].copy_(x)
-        if base_qk is not None:  # base-level scores computed by the caller ([B, H, S])
+        if base_qk is None:
+            scores = N.dilated_scores(xq, xk, xv, dilation, S_tot, D0 ** -0.5) if dilation else None
+        elif full:  # [B, H, S_tot] buffers of a native scorer, base level filled
+            scores = (base_qk, base_kq)
+        else:  # base-level scores computed by the caller ([B, H, S])
             scores = tuple(torch.empty(B, H, S_tot, dtype=torch.float32, device=xq.device) for _ in range(2))
             scores[0][..., :S].copy_(base_qk)
             scores[1][..., :S].copy_(base_kq)
-        else:
-            scores = N.dilated_scores(xq, xk, xv, dilation, S_tot, D0 ** -0.5) if dilation else None
-        _, _, _, sqk, skq = N.pyramid_fwd(xq, xk, xv, L, p, scores=scores,
-                                          pooled_out=tuple(c[:, S:] for c in cats))
+        sqk, skq, *cats = N.pyramid_cat(xq, xk, xv, L, p, scores)
         ctx.geo = (B, S, H, D, L, p, D0)
         ctx.mark_non_differentiable(sqk, skq)
-        return (sqk.to(xq.dtype), skq.to(xq.dtype), *(c[..., :D0].transpose(1, 2) for c in cats))
+        return (sqk, skq, *(c[..., :D0].transpose(1, 2) for c in cats))
 
     @staticmethod
     def backward(ctx, _g1, _g2, gq, gk, gv):
@@ -534,13 +532,13 @@ class _PyramidCatFn(torch.autograd.Function):
         gs = [g if g is not None else None for g in (gq, gk, gv)]
         ref = next((g for g in gs if g is not None), None)
         if ref is None:
-            return None, None, None, None, None, None, None, None
+            return (None,) * 9
         gs = [g if g is not None else torch.zeros_like(ref) for g in gs]
         if D0 < D:
             gs = [torch.nn.functional.pad(g, (0, D - D0)) for g in gs]
         gs = [N.own_rows(g) for g in gs]
         dx = N.pyramid_bwd(*gs, None, B, S, H, L, p, D)
-        return dx[0][..., :D0], dx[1][..., :D0], dx[2][..., :D0], None, None, None, None, None
+        return dx[0][..., :D0], dx[1][..., :D0], dx[2][..., :D0], None, None, None, None, None, None
 
 
 class _GatheredAttnFn(torch.autograd.Function):
@@ -716,7 +714,7 @@ class DilatedLighthouseGLAScorer(nn.Module):
         _, _, S_tot = N.pyramid_lengths(s, self.levels, self.pooling_factor)
         with torch.no_grad():
             sqk, skq = N.gla_scores(*_gla_rows(xq, xk, xv), gk.detach(), self.dilation, S_tot, self.scaling)
-        return _PyramidCatFn.apply(xq, xk, xv, self.levels, self.pooling_factor, 0, sqk[..., :s], skq[..., :s])
+        return _PyramidCatFn.apply(xq, xk, xv, self.levels, self.pooling_factor, 0, sqk, skq, True)
 
 
 class LighthouseLocal(nn.Module):

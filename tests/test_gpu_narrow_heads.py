@@ -146,3 +146,31 @@ def test_attn_delta(pkg, dev, D, dtype):
         # fp32 sums of D products of 16-bit values: D roundings at most
         bound = D * 2.0 ** -24 * (f.double() * o.double()).abs().sum(-1)
         assert bool(((delta.double() - ref).abs() <= bound).all()), f"form {i}"
+
+
+@pytest.mark.parametrize("D,S,L,p,dtype", [(128, 1000, 3, 4, torch.bfloat16), (72, 257, 2, 2, torch.float16),
+                                           (64, 1030, 4, 2, torch.bfloat16), (128, 96, 1, 2, torch.float16)])
+@pytest.mark.parametrize("given", [False, True])
+def test_pyramid_cat(pkg, dev, D, S, L, p, dtype, given):
+    """The one-pass scorer outputs: base rows, pooled rows and scores are those of
+    pyramid_fwd, with S not a multiple of the spans or of the lanes' score runs."""
+    N = pkg._native
+    B, H = 2, 3
+    g = torch.Generator().manual_seed(S)
+    xs = [torch.randn(B, S, H, D, generator=g).to(dtype).to(dev) for _ in range(3)]
+    S_tot = N.pyramid_total(S, L, p)
+    base = [torch.rand(B, H, S, generator=g).to(dtype).float().to(dev) for _ in range(2)]
+
+    def scores():
+        if not given:
+            return None
+        buf = [torch.full((B, H, S_tot), -1.0, device=dev) for _ in range(2)]
+        for x, y in zip(buf, base):
+            x[..., :S] = y
+        return buf
+
+    want = N.pyramid_fwd(*xs, L, p, scores=scores())
+    sqk, skq, *cats = N.pyramid_cat(*xs, L, p, scores())
+    for c, x, pool in zip(cats, xs, want[:3]):
+        assert torch.equal(c[:, :S], x) and torch.equal(c[:, S:], pool)
+    assert torch.equal(sqk, want[3].to(dtype)) and torch.equal(skq, want[4].to(dtype))
