@@ -16,6 +16,8 @@
 // so there are no atomics and the result is deterministic.
 #include "lh_common.h"
 
+#include <algorithm>
+
 namespace {
 
 struct PyrArgs {
@@ -195,6 +197,74 @@ __global__ __launch_bounds__(256) void pyramid_fwd_kernel(const PyrArgs a) {
   }
 }
 
+// The forward for few spans.  pyramid_fwd_kernel has one group walk the
+// p^(L-1) tokens of a span, four loads in flight, so a short sequence leaves
+// most of the chip idle and waits for memory several times in a row (8 heads of
+// 2048 tokens: 64 blocks, 15 us).  Here a block takes a tile of tokens of one
+// (b, h), whole spans, with one token per group at a time, keeps their rows in
+// LDS, and then its groups share the pooled nodes, (level, node, tensor) each,
+// summing a node's tokens in their order: the same bits as the walk.
+constexpr int PYR_TILE = 64;  // most tokens of a tile: spans longer than that take the walk
+
+template <typename T, typename Ln, bool ROPE>
+__global__ __launch_bounds__(256) void pyramid_tile_kernel(const PyrArgs a, int tt) {
+  __shared__ uint4 X[3][PYR_TILE * Ln::LPR];
+  __shared__ float SC[2][PYR_TILE];
+  const int tid = threadIdx.x, g = tid / Ln::LPR, l16 = tid % Ln::LPR;
+  const bool in = Ln::in(l16, a.D);
+  const int chunks = (a.S + tt - 1) / tt;
+  const int bh = blockIdx.x / chunks, b = bh / a.H, h = bh - b * a.H;
+  const int t0 = (blockIdx.x - bh * chunks) * tt;
+  const size_t srow = (size_t)bh * a.S_tot;
+  const int64_t xoff = (int64_t)b * a.sb + (int64_t)h * a.sh + 8 * l16;
+  const uint4 zero = make_uint4(0, 0, 0, 0);
+  for (int i = g; i < tt && t0 + i < a.S; i += Ln::ROWS) {
+    const int t = t0 + i;
+    const int64_t o = xoff + (int64_t)t * a.ss;
+    const uint4 xq = in ? ld16(a.xq + o) : zero, xk = in ? ld16(a.xk + o) : zero, xv = in ? ld16(a.xv + o) : zero;
+    float fq[8], fk[8], fv[8], sq, sk;
+    pyr_token<T, Ln, false, ROPE>(a, b, h, l16, srow, t, xq, xk, xv, fq, fk, fv, sq, sk);
+    X[0][i * Ln::LPR + l16] = ROPE ? pack8_t<T>(fq) : xq;  // the rotated rows' own 16 bits
+    X[1][i * Ln::LPR + l16] = ROPE ? pack8_t<T>(fk) : xk;
+    X[2][i * Ln::LPR + l16] = xv;
+    if (l16 == 0) {
+      SC[0][i] = sq;
+      SC[1][i] = sk;
+    }
+  }
+  __syncthreads();
+  if (tid < 2 * PYR_TILE) {
+    const int i = tid & (PYR_TILE - 1);
+    if (i < tt && t0 + i < a.S) (tid < PYR_TILE ? a.sqk : a.skq)[srow + t0 + i] = SC[tid / PYR_TILE][i];
+  }
+  int task = g;
+  for (int lvl = 2; lvl <= a.L; ++lvl) {
+    const int cs = (lvl - 1) * a.shift, c = 1 << cs, nodes = tt >> cs;
+    for (; task < 3 * nodes; task += Ln::ROWS) {
+      const int x = task / nodes, i = task - x * nodes, node = (t0 >> cs) + i;
+      if (node >= a.len[lvl]) continue;
+      float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0}, mx = -INFINITY;
+      for (int j = i << cs; j < (i + 1) << cs; ++j) {
+        float f[8];
+        unpack8_t<T>(X[x][j * Ln::LPR + l16], f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] += f[e];
+        if (x < 2) mx = fmaxf(mx, SC[x][j]);
+      }
+      const float inv_c = 1.0f / (float)c;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] *= inv_c;
+      const int r = a.off[lvl] + node;
+      bf16_t* pool = x == 0 ? a.pq : x == 1 ? a.pk : a.pv;
+      if (in)
+        *reinterpret_cast<uint4*>(pool + (int64_t)b * a.pb + (int64_t)(r - a.S) * a.ps + (int64_t)h * a.ph + 8 * l16) =
+            pack8_t<T>(acc);
+      if (x < 2 && l16 == 0) (x ? a.skq : a.sqk)[srow + r] = mx;
+    }
+    task -= 3 * nodes;
+  }
+}
+
 struct PyrBwdArgs {
   const bf16_t *gq, *gk, *gv;
   int64_t gb, gh, gs;
@@ -274,8 +344,31 @@ __global__ __launch_bounds__(256) void pyramid_bwd_kernel(const PyrBwdArgs a) {
   if (a.dv) store16_nt(a.dv + o, pack8_t<T>(fv));
 }
 
+// Tokens of a pyramid_tile_kernel block, 0 where the walk is taken: the tiles
+// win while the walk has at most a wave per CU, with the rotation's extra loads
+// up to four.  Cold caches, walk / tiles: 8 heads, L = 3, p = 4, 2048 tokens
+// 25.4 / 20.8 us, 4096 26.7 / 26.9, 8192 33.0 / 39.0; with rotation 33.0 / 22.3,
+// 8192 46.7 / 43.4, 32768 109 / 122; L = 4 (spans of 64) 8192 66.7 / 48.2.
+int tile_tokens(const PyrArgs& a, bool given) {
+  if (given || a.cq || a.cmax > PYR_TILE) return 0;
+  const int rows = a.D <= 64 ? 32 : 16;
+  const int waves = (a.units + rows / 4 - 1) / (rows / 4);
+  return waves <= (a.fs ? 1024 : 256) ? std::max(rows, a.cmax) : 0;
+}
+
 template <typename T, int NL>
 int launch_fwd(const PyrArgs& a, bool given, hipStream_t st) {
+  if (const int tt = tile_tokens(a, given)) {
+    const dim3 grid(a.B * a.H * ((a.S + tt - 1) / tt));
+    if (a.fs) {
+      using Ln = Lanes<16, true>;
+      hipLaunchKernelGGL((pyramid_tile_kernel<BF16, Ln, true>), grid, dim3(256), 0, st, a, tt);
+    } else {
+      LH_DISPATCH_LANES(a.D, hipLaunchKernelGGL((pyramid_tile_kernel<T, Ln, false>), grid, dim3(256), 0, st, a, tt));
+    }
+    LH_CHECK_LAUNCH();
+    return LH_OK;
+  }
   if (a.fs) {  // D == LH_D
     using Ln = Lanes<16, true>;
     hipLaunchKernelGGL((pyramid_fwd_kernel<BF16, Ln, NL, false, true, false>), dim3((a.units + Ln::ROWS - 1) / Ln::ROWS),
