@@ -1751,14 +1751,16 @@ struct GlaArgs {
 constexpr int GLA_WS_WAVE = 2 * 16 * 64;  // fp32 state values held by one wave
 constexpr int GLA_WS_SEG = 8 * GLA_WS_WAVE;
 
+// Wave w of the NW that share a tile's loads
+template <int NW>
 __device__ __forceinline__ void gla_issue(bf16_t* tile, const bf16_t* base, uint32_t stride, int t0, int last,
                                           int w, int lane) {
   const int rsub = lane >> 4, slot = lane & 15;
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int r = 8 * w + 4 * i + rsub;
+  for (int i = 0; i < 16 / NW; ++i) {
+    const int r0 = (64 / NW) * w + 4 * i, r = r0 + rsub;
     const int t = min(t0 + r, last);
-    g2l16(base + (uint32_t)t * stride + 8 * (slot ^ swz(r)), tile + (8 * w + 4 * i) * LH_D);
+    g2l16(base + (uint32_t)t * stride + 8 * (slot ^ swz(r)), tile + r0 * LH_D);
   }
 }
 
@@ -1895,8 +1897,8 @@ __global__ __launch_bounds__(512, 1) void gla_state_kernel(const GlaArgs a) {
 
   auto issue = [&](int c, int buf) {
     const int t0 = 64 * c;
-    gla_issue(Kt[buf], sq.kb, sq.stride, t0, last, w, lane);
-    gla_issue(Vt[buf], sq.vb, sq.stride, t0, last, w, lane);
+    gla_issue<8>(Kt[buf], sq.kb, sq.stride, t0, last, w, lane);
+    gla_issue<8>(Vt[buf], sq.vb, sq.stride, t0, last, w, lane);
     if (w == 0) g2l4(sq.gb + (int64_t)min(t0 + lane, last) * sq.VH, Gs[buf]);
   };
   issue(c0, 0);
@@ -1935,7 +1937,9 @@ __global__ __launch_bounds__(512, 1) void gla_state_kernel(const GlaArgs a) {
 //      double-buffered), so that phase A of the next chunk starts at once.
 // Tiles of chunk c + 2 are issued at the start of phase B of chunk c, into the
 // buffers chunk c has just released, and waited for at the end of phase A of
-// chunk c + 1.
+// chunk c + 1.  Waves 4-7 issue them: waves 0-3 carry phase B's longest chain
+// (the A^T blocks), and with the loads spread over all eight the two passes took
+// 132 instead of 128 us at 8 x 32768 tokens.
 template <typename E>
 __global__ __launch_bounds__(512, 1) void gla_scores_kernel(const GlaArgs a) {
   __shared__ __attribute__((aligned(1024))) bf16_t Qt[2][TILE];
@@ -1976,10 +1980,11 @@ __global__ __launch_bounds__(512, 1) void gla_scores_kernel(const GlaArgs a) {
 
   auto issue = [&](int c, int buf) {
     const int t0 = 64 * c;
-    gla_issue(Qt[buf], sq.qb, sq.stride, t0, last, w, lane);
-    gla_issue(Kt[buf], sq.kb, sq.stride, t0, last, w, lane);
-    gla_issue(Vt[buf], sq.vb, sq.stride, t0, last, w, lane);
-    if (w == 0) g2l4(sq.gb + (int64_t)min(t0 + lane, last) * sq.VH, Gs[buf]);
+    if (w < 4) return;
+    gla_issue<4>(Qt[buf], sq.qb, sq.stride, t0, last, w - 4, lane);
+    gla_issue<4>(Kt[buf], sq.kb, sq.stride, t0, last, w - 4, lane);
+    gla_issue<4>(Vt[buf], sq.vb, sq.stride, t0, last, w - 4, lane);
+    if (w == 4) g2l4(sq.gb + (int64_t)min(t0 + lane, last) * sq.VH, Gs[buf]);
   };
   // A^T blocks (waves 0-2) and decay factors (wave 3) of chunk c from buffer buf
   auto prep = [&](int c, int buf) {
