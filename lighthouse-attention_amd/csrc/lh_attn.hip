@@ -2300,13 +2300,20 @@ int wq_grid(int nblk, int BH, hipStream_t st, WorkQ& q) {
 }
 
 // Whether a query-stationary launch over BH (b, h) of length n runs half blocks
-// (fwd_half_block).  Both ways are estimated in units of 10 ns, with measured
-// constants: a step costs 1.57 us (one tile of 256 queries) or 2.07 us (two of
-// 128) while most of the chip idles, which bounds a launch by its heaviest
-// block, and 2.25 or 2.55 us when all CUs run, plus 7 us for each block of a CU
-// in turn, which bounds it by its share of the whole work.  Half blocks are
-// taken when they are estimated 5% shorter; the estimate is within 10% of the
-// measured time on both sides for 8 to 36 heads of 1152 to 18432 rows.
+// (fwd_half_block).  Both ways are estimated in units of 10 ns of the forward at
+// D = 128, with measured constants: a step costs 1.57 us (one tile of 256
+// queries) or 2.1 us (two of 128) while most of the chip idles, which bounds a
+// launch by its heaviest block, and 1.9 or 2.12 us when all CUs run, plus 7 us
+// for each block of a CU in turn, which bounds it by its share of the whole
+// work; with more blocks than CUs some CU also takes two of the middle ones.
+// dQ and the narrower heads have other times but nearly the same ratios.  Half
+// blocks are taken when they are estimated 7% shorter.  Over 66 shapes of 1 to
+// 256 heads and 256 to 14000 rows at D = 64, 72 and 128 the choice was within 3%
+// of the better side in 379 of 396 forwards and dQs, and within 15% in all (32
+// heads of 2029 rows, forward at D = 64).  The middle blocks' bound is what
+// keeps 64 heads of 744 rows on whole blocks (D = 64: 23 / 27 against 28 / 31 us).
+// Forward / dQ, whole -> half: 12 heads of 6000 rows 157 / 203 -> 140 / 178 us at
+// D = 128, 115 / 125 -> 95 / 105 at 64; 8 of 10236 at 64 188 / 201 -> 168 / 185.
 bool half_blocks(int BH, int n) {
   const int cus = cu_count();
   if (cus <= 0) return false;
@@ -2314,9 +2321,12 @@ bool half_blocks(int BH, int n) {
     const long long nb = (n + rows - 1) / rows, per = (long long)rows / BN / tiles_per_step;
     const long long heavy = ((n + BN - 1) / BN + tiles_per_step - 1) / tiles_per_step;
     const long long steps = per * nb * (nb - 1) / 2 + heavy;
-    return std::max(heavy * chain + 700, BH * (steps * load + nb * 700) / cus);
+    long long t = std::max(heavy * chain + 700, BH * (steps * load + nb * 700) / cus);
+    if (nb * BH > cus)  // the (cus)th and (cus + 1)th heaviest share a CU at best
+      t = std::max(t, (2 * nb - (cus - 1) / BH - cus / BH) * per * chain + 1400);
+    return t;
   };
-  return est(HB, 2, 207, 255) * 105 < est(32 * QW, 1, 157, 225) * 100;
+  return est(HB, 2, 210, 212) * 107 < est(32 * QW, 1, 157, 190) * 100;
 }
 
 // Grid of a query-stationary launch: a packed plan where one applies, else as wq_grid.

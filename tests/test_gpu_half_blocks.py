@@ -24,7 +24,9 @@ def _inputs(n, H, dtype, dev, gathered):
 @pytest.mark.parametrize("n,H,dtype,gathered", [
     (65, 2, torch.bfloat16, True), (127, 1, torch.bfloat16, False), (128, 2, torch.float16, True),
     (129, 2, torch.bfloat16, True), (193, 3, torch.float16, False), (1000, 2, torch.bfloat16, True),
-    (4608, 8, torch.bfloat16, True), (4780, 12, torch.float16, False)])
+    (4608, 8, torch.bfloat16, True), (4780, 12, torch.float16, False),
+    # either side of the rule's bound by shared CUs: 64 heads take whole blocks, 12 of 6000 half blocks
+    (744, 64, torch.bfloat16, False), (6000, 12, torch.float16, True)])
 def test_half_blocks(pkg, dev, n, H, dtype, gathered):
     N = pkg._native
     print(f"half blocks n={n} H={H} {dtype} gathered={gathered}", flush=True)
