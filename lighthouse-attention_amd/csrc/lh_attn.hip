@@ -1731,12 +1731,12 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(const AttnArgs a,
 // .. + 63) with a copy rounded to the row type in LDS as the operand of the
 // inter-chunk product (fp16 rows: fp16 MFMAs, an fp16 state copy).
 // As in the forward kernel, products come out transposed (A^T, O^T), so an
-// accumulator column is a token.  Per chunk: phase 1 (waves 0-2) forms the
-// three causal 32x32 blocks of A^T and hands them over in LDS as packed
-// operands, wave 3 the decay factors; phase 2 every wave forms one 32-token x
-// 32-column block of O^T (norm partials to LDS) and updates its state blocks;
-// phase 3 writes the new state copy and wave 7 finishes the norms.  Tiles
-// of the next chunk are loaded (direct global->LDS) during the current one.
+// accumulator column is a token.  A chunk needs: the three causal 32x32 blocks of
+// A^T (waves 0-2; handed over in LDS as packed operands) and the decay factors
+// (wave 3); one 32-token x 32-column block of O^T (norm partials to LDS) and the
+// state blocks' update of every wave; the new state copy and the norms (wave 7).
+// gla_scores_kernel says how these are split into phases.  Tiles of later chunks
+// are loaded (direct global->LDS) meanwhile.
 // ===========================================================================
 struct GlaArgs {
   const bf16_t *q, *k, *v;  // [B, S, H, D] contiguous
