@@ -1044,9 +1044,12 @@ __device__ __forceinline__ void dq_tile(floatx16 (&acc)[Hd::DB], float& rsum, co
 // keys (|c|^2 about 2 against 126) skip it and give the uncentred result.
 // Every wave forms the same sums in the same order, so the choice is uniform.
 // HALF: a block of HB rows, the key tiles shared out as in fwd_half_block and
-// the two halves' sums joined through LDS.
+// the two halves' sums joined through LDS; K0 .. V1 are then the first group's
+// four tiles of eight, one after the other.  Otherwise they are LDS arrays of
+// their own (carved from one array, 48 more address adds in the loop).
 template <typename T, typename Hd, bool HALF>
-__device__ __forceinline__ void dq_block(const AttnArgs& a, int bh, int qb, bf16_t* KV, float* kc) {
+__device__ __forceinline__ void dq_block(const AttnArgs& a, int bh, int qb, bf16_t* K0, bf16_t* V0, bf16_t* K1,
+                                         bf16_t* V1, float* kc) {
   constexpr int BM = HALF ? HB : 32 * QW;
   constexpr int G = HALF ? 2 : 1;    // key groups
   constexpr int NW = QW / G;         // waves that fill a tile
@@ -1055,11 +1058,20 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, int bh, int qb, bf16
   const int lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = wave / NW, wl = wave % NW;
-  bf16_t *K0 = KV + grp * 4 * Hd::TILE, *V0 = K0 + Hd::TILE, *K1 = K0 + 2 * Hd::TILE, *V1 = K0 + 3 * Hd::TILE;
+  bf16_t* const KV = K0;
   const int n = a.n, D = head_dim<Hd>(a);
   if (!Hd::FULL && D < 16 * Hd::C) {  // each block anew: a half block's join overwrites the tiles
-    zero_tails(KV, 4 * G * Hd::TILE);
+    if (HALF)
+      zero_tails(KV, 8 * Hd::TILE);
+    else
+      for (bf16_t* t : {K0, V0, K1, V1}) zero_tails(t, Hd::TILE);
     __syncthreads();
+  }
+  if (HALF) {
+    K0 += grp * 4 * Hd::TILE;
+    V0 += grp * 4 * Hd::TILE;
+    K1 += grp * 4 * Hd::TILE;
+    V1 += grp * 4 * Hd::TILE;
   }
   const BhRows m = bh_rows(a, bh);
   const int q0 = qb * BM, qw = q0 + wl * 32, my_q = qw + l32;
@@ -1168,7 +1180,11 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, int bh, int qb, bf16
     const int t = G * j + grp, k0 = t * BN;
     if (t + G < nt) issue_rows<Hd, NW>(Kn, m.k, m.kp, Vn, m.v, m.vp, m, rr, D, wl, lane);
     if (t + 2 * G < nt) load_rows<Hd, NW>(rr, m, k0 + 2 * G * BN, wl, lane);
-    if (t < nt && k0 <= qw + 31)
+    // likely: else the tile's blocks are laid out behind the loop's other ones, one
+    // more jump per step.  With the arrays of their own 834 -> 830 us at 8 heads of
+    // 18432 rows, 200 -> 198 at 16 of 8192 and D = 64, 266 -> 263 at 72; the arrays
+    // alone 873 -> 879 at D = 128.
+    if (__builtin_expect(t < nt && k0 <= qw + 31, 1))
       dq_tile<T, Hd, decltype(C)::value>(acc, rsum, qf, df, Ks, Vs, k0, my_q, n, lane, a.sl2, nlse, dlt, t >= nfull);
     wait_loads();
     __syncthreads();
@@ -1221,7 +1237,10 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, int bh, int qb, bf16
 
 template <typename T, typename Hd>
 __global__ __launch_bounds__(64 * QW, 8 / QW) void attn_bwd_dq_kernel(const AttnArgs a, const QPlan p, const WorkQ q) {
-  __shared__ __attribute__((aligned(1024))) bf16_t KV[4 * Hd::TILE];
+  __shared__ __attribute__((aligned(1024))) bf16_t K0[Hd::TILE];
+  __shared__ __attribute__((aligned(1024))) bf16_t K1[Hd::TILE];
+  __shared__ __attribute__((aligned(1024))) bf16_t V0[Hd::TILE];
+  __shared__ __attribute__((aligned(1024))) bf16_t V1[Hd::TILE];
   __shared__ __attribute__((aligned(16))) float KC[128 + QW * 132];  // key centre + per-wave partial sums
   __shared__ int wq_s[2];
   int bh, qb, bin = 0;
@@ -1234,7 +1253,7 @@ __global__ __launch_bounds__(64 * QW, 8 / QW) void attn_bwd_dq_kernel(const Attn
     if (!have && q.ctr) have = wq_next(q, a.nq, a.BH, true, -1, 0, bh, qb, wq_s);
   }
   for (int k = 1; have; ++k) {
-    dq_block<T, Hd, false>(a, bh, qb, KV, KC);
+    dq_block<T, Hd, false>(a, bh, qb, K0, V0, K1, V1, KC);
     // the next block starts after this one's last tile reads
     if (p.bph)
       have = plan_next(p, bin, k, qb);
@@ -1252,7 +1271,7 @@ __global__ __launch_bounds__(64 * QW, 8 / QW) void attn_bwd_dq_half_kernel(const
   bool have = wq_first(q, a.nq, a.BH, true, bh, qb);
   if (!have && q.ctr) have = wq_next(q, a.nq, a.BH, true, -1, 0, bh, qb, wq_s);
   for (int k = 1; have; ++k) {
-    dq_block<T, Hd, true>(a, bh, qb, KV, KC);
+    dq_block<T, Hd, true>(a, bh, qb, KV, KV + Hd::TILE, KV + 2 * Hd::TILE, KV + 3 * Hd::TILE, KC);
     have = q.ctr && wq_next(q, a.nq, a.BH, true, -1, k, bh, qb, wq_s);
   }
 }
