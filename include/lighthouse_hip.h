@@ -272,11 +272,9 @@ int lh_attn_bwd_dq(const void *q, const void *k, const void *v, int64_t sb, int6
 /*
  * lh_attn_fwd and lh_attn_bwd with flags (parts: bit 0 = dK/dV, bit 1 = dQ; the
  * outputs of a part that is not asked for may be NULL).  With LH_ATTN_SHAPED a
- * launch may split its work by its own sizes, B * H and n (here: half blocks of
- * 128 queries whose keys two halves of a workgroup share, where the heaviest
- * 256-query block would outlast the rest); the last bits of its results then
- * depend on them, while with flags = 0 a (b, h) has the same bits alone and
- * beside others.  Unknown bits give LH_ERR_INVALID_ARG.  D: 8..96 in steps of 8,
+ * launch may cut its work by its own sizes, B * H and n (here: query blocks of 128
+ * instead of 256 where the heaviest one would outlast the rest); the results
+ * are the same bits.  Unknown bits give LH_ERR_INVALID_ARG.  D: 8..96 in steps of 8,
  * or 128.
  */
 #define LH_ATTN_SHAPED 1

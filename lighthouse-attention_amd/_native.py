@@ -531,9 +531,8 @@ def attn_fwd(rows: Rows, indices, B: int, H: int, n: int, D: int = D_SUPPORTED, 
              shaped: bool = False):
     """Causal attention over the rows named by ``indices`` [B, H, n] (None = identity).
 
-    ``shaped`` (LH_ATTN_SHAPED): the launch may split its work by B * H and n, and the
-    last bits of the result then depend on them; otherwise a (b, h) has the same bits
-    alone and beside others.
+    ``shaped`` (LH_ATTN_SHAPED): the launch may cut its work by B * H and n.  Either way
+    a (b, h) has the same bits alone and beside others.
 
     Returns ``(O [B, H, n, D] of the rows' dtype, lse fp32 [B, H, n])`` (lse in the
     exp2 domain)."""

@@ -50,7 +50,7 @@ namespace {
 
 constexpr int BMK = 128;  // keys per workgroup of the key-stationary kernel: 4 waves x 32
 constexpr int QW = 8;     // waves per workgroup of the query-stationary kernels (32 queries each)
-constexpr int HB = 128;   // queries per workgroup of the half-block kernels (two waves per 32 queries)
+constexpr int HW = 4;     // waves per workgroup of their half blocks (see half_blocks)
 constexpr int BN = 64;   // rows per LDS tile
 constexpr float RESCALE_LOG2 = 8.0f;
 constexpr int FWD_AHEAD = 4;  // forward: LDS operands read this many MFMAs ahead
@@ -271,8 +271,10 @@ struct WorkQ {
   // (64-bit: workgroups finished in the low half, blocks they ran in the high
   // half), [12] fault flag (sticky: the launches never clear it)
   unsigned* ctr;
-  int slots;  // workgroups per queue (grid / 8); their first blocks are not counted
+  int slots;  // workgroups per queue (grid / 8); their first blocks are not counted.
+              // WQ_SPREAD in a plain grid: heaviest blocks first over all (b, h)
 };
+constexpr int WQ_SPREAD = -1;
 constexpr int WQ_DRAINED = 8, WQ_DONE = 10, WQ_FAULT = 12, WQ_CLEAR = 12;
 
 // Set (bit 0) by a persistent launch whose blocks did not add up to its block
@@ -295,7 +297,13 @@ __device__ __forceinline__ void wq_decode(int x, int j, int nblk, int BH, bool h
 // First block of this workgroup; false when it has none.
 __device__ __forceinline__ bool wq_first(const WorkQ& q, int nblk, int BH, bool heavy_last, int& bh, int& blk) {
   if (!q.ctr) {
-    schedule(blockIdx.x, nblk, BH, bh, blk, heavy_last);
+    if (q.slots == WQ_SPREAD) {
+      blk = blockIdx.x / BH;
+      bh = blockIdx.x - blk * BH;
+      if (heavy_last) blk = nblk - 1 - blk;
+    } else {
+      schedule(blockIdx.x, nblk, BH, bh, blk, heavy_last);
+    }
     return true;
   }
   const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
@@ -502,11 +510,12 @@ __device__ __forceinline__ void issue_rows(bf16_t* tile, const bf16_t* base, con
   }
 }
 
-// Zeros in `elems` elements of LDS (a multiple of 4096) by all 512 threads: the
-// tiles of a head dim below 16 C, whose chunks past D no load writes.  The
-// caller's barrier follows.
+// Zeros in `elems` elements of LDS (a multiple of 4096) by all threads of NW
+// waves: the tiles of a head dim below 16 C, whose chunks past D no load writes.
+// The caller's barrier follows.
+template <int NW>
 __device__ __forceinline__ void zero_tails(bf16_t* t, int elems) {
-  for (int i = threadIdx.x; i < elems / 8; i += 512) reinterpret_cast<u32x4*>(t)[i] = u32x4{};
+  for (int i = threadIdx.x; i < elems / 8; i += 64 * NW) reinterpret_cast<u32x4*>(t)[i] = u32x4{};
 }
 
 // 16-byte operand slices 16 c + 8 hh of a row, zero past D
@@ -592,31 +601,6 @@ __device__ __forceinline__ void store_rows(bf16_t* row, const floatx16 (&acc)[Hd
       if (Hd::FULL || 32 * d + 8 * g < D) *reinterpret_cast<u32x2*>(row + d * 32 + 8 * g + 4 * hh) = w;
     }
   }
-}
-
-// Accumulators of a wave to and from LDS in register order (join: acc = f0 acc + f1 x)
-template <typename Hd>
-__device__ __forceinline__ void acc_store(float* lds, const floatx16 (&acc)[Hd::DB], int lane) {
-  float4* p = reinterpret_cast<float4*>(lds) + lane;
-#pragma unroll
-  for (int d = 0; d < Hd::DB; ++d)
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-      p[(4 * d + g) * 64] = float4{acc[d][4 * g], acc[d][4 * g + 1], acc[d][4 * g + 2], acc[d][4 * g + 3]};
-}
-template <typename Hd>
-__device__ __forceinline__ void acc_join(floatx16 (&acc)[Hd::DB], float f0, float f1, const float* lds, int lane) {
-  const float4* p = reinterpret_cast<const float4*>(lds) + lane;
-#pragma unroll
-  for (int d = 0; d < Hd::DB; ++d)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const float4 x = p[(4 * d + g) * 64];
-      acc[d][4 * g + 0] = fmaf(f0, acc[d][4 * g + 0], f1 * x.x);
-      acc[d][4 * g + 1] = fmaf(f0, acc[d][4 * g + 1], f1 * x.y);
-      acc[d][4 * g + 2] = fmaf(f0, acc[d][4 * g + 2], f1 * x.z);
-      acc[d][4 * g + 3] = fmaf(f0, acc[d][4 * g + 3], f1 * x.w);
-    }
 }
 
 #define SCHED_GROUP(mask, n) __builtin_amdgcn_sched_group_barrier(mask, n, 0)
@@ -730,11 +714,11 @@ __device__ __forceinline__ void fwd_tile(FwdState<Hd>& st, const u32x4 (&qf)[Hd:
   }
 }
 
-// One query block qb of (b, h) bh.
-template <typename T, typename Hd, int EPI>  // 0: O + LSE;  1: rounded row norms of O into `scores`
+// One query block qb of (b, h) bh: 32 queries for each of the NW waves.
+template <typename T, typename Hd, int NW, int EPI>  // 0: O + LSE;  1: rounded row norms of O into `scores`
 __device__ __forceinline__ void fwd_block(const AttnArgs& a, int bh, int qb, bf16_t* KV) {
   bf16_t *K0 = KV, *V0 = K0 + Hd::TILE, *K1 = K0 + 2 * Hd::TILE, *V1 = K0 + 3 * Hd::TILE;
-  constexpr int BM = 32 * QW;
+  constexpr int BM = 32 * NW;
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = a.n, D = head_dim<Hd>(a);
@@ -750,7 +734,7 @@ __device__ __forceinline__ void fwd_block(const AttnArgs& a, int bh, int qb, bf1
   const int q0 = qb * BM, qw = q0 + wave * 32, my_q = qw + l32;
 
   if (!Hd::FULL && D < 16 * Hd::C) {
-    zero_tails(KV, 4 * Hd::TILE);
+    zero_tails<NW>(KV, 4 * Hd::TILE);
     __syncthreads();
   }
   u32x4 qf[Hd::C];
@@ -762,10 +746,10 @@ __device__ __forceinline__ void fwd_block(const AttnArgs& a, int bh, int qb, bf1
 
   const int kend = min(q0 + BM, n);
   const int nt = (kend + BN - 1) / BN;
-  int rr[Hd::template loads<QW>()];
-  load_rows<Hd, QW>(rr, m, 0, wave, lane);
-  issue_rows<Hd, QW>(K0, m.k, m.kp, V0, m.v, m.vp, m, rr, D, wave, lane);
-  load_rows<Hd, QW>(rr, m, BN, wave, lane);
+  int rr[Hd::template loads<NW>()];
+  load_rows<Hd, NW>(rr, m, 0, wave, lane);
+  issue_rows<Hd, NW>(K0, m.k, m.kp, V0, m.v, m.vp, m, rr, D, wave, lane);
+  load_rows<Hd, NW>(rr, m, BN, wave, lane);
   wait_loads();
   __syncthreads();
 
@@ -779,8 +763,8 @@ __device__ __forceinline__ void fwd_block(const AttnArgs& a, int bh, int qb, bf1
 
   auto step = [&](int j, const bf16_t* Ks, const bf16_t* Vs, bf16_t* Kn, bf16_t* Vn) {
     const int k0 = j * BN;
-    if (j + 1 < nt) issue_rows<Hd, QW>(Kn, m.k, m.kp, Vn, m.v, m.vp, m, rr, D, wave, lane);
-    if (j + 2 < nt) load_rows<Hd, QW>(rr, m, k0 + 2 * BN, wave, lane);
+    if (j + 1 < nt) issue_rows<Hd, NW>(Kn, m.k, m.kp, Vn, m.v, m.vp, m, rr, D, wave, lane);
+    if (j + 2 < nt) load_rows<Hd, NW>(rr, m, k0 + 2 * BN, wave, lane);
     if (j < nt && k0 <= qw + 31) fwd_tile<T, Hd>(st, qf, Ks, Vs, k0, my_q, n, lane, a.sl2, j >= nfull);
     wait_loads();
     __syncthreads();
@@ -819,105 +803,8 @@ __device__ __forceinline__ void fwd_block(const AttnArgs& a, int bh, int qb, bf1
   }
 }
 
-// One query block of HB = 128 rows: waves w and w + 4 own the same 32 queries,
-// waves 0-3 take the even key tiles and waves 4-7 the odd ones, and the two
-// halves' states are joined through LDS at the end.  KV: 8 tiles, ML: 2 KB.
-//
-// Bound by the chain of one block's tiles, which it halves: a step of two tiles
-// takes about 1.3 times a step of one (twice the K/V copies for half the
-// queries), so it is for launches whose heaviest block outlasts the chip's
-// share of the work (half_blocks).  Forward / dQ, one box: 8 heads of 1152 rows
-// 35 / 43 -> 26 / 33 us, of 2048 59 / 73 -> 40 / 49, of 4608 119 / 149 -> 84 /
-// 104, of 7000 180 / 220 -> 126 / 164, 12 of 4780 124 / 157 -> 97 / 123; but 32
-// of 4608 184 / 240 -> 222 / 283 and 8 of 18432 646 / 847 -> 747 / 961.
-template <typename T, typename Hd>
-__device__ __forceinline__ void fwd_half_block(const AttnArgs& a, int bh, int qb, bf16_t* KV, float* ML) {
-  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), grp = wave >> 2, w4 = wave & 3;
-  const int n = a.n, D = head_dim<Hd>(a);
-  const BhRows m = bh_rows(a, bh);
-  const int q0 = qb * HB, qw = q0 + w4 * 32, my_q = qw + l32;
-
-  u32x4 qf[Hd::C];
-  {
-    bool pooled;
-    const uint32_t o = row_off(m, my_q, pooled);
-    load_operand<Hd>(qf, (pooled ? m.qp : m.q) + o, D, hh);
-  }
-
-  const int kend = min(q0 + HB, n);
-  const int nt = (kend + BN - 1) / BN, ns = (nt + 1) >> 1;  // key tiles, steps of two
-  // step j: tile 2 j + grp, in buffer j & 1 of this group
-  bf16_t *K0 = KV + grp * 4 * Hd::TILE, *V0 = K0 + Hd::TILE, *K1 = K0 + 2 * Hd::TILE, *V1 = K0 + 3 * Hd::TILE;
-  if (!Hd::FULL && D < 16 * Hd::C) {  // each block anew: the join below overwrites the tiles
-    zero_tails(KV, 8 * Hd::TILE);
-    __syncthreads();
-  }
-  int rr[Hd::template loads<4>()];
-  load_rows<Hd, 4>(rr, m, grp * BN, w4, lane);
-  issue_rows<Hd, 4>(K0, m.k, m.kp, V0, m.v, m.vp, m, rr, D, w4, lane);
-  load_rows<Hd, 4>(rr, m, (2 + grp) * BN, w4, lane);
-  wait_loads();
-  __syncthreads();
-
-  FwdState<Hd> st;
-#pragma unroll
-  for (int d = 0; d < Hd::DB; ++d) st.o[d] = floatx16{};
-  st.m = -INFINITY;
-  st.l = 0.f;
-  const int nfull = min((qw + 1) / BN, n / BN);
-
-  auto step = [&](int j, const bf16_t* Ks, const bf16_t* Vs, bf16_t* Kn, bf16_t* Vn) {
-    const int t = 2 * j + grp;
-    if (t + 2 < nt) issue_rows<Hd, 4>(Kn, m.k, m.kp, Vn, m.v, m.vp, m, rr, D, w4, lane);
-    if (t + 4 < nt) load_rows<Hd, 4>(rr, m, (t + 4) * BN, w4, lane);
-    if (t < nt && t * BN <= qw + 31) fwd_tile<T, Hd>(st, qf, Ks, Vs, t * BN, my_q, n, lane, a.sl2, t >= nfull);
-    wait_loads();
-    __syncthreads();
-  };
-  for (int j = 0; j < ns; j += 2) {
-    step(j, K0, V0, K1, V1);
-    step(j + 1, K1, V1, K0, V0);
-  }
-
-  // the odd tiles' state -> LDS (register order) -> the even tiles' waves
-  float* ox = reinterpret_cast<float*>(KV) + w4 * Hd::DB * 1024;
-  if (grp) {
-    acc_store<Hd>(ox, st.o, lane);
-    ML[w4 * 128 + lane] = st.m;
-    ML[w4 * 128 + 64 + lane] = st.l;
-  }
-  __syncthreads();
-  if (grp || my_q >= n) return;
-  const float m1 = ML[w4 * 128 + lane], l1 = ML[w4 * 128 + 64 + lane];
-  const float mx = fmaxf(st.m, m1);
-  // -inf: none of the half's keys is visible, or all their scores are -inf
-  const float f0 = st.m == -INFINITY ? 0.f : ex2((st.m - mx) * a.sl2);
-  const float f1 = m1 == -INFINITY ? 0.f : ex2((m1 - mx) * a.sl2);
-  float l = fmaf(f0, st.l, f1 * l1);
-  l += __shfl_xor(l, 32);
-  const float inv_l = l > 0.f ? 1.0f / l : 0.f;
-  acc_join<Hd>(st.o, f0, f1, ox, lane);
-  store_rows<T, Hd>(a.out + ((int64_t)bh * n + my_q) * D, st.o, inv_l, D, hh);
-  if (hh == 0) a.lse[(int64_t)bh * n + my_q] = l > 0.f ? mx * a.sl2 + __log2f(l) : -INFINITY;
-}
-
-template <typename T, typename Hd>
-__global__ __launch_bounds__(64 * QW, 8 / QW) void attn_fwd_half_kernel(const AttnArgs a, const WorkQ q) {
-  __shared__ __attribute__((aligned(1024))) bf16_t KV[8 * Hd::TILE];
-  __shared__ float ML[4 * 128];
-  __shared__ int wq_s[2];
-  int bh, qb;
-  bool have = wq_first(q, a.nq, a.BH, true, bh, qb);
-  if (!have && q.ctr) have = wq_next(q, a.nq, a.BH, true, -1, 0, bh, qb, wq_s);
-  for (int k = 1; have; ++k) {
-    fwd_half_block<T, Hd>(a, bh, qb, KV, ML);
-    have = q.ctr && wq_next(q, a.nq, a.BH, true, -1, k, bh, qb, wq_s);
-  }
-}
-
-template <typename T, typename Hd, int EPI>
-__global__ __launch_bounds__(64 * QW, 8 / QW) void attn_fwd_kernel(const AttnArgs a, const QPlan p, const WorkQ q) {
+template <typename T, typename Hd, int NW, int EPI>
+__global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fwd_kernel(const AttnArgs a, const QPlan p, const WorkQ q) {
   __shared__ __attribute__((aligned(1024))) bf16_t KV[4 * Hd::TILE];
   __shared__ int wq_s[2];
   int bh, qb, bin = 0;
@@ -930,7 +817,7 @@ __global__ __launch_bounds__(64 * QW, 8 / QW) void attn_fwd_kernel(const AttnArg
     if (!have && q.ctr) have = wq_next(q, a.nq, a.BH, true, -1, 0, bh, qb, wq_s);
   }
   for (int k = 1; have; ++k) {
-    fwd_block<T, Hd, EPI>(a, bh, qb, KV);
+    fwd_block<T, Hd, NW, EPI>(a, bh, qb, KV);
     // the next block starts after this one's last tile reads
     if (p.bph)
       have = plan_next(p, bin, k, qb);
@@ -1043,38 +930,21 @@ __device__ __forceinline__ void dq_tile(floatx16 (&acc)[Hd::DB], float& rsum, co
 // over the sample (|c| above a quarter of the keys' spread about it); N(0, 1)
 // keys (|c|^2 about 2 against 126) skip it and give the uncentred result.
 // Every wave forms the same sums in the same order, so the choice is uniform.
-// HALF: a block of HB rows, the key tiles shared out as in fwd_half_block and
-// the two halves' sums joined through LDS; K0 .. V1 are then the first group's
-// four tiles of eight, one after the other.  Otherwise they are LDS arrays of
-// their own (carved from one array, 48 more address adds in the loop).
-template <typename T, typename Hd, bool HALF>
+template <typename T, typename Hd, int NW>
 __device__ __forceinline__ void dq_block(const AttnArgs& a, int bh, int qb, bf16_t* K0, bf16_t* V0, bf16_t* K1,
                                          bf16_t* V1, float* kc) {
-  constexpr int BM = HALF ? HB : 32 * QW;
-  constexpr int G = HALF ? 2 : 1;    // key groups
-  constexpr int NW = QW / G;         // waves that fill a tile
+  constexpr int BM = 32 * NW;
   int tid = threadIdx.x;  // opaque, as in dkdv_block
   asm volatile("" : "+v"(tid));
   const int lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int grp = wave / NW, wl = wave % NW;
-  bf16_t* const KV = K0;
   const int n = a.n, D = head_dim<Hd>(a);
-  if (!Hd::FULL && D < 16 * Hd::C) {  // each block anew: a half block's join overwrites the tiles
-    if (HALF)
-      zero_tails(KV, 8 * Hd::TILE);
-    else
-      for (bf16_t* t : {K0, V0, K1, V1}) zero_tails(t, Hd::TILE);
+  if (!Hd::FULL && D < 16 * Hd::C) {
+    for (bf16_t* t : {K0, V0, K1, V1}) zero_tails<NW>(t, Hd::TILE);
     __syncthreads();
   }
-  if (HALF) {
-    K0 += grp * 4 * Hd::TILE;
-    V0 += grp * 4 * Hd::TILE;
-    K1 += grp * 4 * Hd::TILE;
-    V1 += grp * 4 * Hd::TILE;
-  }
   const BhRows m = bh_rows(a, bh);
-  const int q0 = qb * BM, qw = q0 + wl * 32, my_q = qw + l32;
+  const int q0 = qb * BM, qw = q0 + wave * 32, my_q = qw + l32;
   const int qc = min(my_q, n - 1);
 
   u32x4 qf[Hd::C], df[Hd::C];
@@ -1100,30 +970,36 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, int bh, int qb, bf16
   const int kend = min(q0 + BM, n);
   const int nt = (kend + BN - 1) / BN;
   int rr[Hd::template loads<NW>()];
-  load_rows<Hd, NW>(rr, m, grp * BN, wl, lane);
-  issue_rows<Hd, NW>(K0, m.k, m.kp, V0, m.v, m.vp, m, rr, D, wl, lane);
-  load_rows<Hd, NW>(rr, m, (G + grp) * BN, wl, lane);
-  // key sample for the centre: thread t reads 16 bytes (dims 8 (t % 16) ..) of
-  // sample rows t / 16 and t / 16 + 32, sample s at key (s kend) / 64
-  u32x4 ks0, ks1;
-  {
-    const int ch = tid & 15, s0 = tid >> 4;
+  load_rows<Hd, NW>(rr, m, 0, wave, lane);
+  issue_rows<Hd, NW>(K0, m.k, m.kp, V0, m.v, m.vp, m, rr, D, wave, lane);
+  load_rows<Hd, NW>(rr, m, BN, wave, lane);
+  // key sample for the centre: of the QW parts that its sums go by, wave w takes
+  // parts w, w + NW, ..; thread t of part p (t in [64 p, 64 p + 64)) reads 16 bytes
+  // (dims 8 (t % 16) ..) of sample rows t / 16 and t / 16 + 32, sample s at key
+  // (s cend) / 64, where cend ends the causal range of the whole block
+  constexpr int PARTS = QW / NW;
+  u32x4 ks0[PARTS], ks1[PARTS];
+  const int cend = min((q0 / (32 * QW) + 1) * (32 * QW), n);
+#pragma unroll
+  for (int u = 0; u < PARTS; ++u) {
+    const int ch = tid & 15, s0 = (tid + 64 * NW * u) >> 4;
     bool pooled;
-    uint32_t o = row_off(m, (s0 * kend) >> 6, pooled);
+    uint32_t o = row_off(m, (s0 * cend) >> 6, pooled);
     const bool in = Hd::FULL || 8 * ch < D;
-    ks0 = in ? ldg16((pooled ? m.kp : m.k) + o + 8 * ch) : u32x4{};
-    o = row_off(m, ((s0 + 32) * kend) >> 6, pooled);
-    ks1 = in ? ldg16((pooled ? m.kp : m.k) + o + 8 * ch) : u32x4{};
+    ks0[u] = in ? ldg16((pooled ? m.kp : m.k) + o + 8 * ch) : u32x4{};
+    o = row_off(m, ((s0 + 32) * cend) >> 6, pooled);
+    ks1[u] = in ? ldg16((pooled ? m.kp : m.k) + o + 8 * ch) : u32x4{};
   }
   wait_loads();
-  float* kcp = kc + 128;  // per wave: 128 dim sums, then the sum of squares
+  float* kcp = kc + 128;  // per part: 128 dim sums, then the sum of squares
   int ln = lane;  // opaque: its LDS addresses are not hoisted out of the block loop (they would spill)
   asm volatile("" : "+v"(ln));
-  {
+#pragma unroll
+  for (int u = 0; u < PARTS; ++u) {
     // sum the two rows, then over the four lanes of this wave that hold the
-    // same 8 dims, then over the waves in LDS; beside it the sum of squares
+    // same 8 dims, then over the parts in LDS; beside it the sum of squares
     float c8[8], k2 = 0.f;
-    const uint32_t w0[4] = {ks0.x, ks0.y, ks0.z, ks0.w}, w1[4] = {ks1.x, ks1.y, ks1.z, ks1.w};
+    const uint32_t w0[4] = {ks0[u].x, ks0[u].y, ks0[u].z, ks0[u].w}, w1[4] = {ks1[u].x, ks1[u].y, ks1[u].z, ks1[u].w};
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const float a0 = T::lo(w0[e]), a1 = T::hi(w0[e]);
@@ -1140,11 +1016,11 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, int bh, int qb, bf16
 #pragma unroll
     for (int x = 1; x < 64; x <<= 1) k2 += __shfl_xor(k2, x);
     if (ln < 16) {
-      float4* dst = reinterpret_cast<float4*>(kcp + wave * 132 + 8 * ln);
+      float4* dst = reinterpret_cast<float4*>(kcp + (wave + NW * u) * 132 + 8 * ln);
       dst[0] = float4{c8[0], c8[1], c8[2], c8[3]};
       dst[1] = float4{c8[4], c8[5], c8[6], c8[7]};
     }
-    if (ln == 0) kcp[wave * 132 + 128] = k2;
+    if (ln == 0) kcp[(wave + NW * u) * 132 + 128] = k2;
   }
   __syncthreads();
   bool ctr;
@@ -1175,44 +1051,31 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, int bh, int qb, bf16
   float rsum = 0.f;
   const int nfull = min((qw + 1) / BN, n / BN);
 
-  // step j: key tile G j + grp
   auto step = [&](auto C, int j, const bf16_t* Ks, const bf16_t* Vs, bf16_t* Kn, bf16_t* Vn) {
-    const int t = G * j + grp, k0 = t * BN;
-    if (t + G < nt) issue_rows<Hd, NW>(Kn, m.k, m.kp, Vn, m.v, m.vp, m, rr, D, wl, lane);
-    if (t + 2 * G < nt) load_rows<Hd, NW>(rr, m, k0 + 2 * G * BN, wl, lane);
+    const int k0 = j * BN;
+    if (j + 1 < nt) issue_rows<Hd, NW>(Kn, m.k, m.kp, Vn, m.v, m.vp, m, rr, D, wave, lane);
+    if (j + 2 < nt) load_rows<Hd, NW>(rr, m, k0 + 2 * BN, wave, lane);
     // likely: else the tile's blocks are laid out behind the loop's other ones, one
     // more jump per step.  With the arrays of their own 834 -> 830 us at 8 heads of
     // 18432 rows, 200 -> 198 at 16 of 8192 and D = 64, 266 -> 263 at 72; the arrays
     // alone 873 -> 879 at D = 128.
-    if (__builtin_expect(t < nt && k0 <= qw + 31, 1))
-      dq_tile<T, Hd, decltype(C)::value>(acc, rsum, qf, df, Ks, Vs, k0, my_q, n, lane, a.sl2, nlse, dlt, t >= nfull);
+    if (__builtin_expect(j < nt && k0 <= qw + 31, 1))
+      dq_tile<T, Hd, decltype(C)::value>(acc, rsum, qf, df, Ks, Vs, k0, my_q, n, lane, a.sl2, nlse, dlt, j >= nfull);
     wait_loads();
     __syncthreads();
   };
-  const int ns = (nt + G - 1) / G;
   if (ctr) {
-    for (int j = 0; j < ns; j += 2) {
+    for (int j = 0; j < nt; j += 2) {
       step(std::true_type{}, j, K0, V0, K1, V1);
       step(std::true_type{}, j + 1, K1, V1, K0, V0);
     }
   } else {
-    for (int j = 0; j < ns; j += 2) {
+    for (int j = 0; j < nt; j += 2) {
       step(std::false_type{}, j, K0, V0, K1, V1);
       step(std::false_type{}, j + 1, K1, V1, K0, V0);
     }
   }
 
-  if (HALF) {  // the odd tiles' sums -> LDS (register order) -> the even tiles' waves
-    float* ax = reinterpret_cast<float*>(KV) + wl * Hd::DB * 1024;
-    if (grp) {
-      acc_store<Hd>(ax, acc, ln);
-      kcp[wl * 64 + ln] = rsum;
-    }
-    __syncthreads();
-    if (grp) return;
-    rsum += kcp[wl * 64 + ln];
-    acc_join<Hd>(acc, 1.0f, 1.0f, ax, ln);
-  }
   // the two lane halves hold the two halves of each row's keys
   rsum += __shfl_xor(rsum, 32);
   if (my_q >= n) return;
@@ -1235,8 +1098,8 @@ __device__ __forceinline__ void dq_block(const AttnArgs& a, int bh, int qb, bf16
   }
 }
 
-template <typename T, typename Hd>
-__global__ __launch_bounds__(64 * QW, 8 / QW) void attn_bwd_dq_kernel(const AttnArgs a, const QPlan p, const WorkQ q) {
+template <typename T, typename Hd, int NW>
+__global__ __launch_bounds__(64 * NW, 8 / NW) void attn_bwd_dq_kernel(const AttnArgs a, const QPlan p, const WorkQ q) {
   __shared__ __attribute__((aligned(1024))) bf16_t K0[Hd::TILE];
   __shared__ __attribute__((aligned(1024))) bf16_t K1[Hd::TILE];
   __shared__ __attribute__((aligned(1024))) bf16_t V0[Hd::TILE];
@@ -1253,26 +1116,12 @@ __global__ __launch_bounds__(64 * QW, 8 / QW) void attn_bwd_dq_kernel(const Attn
     if (!have && q.ctr) have = wq_next(q, a.nq, a.BH, true, -1, 0, bh, qb, wq_s);
   }
   for (int k = 1; have; ++k) {
-    dq_block<T, Hd, false>(a, bh, qb, K0, V0, K1, V1, KC);
+    dq_block<T, Hd, NW>(a, bh, qb, K0, V0, K1, V1, KC);
     // the next block starts after this one's last tile reads
     if (p.bph)
       have = plan_next(p, bin, k, qb);
     else
       have = q.ctr && wq_next(q, a.nq, a.BH, true, -1, k, bh, qb, wq_s);
-  }
-}
-
-template <typename T, typename Hd>
-__global__ __launch_bounds__(64 * QW, 8 / QW) void attn_bwd_dq_half_kernel(const AttnArgs a, const WorkQ q) {
-  __shared__ __attribute__((aligned(1024))) bf16_t KV[8 * Hd::TILE];
-  __shared__ __attribute__((aligned(16))) float KC[128 + QW * 132];
-  __shared__ int wq_s[2];
-  int bh, qb;
-  bool have = wq_first(q, a.nq, a.BH, true, bh, qb);
-  if (!have && q.ctr) have = wq_next(q, a.nq, a.BH, true, -1, 0, bh, qb, wq_s);
-  for (int k = 1; have; ++k) {
-    dq_block<T, Hd, true>(a, bh, qb, KV, KV + Hd::TILE, KV + 2 * Hd::TILE, KV + 3 * Hd::TILE, KC);
-    have = q.ctr && wq_next(q, a.nq, a.BH, true, -1, k, bh, qb, wq_s);
   }
 }
 
@@ -1709,7 +1558,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_dkdv_kernel(const AttnArgs a,
   __shared__ int wq_s[2];
   const DkdvLds lds{Q0, Q1, Q2, Q3, D0, D1, D2, D3, L0, L1, L2, L3, EX, IX};
   if (!Hd::FULL && a.D < 16 * Hd::C) {
-    for (bf16_t* t : {Q0, Q1, Q2, Q3, D0, D1, D2, D3}) zero_tails(t, TILE);
+    for (bf16_t* t : {Q0, Q1, Q2, Q3, D0, D1, D2, D3}) zero_tails<8>(t, TILE);
     __syncthreads();
   }
   int bh, kblk;
@@ -2318,34 +2167,32 @@ int wq_grid(int nblk, int BH, hipStream_t st, WorkQ& q) {
   return cus;
 }
 
-// Whether a query-stationary launch over BH (b, h) of length n runs half blocks
-// (fwd_half_block).  Both ways are estimated in units of 10 ns of the forward at
-// D = 128, with measured constants: a step costs 1.57 us (one tile of 256
-// queries) or 2.1 us (two of 128) while most of the chip idles, which bounds a
-// launch by its heaviest block, and 1.9 or 2.12 us when all CUs run, plus 7 us
-// for each block of a CU in turn, which bounds it by its share of the whole
-// work; with more blocks than CUs some CU also takes two of the middle ones.
-// dQ and the narrower heads have other times but nearly the same ratios.  Half
-// blocks are taken when they are estimated 7% shorter.  Over 66 shapes of 1 to
-// 256 heads and 256 to 14000 rows at D = 64, 72 and 128 the choice was within 3%
-// of the better side in 379 of 396 forwards and dQs, and within 15% in all (32
-// heads of 2029 rows, forward at D = 64).  The middle blocks' bound is what
-// keeps 64 heads of 744 rows on whole blocks (D = 64: 23 / 27 against 28 / 31 us).
-// Forward / dQ, whole -> half: 12 heads of 6000 rows 157 / 203 -> 140 / 178 us at
-// D = 128, 115 / 125 -> 95 / 105 at 64; 8 of 10236 at 64 188 / 201 -> 168 / 185.
+// Whether a query-stationary launch over BH (b, h) of length n runs half blocks:
+// workgroups of HW waves, 128 queries, two to a CU where there are more than CUs.
+// A wave's work is the same as in a whole block (32 queries against their keys
+// in order, and dQ's key centre from the whole block's sample), and so are its
+// results, bit for bit: a row does not depend on the batch it comes with.
+//
+// A launch that leaves most of the chip idle is bound by the chain of its
+// heaviest block, a key tile at a time.  With one wave per SIMD a tile takes 1.3
+// us instead of 1.57 (forward, D = 128); a second workgroup on the CU brings
+// that back to about 2.  So half blocks are for launches in which each of them
+// has half a CU to itself, n / 128 blocks of all (b, h) within twice the CUs, the
+// heaviest ones started first, on CUs of their own (WQ_SPREAD; with the plain
+// order 12 heads of 4780 rows, whose second heads' heavy blocks then join the
+// first ones', 120 -> 130 us forward).  Beyond that the doubled K / V copies show.
+// Forward / dQ, whole -> half: 8 heads of 1152 rows 33 / 41 -> 28 / 36 us, of 4608
+// 115 / 143 -> 95 / 118, 12 of 4780 121 / 149 -> 106 / 138, 32 of 2029 60 / 77 ->
+// 53 / 70, 8 of 4608 at D = 64 86 / 90 -> 71 / 81; past the line 8 of 10236 253 /
+// 314 -> 251 / 332, 8 of 18432 639 / 825 -> 705 / 933.  Over 251 shapes of 1 to 256
+// heads and 65 to 18432 rows at D = 64, 72 and 128, the 169 within the line: 0.72 to 1.00
+// of the whole blocks' time (one dQ 1.06: 256 heads of 202 rows, D = 72).  Up to
+// 128 rows a whole block has only these waves at work too, and four more to copy.
+// (Two waves sharing 32 queries, one for the even and one for the odd key tiles,
+// cut the chain further, 8 heads of 4608 to 75 / 93 us, but round P against two
+// maxima: other bits, by the batch.)
 bool half_blocks(int BH, int n) {
-  const int cus = cu_count();
-  if (cus <= 0) return false;
-  auto est = [&](int rows, int tiles_per_step, int chain, int load) {
-    const long long nb = (n + rows - 1) / rows, per = (long long)rows / BN / tiles_per_step;
-    const long long heavy = ((n + BN - 1) / BN + tiles_per_step - 1) / tiles_per_step;
-    const long long steps = per * nb * (nb - 1) / 2 + heavy;
-    long long t = std::max(heavy * chain + 700, BH * (steps * load + nb * 700) / cus);
-    if (nb * BH > cus)  // the (cus)th and (cus + 1)th heaviest share a CU at best
-      t = std::max(t, (2 * nb - (cus - 1) / BH - cus / BH) * per * chain + 1400);
-    return t;
-  };
-  return est(HB, 2, 210, 212) * 107 < est(32 * QW, 1, 157, 190) * 100;
+  return n > 32 * HW && (long long)((n - 1) / (32 * HW) + 1) * BH <= (QW / HW) * cu_count();
 }
 
 // Grid of a query-stationary launch: a packed plan where one applies, else as wq_grid.
@@ -2354,6 +2201,15 @@ int query_grid(int BH, int n, hipStream_t st, QPlan& p, WorkQ& q) {
   q.ctr = nullptr;
   q.slots = 0;
   return p.bph ? grid : wq_grid((n + 32 * QW - 1) / (32 * QW), BH, st, q);
+}
+
+// Grid of a query-stationary launch of half blocks.
+int half_grid(AttnArgs& a, QPlan& p, WorkQ& q) {
+  a.nq = (a.n - 1) / (32 * HW) + 1;
+  p.bph = p.ipb = 0;
+  q.ctr = nullptr;
+  q.slots = WQ_SPREAD;
+  return a.nq * a.BH;
 }
 
 }  // namespace
@@ -2372,12 +2228,11 @@ int attn_fwd_impl(const void* q, const void* k, const void* v, int64_t sb, int64
   QPlan p;
   WorkQ wq;
   if ((flags & LH_ATTN_SHAPED) && half_blocks(a.BH, n)) {
-    a.nq = (n + HB - 1) / HB;
-    const int grid = wq_grid(a.nq, a.BH, st, wq);
-    LH_DISPATCH_HEAD(dtype, D, hipLaunchKernelGGL((attn_fwd_half_kernel<T, Hd>), dim3(grid), dim3(64 * QW), 0, st, a, wq));
+    const int grid = half_grid(a, p, wq);
+    LH_DISPATCH_HEAD(dtype, D, hipLaunchKernelGGL((attn_fwd_kernel<T, Hd, HW, 0>), dim3(grid), dim3(64 * HW), 0, st, a, p, wq));
   } else {
     const int grid = query_grid(a.BH, a.n, st, p, wq);
-    LH_DISPATCH_HEAD(dtype, D, hipLaunchKernelGGL((attn_fwd_kernel<T, Hd, 0>), dim3(grid), dim3(64 * QW), 0, st, a, p, wq));
+    LH_DISPATCH_HEAD(dtype, D, hipLaunchKernelGGL((attn_fwd_kernel<T, Hd, QW, 0>), dim3(grid), dim3(64 * QW), 0, st, a, p, wq));
   }
   LH_CHECK_LAUNCH();
   return LH_OK;
@@ -2417,13 +2272,11 @@ int attn_bwd_parts(int parts, const void* q, const void* k, const void* v, int64
     QPlan p;
     WorkQ wq;
     if ((flags & LH_ATTN_SHAPED) && half_blocks(a.BH, n)) {
-      a.nq = (n + HB - 1) / HB;
-      const int grid = wq_grid(a.nq, a.BH, st, wq);
-      LH_DISPATCH_HEAD(dtype, D,
-                       hipLaunchKernelGGL((attn_bwd_dq_half_kernel<T, Hd>), dim3(grid), dim3(64 * QW), 0, st, a, wq));
+      const int grid = half_grid(a, p, wq);
+      LH_DISPATCH_HEAD(dtype, D, hipLaunchKernelGGL((attn_bwd_dq_kernel<T, Hd, HW>), dim3(grid), dim3(64 * HW), 0, st, a, p, wq));
     } else {
       const int grid = query_grid(a.BH, a.n, st, p, wq);
-      LH_DISPATCH_HEAD(dtype, D, hipLaunchKernelGGL((attn_bwd_dq_kernel<T, Hd>), dim3(grid), dim3(64 * QW), 0, st, a, p, wq));
+      LH_DISPATCH_HEAD(dtype, D, hipLaunchKernelGGL((attn_bwd_dq_kernel<T, Hd, QW>), dim3(grid), dim3(64 * QW), 0, st, a, p, wq));
     }
     LH_CHECK_LAUNCH();
   }
@@ -2563,7 +2416,7 @@ extern "C" int lh_dilated_scores_nd(const void* xq, const void* xk, const void* 
   if (!twice) a.BH *= 2;
   for (a.bh0 = 0; a.bh0 < 2 * a.B * a.H; a.bh0 += a.BH) {
     const int grid = query_grid(a.BH, a.n, st, p, wq);
-    LH_DISPATCH_HEAD(dtype, D, hipLaunchKernelGGL((attn_fwd_kernel<T, Hd, 1>), dim3(grid), dim3(64 * QW), 0, st, a, p,
+    LH_DISPATCH_HEAD(dtype, D, hipLaunchKernelGGL((attn_fwd_kernel<T, Hd, QW, 1>), dim3(grid), dim3(64 * QW), 0, st, a, p,
                                                   wq));
     LH_CHECK_LAUNCH();
   }

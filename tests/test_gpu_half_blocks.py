@@ -1,7 +1,8 @@
-"""Half blocks of the query-stationary attention kernels (128 queries per
-workgroup, the key tiles shared by its two halves; lh_attn.hip, fwd_half_block):
-forward, dQ and the unchanged dK/dV against fp32 attention, at sizes around the
-64-row tiles and the 128-row blocks, for few and for many heads."""
+"""Half blocks of the query-stationary attention kernels (128 queries to a
+workgroup of four waves; lh_attn.hip, half_blocks): forward, dQ and the unchanged
+dK/dV against fp32 attention, at sizes around the 64-row tiles and the 128-row
+blocks, for few and for many heads; and bit for bit against whole blocks, so that
+a sequence has the same results alone and in a batch."""
 import pytest
 import torch
 
@@ -19,13 +20,13 @@ def _inputs(n, H, dtype, dev, gathered):
     return [x.to(dev) for x in xs], idx.to(dev) if gathered else None, do.to(dev)
 
 
-# 65: two tiles, one per half; 127, 128, 129: one block and its edge; 193: a third
-# tile, so one half runs a step more; 1000, 4608: the layer's short lengths
+# 65: two tiles; 127, 128, 129: one block and its edge; 193: a block and a half;
+# 1000, 4608: the layer's short lengths
 @pytest.mark.parametrize("n,H,dtype,gathered", [
     (65, 2, torch.bfloat16, True), (127, 1, torch.bfloat16, False), (128, 2, torch.float16, True),
     (129, 2, torch.bfloat16, True), (193, 3, torch.float16, False), (1000, 2, torch.bfloat16, True),
     (4608, 8, torch.bfloat16, True), (4780, 12, torch.float16, False),
-    # either side of the rule's bound by shared CUs: 64 heads take whole blocks, 12 of 6000 half blocks
+    # either side of the rule's line of two blocks per CU (256): 384 and 564 half blocks
     (744, 64, torch.bfloat16, False), (6000, 12, torch.float16, True)])
 def test_half_blocks(pkg, dev, n, H, dtype, gathered):
     N = pkg._native
@@ -61,3 +62,93 @@ def test_half_blocks_no_finite_score(pkg, dev):
     o1, lse1 = N.attn_fwd(rows, None, 1, H, n)
     assert torch.equal(lse[:, :, :3], lse1[:, :, :3]) and bool((lse[:, :, :3] == -float("inf")).all())
     assert torch.equal(o[:, :, :3], o1[:, :, :3]) and not bool(o[:, :, :3].any())
+
+
+def _calls(pkg, xs, idx, do, n, H, D, shaped):
+    N = pkg._native
+    st = xs[0].stride()[:3]
+    rows = N.Rows(*xs, st, *xs, st, split=n) if idx is not None else N.Rows(*xs, st)
+    o, lse = N.attn_fwd(rows, idx, xs[0].shape[0], H, n, D, shaped=shaped)
+    delta = (do.float() * o.float()).sum(-1)
+    return (o, lse) + tuple(N.attn_bwd(rows, idx, xs[0].shape[0], H, n, do, lse, delta, D, shaped=shaped))
+
+
+# 129 to 300: two and three half blocks, the last one nearly empty or full, beside one
+# and two whole blocks; 1500 and 4780: more half blocks than CUs; 8192: exactly two to
+# a CU (256); D: both narrow layouts, with zero tails (40, 72) and without
+@pytest.mark.parametrize("n,H,D,dtype,gathered", [
+    (129, 3, 128, torch.bfloat16, True), (200, 2, 64, torch.float16, True), (256, 2, 40, torch.bfloat16, False),
+    (257, 3, 72, torch.bfloat16, True), (300, 2, 128, torch.float16, False), (1500, 36, 72, torch.bfloat16, True),
+    (4780, 12, 128, torch.float16, True), (4608, 8, 40, torch.bfloat16, True), (8192, 8, 64, torch.bfloat16, False)])
+@pytest.mark.parametrize("centred", [False, True])
+def test_half_blocks_have_whole_blocks_bits(pkg, dev, n, H, D, dtype, gathered, centred):
+    """centred: keys that share a large channel, so that dQ subtracts the key centre."""
+    print(f"half blocks' bits n={n} H={H} D={D} {dtype} gathered={gathered} centred={centred}", flush=True)
+    g = torch.Generator().manual_seed(n + H + D)
+    xs = [torch.randn(1, n, H, D, generator=g).to(dtype).to(dev) for _ in range(3)]
+    if centred:
+        xs[1][..., 3] = 8.0
+    idx = torch.stack([torch.randperm(n, generator=g) for _ in range(H)])[None].int().to(dev) if gathered else None
+    do = torch.randn(1, H, n, D, generator=g).to(dtype).to(dev)
+    for name, a, b in zip(("o", "lse", "dq", "dk", "dv"), _calls(pkg, xs, idx, do, n, H, D, True),
+                          _calls(pkg, xs, idx, do, n, H, D, False)):
+        assert torch.equal(a, b), name
+
+
+def _kernel_names(f):
+    from torch.profiler import ProfilerActivity, profile
+    f()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        f()
+        torch.cuda.synchronize()
+    return [e.name for e in prof.events()]
+
+
+def test_which_launches_take_half_blocks(pkg, dev):
+    """Waves of a workgroup by the kernels' names: four up to two half blocks per CU,
+    eight beyond, for one block of 128 rows, and in calls without the flag."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    rows = 2 * cus // 8 * 128  # 8 heads: two half blocks to a CU
+    for n, shaped, waves in ((129, True, 4), (rows, True, 4), (128, True, 8), (rows + 1, True, 8), (129, False, 8)):
+        xs, _, do = _inputs(n, 8, torch.bfloat16, dev, False)
+        names = _kernel_names(lambda: _calls(pkg, xs, None, do, n, 8, 128, shaped))
+        for kernel, args in (("attn_fwd_kernel", f", {waves}, 0>"), ("attn_bwd_dq_kernel", f", {waves}>")):
+            got = [x for x in names if kernel in x]
+            assert got and all(args in x for x in got), f"n={n} shaped={shaped}: {got}"
+
+
+@pytest.mark.parametrize("D", [128, 64])
+def test_public_calls_do_not_depend_on_the_batch(pkg, dev, D):
+    """A sequence's results and gradients alone (half blocks) and as one of four (whole blocks)."""
+    B, H, S, k = 4, 8, 8192, 512
+    print(f"batch independence D={D}", flush=True)
+    g = torch.Generator().manual_seed(D)
+    xs = [torch.randn(B, S, H, D, generator=g).bfloat16().to(dev) for _ in range(3)]
+    dout = torch.randn(B, H, S, D, generator=g).bfloat16().to(dev)
+
+    def run(f, ins, up):
+        ins = [x.detach().requires_grad_() for x in ins]
+        out = f(*ins)
+        return (out,) + torch.autograd.grad(out, ins, up)
+
+    def layer(*x):
+        return pkg.lighthouse_layer(*x, 3, 4, k)[0]
+
+    def dense(*x):
+        return pkg.dense_attention.dense_causal_attention(*(t[:, :4608].transpose(1, 2) for t in x))
+
+    freqs = torch.randn(S, 64, 2, generator=g).to(dev)
+
+    def rope(x):
+        return pkg.lighthouse_layer_rope(x, freqs, H, 3, 4, k)[0]
+
+    calls = [(layer, xs, dout), (dense, xs, dout[:, :, :4608])]
+    if D == 128:
+        calls.append((rope, [torch.cat([x.flatten(2) for x in xs], -1)], dout))
+    for f, ins, up in calls:
+        batch = run(f, ins, up)
+        for b in (0, B - 1):
+            alone = run(f, [x[b:b + 1] for x in ins], up[b:b + 1])
+            for i, (x, y) in enumerate(zip(alone, batch)):
+                assert torch.equal(x[0], y[b]), f"{f.__name__}: result {i} of sequence {b}"
