@@ -13,7 +13,7 @@ import ctypes
 import os
 import subprocess
 import threading
-from functools import lru_cache
+from functools import lru_cache, wraps
 
 import torch
 
@@ -248,7 +248,18 @@ def check_indices(indices, lo: int, hi: int, unique: bool = True, what: str = "i
         raise IndexError(f"{what}: {dup} duplicate entries (indices must be unique per (batch, head))")
 
 
-@lru_cache(maxsize=256)
+def _cached_sizes(f):
+    """``f`` cached where its arguments are plain ints; sizes are symbolic, and cannot be
+    hashed, where ``torch.compile`` traces a second sequence length."""
+    cached = lru_cache(maxsize=256)(f)
+
+    @wraps(f)
+    def sizes(*args, **kw):
+        return cached(*args) if not kw and all(type(x) in (int, bool) for x in args) else f(*args, **kw)
+    return sizes
+
+
+@_cached_sizes
 def geometry(S: int, L: int, p: int, topk: int, strict: bool = True):
     """``(num_tiles, nodes_per_tile, per_tile, S_sel)``; raises like the reference outside
     its domain when ``strict``."""
@@ -263,7 +274,7 @@ def geometry(S: int, L: int, p: int, topk: int, strict: bool = True):
     return tuple(o.value for o in out)
 
 
-@lru_cache(maxsize=256)
+@_cached_sizes
 def pyramid_total(S: int, L: int, p: int) -> int:
     return pyramid_lengths(S, L, p)[2]
 

@@ -58,6 +58,29 @@ def test_layer_compiled_fullgraph_bit_equal(pkg, dev, seq_major):
         assert torch.equal(a, b)
 
 
+def test_layer_compiled_at_two_lengths(pkg, dev):
+    """A second sequence length makes dynamo trace the layer with a symbolic one."""
+    L, p, k, H, D = 3, 4, 128, 2, 64
+    torch._dynamo.reset()
+
+    def f(q, k_, v):
+        return pkg.lighthouse_layer(q, k_, v, L, p, k, strict=False)[0] * 1.0
+
+    cf = torch.compile(f, fullgraph=True, backend="aot_eager")
+    for S in (2048, 4096, 3000):
+        g = torch.Generator(device=dev).manual_seed(S)
+        base = [torch.randn(1, S, H, D, device=dev, generator=g).bfloat16() for _ in range(3)]
+        dout = torch.randn(1, H, S, D, device=dev, generator=g).bfloat16()
+        res = []
+        for fn in (f, cf):
+            xs = [b.clone().requires_grad_() for b in base]
+            out = fn(*xs)
+            res.append((out,) + torch.autograd.grad(out, xs, dout))
+        for a, b in zip(*res):
+            assert torch.equal(a, b), S
+    torch._dynamo.reset()
+
+
 @pytest.mark.parametrize("backend", ["inductor", "aot_eager"])
 def test_block_compiled_like_the_reference(pkg, dev, backend):
     """One Lighthouse TransformerBlock of the 270M flavor (dim 1024, 8 heads of 128,
