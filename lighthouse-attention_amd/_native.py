@@ -649,7 +649,10 @@ def scatter_fwd(attn, inverse, S: int, S_out: int, L: int, p: int, seq_major: bo
 
 def scatter_bwd(dout, indices, o, S: int, L: int, p: int):
     """``(dattn [B, H, n, D] of dout's dtype, delta fp32 [B, H, n] or None)``; ``dout``
-    may have any (batch, head, seq) strides with D contiguous."""
+    may have any (batch, head, seq) strides with D contiguous; below 128 columns any
+    strides (what the kernel cannot read in place, such as an expanded row, is copied)."""
+    if dout.shape[-1] < D_SUPPORTED and (dout.stride(-1) != 1 or dout.stride(2) <= 0):
+        dout = dout.contiguous()
     dt = _need_rows("scatter_bwd", dout, o)
     _need_dtype("scatter_bwd indices", torch.int32, indices)
     _need_gpu(dout, indices, o)

@@ -115,6 +115,32 @@ def test_narrow_inputs_that_are_copied(pkg, dev):
         assert torch.equal(x, y)
 
 
+@pytest.mark.parametrize("D", [64, 72, 104])
+def test_narrow_upstream_gradients_of_any_strides(pkg, dev, D):
+    """Expanded gradients (a sum's, over all or over the sequence) and a strided head dim
+    give the layer, dense attention and the fan-out what a contiguous copy gives them."""
+    S, H, n = 2048, 2, 300
+    g = torch.Generator().manual_seed(D)
+    xs = [torch.randn(1, S, H, D, generator=g).bfloat16().to(dev) for _ in range(3)]
+    att = torch.randn(1, H, n, D, generator=g).bfloat16().to(dev)
+    idx = torch.stack([torch.randperm(S + S // 4, generator=g)[:n] for _ in range(H)])[None].int().to(dev)
+    calls = [(lambda *x: pkg.lighthouse_layer(*x, 3, 4, 128)[0], xs),
+             (lambda *x: pkg.dense_attention.dense_causal_attention(*(t.transpose(1, 2) for t in x)), xs),
+             (lambda a: pkg.scatter_to_base_sequence(a, idx, None, S, S, 2, 4), [att])]
+    one = torch.randn(1, H, 1, D, generator=g).bfloat16().to(dev)
+    ups = [torch.ones(1, dtype=torch.bfloat16, device=dev).expand(1, H, S, D), one.expand(1, H, S, D),
+           one[:, :1].expand(1, H, S, D), torch.randn(1, H, D, S, generator=g).bfloat16().to(dev).transpose(2, 3)]
+    for c, (f, ins) in enumerate(calls):
+        for u, up in enumerate(ups):
+            print(f"upstream D={D} call {c} form {u}", flush=True)
+            res = []
+            for d in (up, up.contiguous()):
+                leaves = [x.clone().requires_grad_() for x in ins]
+                res.append(torch.autograd.grad(f(*leaves), leaves, d))
+            for a, b in zip(*res):
+                assert torch.equal(a, b), f"call {c}, form {u}"
+
+
 def test_fan_out_any_width(pkg, dev):
     """scatter_to_base_sequence takes row widths that are no multiple of 8."""
     S, H, L, p = 512, 2, 2, 2
