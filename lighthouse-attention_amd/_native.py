@@ -31,9 +31,18 @@ def padded_dim(D: int) -> int:
 
 def own_rows(x):
     """``x`` contiguous and, for head dims below 128, on a 16-byte boundary (copied if
-    it is not; 128-wide rows off the boundary are refused by the library)."""
+    it is not; 128-wide rows off the boundary are refused by the library) and with the
+    strides of its shape also where a dimension has one element, which ``contiguous``
+    leaves as they are: q, k, v of one shape then share them."""
     x = x.contiguous()
-    return x.clone() if x.shape[-1] < D_SUPPORTED and x.data_ptr() % 16 else x
+    if x.shape[-1] == D_SUPPORTED:
+        return x
+    if x.data_ptr() % 16:
+        x = x.clone()
+    strides = [1]
+    for size in x.shape[:0:-1]:
+        strides.insert(0, strides[0] * size)
+    return x if x.stride() == tuple(strides) else x.as_strided(x.shape, strides)
 
 
 def shared_rows(q, k, v):

@@ -116,6 +116,45 @@ def test_narrow_inputs_that_are_copied(pkg, dev):
 
 
 @pytest.mark.parametrize("D", [64, 72, 104])
+def test_narrow_inputs_whose_single_dims_have_strides_of_their_own(pkg, dev, D):
+    """One sequence or one head cut out of a larger tensor keeps that tensor's stride in
+    the dimension of one element: q, k, v then differ in strides that nobody reads."""
+    S = 2048
+    g = torch.Generator().manual_seed(D)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g).bfloat16().to(dev)
+
+    forms = {  # [B, S, H, D] each
+        "k, v a prefix of longer ones": [rnd(1, S, 2, D), rnd(1, S + 64, 2, D)[:, :S], rnd(1, S + 64, 2, D)[:, :S]],
+        "v out of a fused buffer": [rnd(1, S, 2, D), rnd(1, S, 2, D), rnd(1, 3, S, 2, D)[:, 2]],
+        "one head, q head-major": [rnd(1, 1, S, D).transpose(1, 2), rnd(1, S, 1, D), rnd(1, S, 1, D)],
+        "one head of a prefix": [rnd(1, S, 1, D), rnd(1, S + 64, 1, D)[:, :S], rnd(1, S + 64, 1, D)[:, :S]],
+        "off a 16-byte boundary": [rnd(1, S, 2, D), rnd(1, 3 * S * 2 * D + 1)[:, 1:].view(1, 3, S, 2, D)[:, 1], rnd(1, S, 2, D)],
+    }
+    gk = torch.nn.functional.logsigmoid(rnd(1, S, 2))
+
+    def sums(out):
+        return sum(x.float().sum() for x in out[2:])
+
+    calls = {"layer": lambda *x: pkg.lighthouse_layer(*x, 3, 4, 128)[0],
+             "dilated layer": lambda *x: pkg.lighthouse_layer(*x, 3, 4, 128, dilation=4)[0],
+             "gla layer": lambda *x: pkg.lighthouse_layer(*x, 3, 4, 128, dilation=4, gk=gk[..., :x[0].shape[2]])[0],
+             "scorer": lambda *x: sums(pkg.DialatedLighthouseNormScorer(4, 3)(*x)),
+             "dense": lambda *x: pkg.dense_attention.dense_causal_attention(*(t.transpose(1, 2) for t in x))}
+    for form, xs in forms.items():
+        for name, f in calls.items():
+            print(f"D={D} {form}: {name}", flush=True)
+            res = []
+            for ins in (xs, [x.clone(memory_format=torch.contiguous_format) for x in xs]):
+                leaves = [x.detach().requires_grad_() for x in ins]
+                out = f(*leaves)
+                res.append((out,) + torch.autograd.grad(out, leaves, torch.ones_like(out)))
+            for a, b in zip(*res):
+                assert torch.equal(a, b), f"{form}: {name}"
+
+
+@pytest.mark.parametrize("D", [64, 72, 104])
 def test_narrow_upstream_gradients_of_any_strides(pkg, dev, D):
     """Expanded gradients (a sum's, over all or over the sequence) and a strided head dim
     give the layer, dense attention and the fan-out what a contiguous copy gives them."""
