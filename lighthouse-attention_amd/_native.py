@@ -24,9 +24,9 @@ D_SUPPORTED = 128
 
 
 def padded_dim(D: int) -> int:
-    """Width a head dim D (a multiple of 8, at most 128) runs at: its own up to 96, else
-    128 with zero columns (no attention layout between the two)."""
-    return D if D <= 96 else D_SUPPORTED
+    """Width a head dim D (at most 128) runs at, with zero columns where that is wider:
+    the next multiple of 8 up to 96, else 128 (no attention layout between the two)."""
+    return -(-D // 8) * 8 if D <= 96 else D_SUPPORTED
 
 
 def own_rows(x):

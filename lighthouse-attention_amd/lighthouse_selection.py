@@ -503,7 +503,8 @@ _compiled_ops = _CompiledOps()
 class _PyramidCatFn(torch.autograd.Function):
     """The reference scorer's 5-tuple from the native pyramid; backward through the
     dense pyramid adjoint (``g[pyramid row]`` gathered onto base rows).  Head dims
-    from 104 to 120 run zero-padded (the padded columns of the returned rows are cut off)."""
+    that are no multiple of 8, or between 96 and 128, run zero-padded (the padded
+    columns of the returned rows are cut off)."""
 
     @staticmethod
     def forward(ctx, xq, xk, xv, L, p, dilation, base_qk=None, base_kq=None, full=False):

@@ -180,6 +180,52 @@ def test_narrow_upstream_gradients_of_any_strides(pkg, dev, D):
                 assert torch.equal(a, b), f"call {c}, form {u}"
 
 
+@pytest.mark.parametrize("D", [4, 20, 36, 97, 100, 127])
+def test_scorer_modules_any_width(pkg, dev, D):
+    """The scorer modules and the layer composed from one take head dims that are no
+    multiple of 8: the same rows as with columns of zeros, scores and attention with the
+    scale of the D columns."""
+    B, S, H, L, p, k = 1, 2048, 2, 3, 4, 128
+    print(f"scorers D={D}", flush=True)
+    g = torch.Generator().manual_seed(D)
+    xs = [torch.randn(B, S, H, D, generator=g).bfloat16().to(dev) for _ in range(3)]
+    gk = torch.nn.functional.logsigmoid(torch.randn(B, S, H, generator=g).to(dev)) / 16
+
+    class Scorer(pkg.DialatedLighthouseNormScorer):  # not the class itself: the composed path
+        pass
+
+    def reference(dil, gate=None):
+        """Scores by the 128-wide kernels on padded rows."""
+        wide = [torch.nn.functional.pad(x, (0, 128 - D)) for x in xs]
+        S_tot = pkg._native.pyramid_total(S, L, p)
+        if gate is not None:
+            base = pkg._native.gla_scores(*wide, gate, dil, S_tot, D ** -0.5)
+        else:
+            base = pkg._native.dilated_scores(*wide, dil, S_tot, D ** -0.5) if dil else None
+        return pkg._native.pyramid_fwd(*wide, L, p, scores=base)
+
+    for name, out, (pq, pk, pv, sqk, skq) in (
+            ("norm", Scorer(p, L)(*xs), reference(0)),
+            ("dilated", pkg.DilatedLighthouseScorer(None, 4, p, L)(*xs), reference(4)),
+            ("gla", pkg.DilatedLighthouseGLAScorer(D, 4, p, L)(*xs, gk), reference(4, gk))):
+        for got, want in zip(out[:2], (sqk, skq)):
+            assert_close(got, want, f"{name} scores", max_abs=4e-3, rel_l2=4e-3)  # bf16 scores
+        for got, x, pool in zip(out[2:], xs, (pq, pk, pv)):
+            assert torch.equal(got[:, :, :S], x.transpose(1, 2)) and torch.equal(got[:, :, S:],
+                                                                                 pool[..., :D].transpose(1, 2)), name
+    layer = pkg.LighthouseLocal(None, Scorer(p, L), L, p, k)
+    leaves = [x.clone().requires_grad_() for x in xs]
+    out = layer(*leaves)
+    do = torch.randn(B, H, S, D, generator=g).bfloat16().to(dev)
+    out.backward(do)
+    xc = [x.float().cpu().requires_grad_() for x in xs]
+    ref, _ = O.lighthouse_layer(*xc, L, p, k, indices=layer.last_indices.cpu().numpy())
+    ref.backward(do.float().cpu())
+    assert_close(out, ref, f"D={D} out")
+    for name, x, c in zip("qkv", leaves, xc):
+        assert_close(x.grad, c.grad, f"D={D} d{name}")
+
+
 def test_fan_out_any_width(pkg, dev):
     """scatter_to_base_sequence takes row widths that are no multiple of 8."""
     S, H, L, p = 512, 2, 2, 2
