@@ -121,10 +121,11 @@ def _mark(name):
 
 
 def _gla_rows(*xs):
-    """Rows as the GLA scorer takes them: contiguous, zero-padded to 128 columns (zero
-    columns change no product, so the scores are the D-wide rows')."""
+    """Rows as the GLA scorer takes them: contiguous (``pad`` keeps the order that it finds
+    its input in), zero-padded to 128 columns (zero columns change no product, so the
+    scores are the D-wide rows')."""
     pad = N.D_SUPPORTED - xs[0].shape[-1]
-    return tuple(torch.nn.functional.pad(x, (0, pad)) if pad else x.contiguous() for x in xs)
+    return tuple((torch.nn.functional.pad(x, (0, pad)) if pad > 0 else x).contiguous() for x in xs)
 
 
 def _layer_fwd(xq, xk, xv, L, p, topk, tie, strict, dilation, seq_major, gk=None, scale=None):

@@ -180,6 +180,27 @@ def test_narrow_upstream_gradients_of_any_strides(pkg, dev, D):
                 assert torch.equal(a, b), f"call {c}, form {u}"
 
 
+@pytest.mark.parametrize("D", [64, 104, 128])
+def test_scorers_take_any_order(pkg, dev, D):
+    """Rows stored with the sequence or the heads running fastest give the scorer modules
+    what contiguous rows give them."""
+    B, S, H = 2, 2048, 2
+    g = torch.Generator().manual_seed(D)
+    xs = [torch.randn(B, S, H, D, generator=g).bfloat16().to(dev) for _ in range(3)]
+    gk = torch.nn.functional.logsigmoid(torch.randn(B, S, H, generator=g).to(dev)) / 16
+    orders = {"sequence fastest": lambda x: x.permute(0, 2, 3, 1).contiguous().permute(0, 3, 1, 2),
+              "channels last": lambda x: x.contiguous(memory_format=torch.channels_last),
+              "heads fastest": lambda x: x.transpose(2, 3).contiguous().transpose(2, 3)}
+    scorers = {"gla": lambda *x: pkg.DilatedLighthouseGLAScorer(D, 4, 4, 3)(*x, gk),
+               "dilated": pkg.DilatedLighthouseScorer(None, 4, 4, 3), "norm": pkg.DialatedLighthouseNormScorer(4, 3)}
+    for name, f in scorers.items():
+        want = f(*xs)
+        for order, store in orders.items():
+            print(f"D={D} {name} {order}", flush=True)
+            for i, (a, b) in enumerate(zip(f(*[store(x) for x in xs]), want)):
+                assert torch.equal(a, b), f"{name}, {order}: output {i}"
+
+
 @pytest.mark.parametrize("D", [4, 20, 36, 97, 100, 127])
 def test_scorer_modules_any_width(pkg, dev, D):
     """The scorer modules and the layer composed from one take head dims that are no
