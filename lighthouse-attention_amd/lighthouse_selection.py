@@ -525,11 +525,10 @@ class _PyramidCatFn(torch.autograd.Function):
             scores[1][..., :S].copy_(base_kq)
         sqk, skq, *cats = N.pyramid_cat(xq, xk, xv, L, p, scores)
         ctx.geo = (B, S, H, D, L, p, D0)
-        ctx.mark_non_differentiable(sqk, skq)
         return (sqk, skq, *(c[..., :D0].transpose(1, 2) for c in cats))
 
     @staticmethod
-    def backward(ctx, _g1, _g2, gq, gk, gv):
+    def backward(ctx, _g1, _g2, gq, gk, gv):  # the scores only feed the selection: they pass no gradient on
         B, S, H, D, L, p, D0 = ctx.geo
         gs = [g if g is not None else None for g in (gq, gk, gv)]
         ref = next((g for g in gs if g is not None), None)

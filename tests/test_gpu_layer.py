@@ -119,3 +119,18 @@ def test_layer_backward_two_streams(pkg, dev):
             pkg.lighthouse_selection.set_backward_streams(prev)
     for n, g1, g2 in zip("qkv", *grads):
         assert torch.equal(g1, g2), f"d{n} differs between one and two backward streams"
+
+
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("dilation", [0, 4])
+def test_scores_of_a_scorer_carry_no_gradient_on(pkg, dev, D, dilation):
+    """The scores of inputs that are trained require a gradient themselves, and a
+    backward from them alone is zero."""
+    g = torch.Generator().manual_seed(D)
+    xs = [torch.randn(1, 2048, 2, D, generator=g).bfloat16().to(dev).requires_grad_() for _ in range(3)]
+    scorer = pkg.DilatedLighthouseScorer(None, dilation, 4, 3) if dilation else pkg.DialatedLighthouseNormScorer(4, 3)
+    out = scorer(*xs)
+    assert all(x.requires_grad for x in out)
+    (out[0].float().sum() + out[1].float().sum()).backward()
+    for x in xs:
+        assert x.grad is not None and not bool(x.grad.any())
