@@ -2408,11 +2408,17 @@ extern "C" int lh_dilated_scores_nd(const void* xq, const void* xk, const void* 
   // Both directions in one launch, the second one's blocks filling the end of
   // the first one's: 8 heads, dilation 4, 8192 tokens 119 -> 79 us, 24000 tokens
   // 585 -> 564, 131072 tokens 15870 -> 15610; 2 x 4 heads, 6000 tokens 84 -> 47.
-  // Where a plan packs one direction's blocks two to a bin, twice that plan is
-  // the better schedule (16384 tokens: 266 us against 270 in one launch).
+  // Except where a plan packs one direction's blocks two to a bin, nearly fills
+  // the bins, and the joint launch with half as many bins per (b, h) is past the
+  // plans' limit (from 1.75 blocks per bin).  Two launches / one, D = 128 and 64,
+  // by the blocks per bin of one direction: 1.03 400 / 258 us, 304 / 174 (8 virtual
+  // heads of 8448 rows); 1.5 307 / 281, 226 / 189 (16 of 6144); 1.75 201 / 204, 138 /
+  // 137 (32 of 3584); 2 262 / 266, 173 / 187 (32 of 4096), 91 / 105, 65 / 81 (128 of
+  // 1024).  Over 8 to 128 virtual heads one launch takes 0.57 to 0.97 of the time of two
+  // below 1.75 and 0.93 to 1.25 from there on.
   QPlan p;
   WorkQ wq;
-  const bool twice = make_plan(a.BH, n, p) && p.bph && a.nq <= 2 * p.bph;
+  const bool twice = make_plan(a.BH, n, p) && p.bph && 4 * a.nq >= 7 * p.bph && a.nq <= 2 * p.bph;
   if (!twice) a.BH *= 2;
   for (a.bh0 = 0; a.bh0 < 2 * a.B * a.H; a.bh0 += a.BH) {
     const int grid = query_grid(a.BH, a.n, st, p, wq);

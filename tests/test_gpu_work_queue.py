@@ -104,6 +104,21 @@ def test_queue_dilated_scores_bit_equal(pkg, dev):
         assert torch.equal(skq[:, h:h + 1, :S], rk[..., :S]), f"head {h}: kq scores differ"
 
 
+@pytest.mark.parametrize("S,H,D", [(12288, 8, 128), (14336, 8, 64), (14332, 4, 128), (26000, 4, 72)])
+def test_dilated_scores_one_launch_or_two(pkg, dev, S, H, D):
+    """Either side of the line between one launch for both directions and one for each:
+    1.5 and 1.75 blocks per plan bin, fewer, and 1.625 in a ragged length; equal to single heads' scores."""
+    dil = 4
+    print(f"dilated S={S} H={H} D={D}", flush=True)
+    N = pkg._native
+    xs = [_rand((1, S, H, D), 60 + i, dev) for i in range(3)]
+    got = N.dilated_scores(*xs, dil, S)
+    for h in (0, H - 1):
+        alone = N.dilated_scores(*[x[:, :, h:h + 1].contiguous() for x in xs], dil, S)
+        for name, a, b in zip(("qk", "kq"), got, alone):
+            assert torch.equal(a[:, h:h + 1], b), f"head {h}: {name} scores differ"
+
+
 def test_queue_two_streams(pkg, dev):
     """The same launches on the default stream and a second stream (separate counter slots), three times each."""
     n, B, H = 20000, 1, 8
