@@ -297,13 +297,12 @@ def pyramid_lengths(S: int, L: int, p: int):
 # ---------------------------------------------------------------------------
 # op wrappers (tensor in, tensor out; all on the current stream)
 # ---------------------------------------------------------------------------
-def pyramid_fwd(xq, xk, xv, L: int, p: int, scores=None, pooled_out=None):
+def pyramid_fwd(xq, xk, xv, L: int, p: int, scores=None):
     """Norm scores + pooled Q/K/V.  ``xq/xk/xv`` bf16 or fp16 [B, S, H, D] with D contiguous.
 
     Returns ``(pq, pk, pv, scores_qk, scores_kq)`` with pooled rows of the input
     dtype [B, Sp, H, D] and scores fp32 [B, H, S_tot].  If ``scores`` is given
     (dilated scorer), its base level is kept and only pooled.
-    ``pooled_out`` may supply three pooled destinations (any strides, D contiguous).
     """
     _need_gpu(xq, xk, xv)
     dt = _need_rows("pyramid_fwd", xq, xk, xv)
@@ -313,11 +312,7 @@ def pyramid_fwd(xq, xk, xv, L: int, p: int, scores=None, pooled_out=None):
     S_tot = pyramid_total(S, L, p)
     Sp = S_tot - S
     dev = xq.device
-    if pooled_out is None:
-        pq, pk, pv = (torch.empty(B, Sp, H, D, dtype=xq.dtype, device=dev) for _ in range(3))
-    else:
-        pq, pk, pv = pooled_out
-        _need_rows("pyramid_fwd pooled_out", xq, pq, pk, pv)
+    pq, pk, pv = (torch.empty(B, Sp, H, D, dtype=xq.dtype, device=dev) for _ in range(3))
     if scores is None:
         sqk = torch.empty(B, H, S_tot, dtype=torch.float32, device=dev)
         skq = torch.empty_like(sqk)

@@ -1986,19 +1986,6 @@ int fill_rows(AttnArgs& a, const void* q, const void* k, const void* v, int64_t 
   return LH_OK;
 }
 
-// CUs of the current device (cached per device); 0 when unknown.
-int cu_count() {
-  static std::atomic<int> cache[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  int c = cache[dev].load(std::memory_order_relaxed);
-  if (c == 0) {
-    if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c <= 0) c = -1;
-    cache[dev].store(c, std::memory_order_relaxed);
-  }
-  return c > 0 ? c : 0;
-}
-
 // Best-fit-decreasing packing of costs w into at most nb bins of capacity cap:
 // each block, heaviest first, goes to the fullest bin it still fits in.
 bool pack_bfd(const std::vector<int>& w, const std::vector<int>& order, int nb, long long cap,
@@ -2036,7 +2023,7 @@ int make_plan(int BH, int n, QPlan& p) {
   const int nb = (n + 32 * QW - 1) / (32 * QW);
   const int plain = nb * BH;
   if (g_schedule.load(std::memory_order_relaxed) & LH_SCHED_NO_PLAN) return plain;
-  const int cus = cu_count();
+  const int cus = lh_cu_count();
   if (cus <= 0 || cus % 8 || BH % 8 || BH > cus || (cus / 8) % (BH / 8)) return plain;
   const int bph = cus / BH;
   if (nb <= bph || 2 * nb > 7 * bph || nb >= (int)PLAN_NONE) return plain;
@@ -2157,7 +2144,7 @@ int wq_grid(int nblk, int BH, hipStream_t st, WorkQ& q) {
   q.ctr = nullptr;
   q.slots = 0;
   const long long total = (long long)nblk * BH;
-  const int cus = cu_count();
+  const int cus = lh_cu_count();
   if (cus <= 0 || cus % 8 || total <= cus || total > 12LL * cus) return (int)total;
   if (g_schedule.load(std::memory_order_relaxed) & LH_SCHED_NO_QUEUE) return (int)total;
   unsigned* c = wq_counters(st);
@@ -2192,7 +2179,7 @@ int wq_grid(int nblk, int BH, hipStream_t st, WorkQ& q) {
 // cut the chain further, 8 heads of 4608 to 75 / 93 us, but round P against two
 // maxima: other bits, by the batch.)
 bool half_blocks(int BH, int n) {
-  return n > 32 * HW && (long long)((n - 1) / (32 * HW) + 1) * BH <= (QW / HW) * cu_count();
+  return n > 32 * HW && (long long)((n - 1) / (32 * HW) + 1) * BH <= (QW / HW) * lh_cu_count();
 }
 
 // Grid of a query-stationary launch: a packed plan where one applies, else as wq_grid.

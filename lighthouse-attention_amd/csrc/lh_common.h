@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "../../include/lighthouse_hip.h"
 
 #define LH_D 128  // widest head dimension; D below it: see Lanes
@@ -112,6 +114,19 @@ struct Lanes {
     }                                  \
   } while (0)
 static inline bool lanes_supported(int D) { return D > 0 && D <= LH_D && D % 8 == 0; }
+
+// CUs of the current device (cached per device); 0 when unknown.
+static inline int lh_cu_count() {
+  static std::atomic<int> cache[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  int c = cache[dev].load(std::memory_order_relaxed);
+  if (c == 0) {
+    if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c <= 0) c = -1;
+    cache[dev].store(c, std::memory_order_relaxed);
+  }
+  return c > 0 ? c : 0;
+}
 
 // Launch helper: F(tag) for the element type named by a dtype code.
 #define LH_DISPATCH_DTYPE(dtype, ...)                         \

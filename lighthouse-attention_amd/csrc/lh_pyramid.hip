@@ -45,7 +45,7 @@ constexpr int PYR_CHUNK = 4;  // base tokens whose loads are issued together
 // (every lane of the row's group gets them), or the given ones (GIVEN: sq, sk
 // on entry).
 template <typename T, typename Ln, bool GIVEN, bool ROPE>
-__device__ __forceinline__ void pyr_token(const PyrArgs& a, int b, int h, int l16, size_t srow, int t,
+__device__ __forceinline__ void pyr_token(const PyrArgs& a, int b, int h, int l16, int t,
                                           const uint4 xq, const uint4 xk, const uint4 xv, float* fq, float* fk,
                                           float* fv, float& sq, float& sk) {
   unpack8_t<T>(xq, fq);
@@ -111,7 +111,7 @@ __global__ __launch_bounds__(256) void pyramid_fwd_kernel(const PyrArgs a) {
   auto token = [&](int t, const uint4 xq, const uint4 xk, const uint4 xv, float sq, float sk)
       __attribute__((always_inline)) {
     float fq[8], fk[8], fv[8];
-    pyr_token<T, Ln, GIVEN, ROPE>(a, b, h, l16, srow, t, xq, xk, xv, fq, fk, fv, sq, sk);
+    pyr_token<T, Ln, GIVEN, ROPE>(a, b, h, l16, t, xq, xk, xv, fq, fk, fv, sq, sk);
     if (CAT && in) {
       const int64_t co = (int64_t)b * a.pb + (int64_t)t * a.ps + (int64_t)h * a.ph + 8 * l16;
       *reinterpret_cast<uint4*>(a.cq + co) = xq;
@@ -223,7 +223,7 @@ __global__ __launch_bounds__(256) void pyramid_tile_kernel(const PyrArgs a, int 
     const int64_t o = xoff + (int64_t)t * a.ss;
     const uint4 xq = in ? ld16(a.xq + o) : zero, xk = in ? ld16(a.xk + o) : zero, xv = in ? ld16(a.xv + o) : zero;
     float fq[8], fk[8], fv[8], sq, sk;
-    pyr_token<T, Ln, false, ROPE>(a, b, h, l16, srow, t, xq, xk, xv, fq, fk, fv, sq, sk);
+    pyr_token<T, Ln, false, ROPE>(a, b, h, l16, t, xq, xk, xv, fq, fk, fv, sq, sk);
     X[0][i * Ln::LPR + l16] = ROPE ? pack8_t<T>(fq) : xq;  // the rotated rows' own 16 bits
     X[1][i * Ln::LPR + l16] = ROPE ? pack8_t<T>(fk) : xk;
     X[2][i * Ln::LPR + l16] = xv;
@@ -353,7 +353,7 @@ int tile_tokens(const PyrArgs& a, bool given) {
   if (given || a.cq || a.cmax > PYR_TILE) return 0;
   const int rows = a.D <= 64 ? 32 : 16;
   const int waves = (a.units + rows / 4 - 1) / (rows / 4);
-  return waves <= (a.fs ? 1024 : 256) ? std::max(rows, a.cmax) : 0;
+  return waves <= (a.fs ? 4 : 1) * lh_cu_count() ? std::max(rows, a.cmax) : 0;
 }
 
 template <typename T, int NL>
