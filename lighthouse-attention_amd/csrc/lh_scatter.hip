@@ -154,7 +154,9 @@ __global__ __launch_bounds__(64) void scatter_bwd_kernel(const ScatArgs a) {
 // causal attention), and dout copied to contiguous rows on the way where its
 // strides ask for it: one pass over both tensors.  Bound by memory; as torch
 // operations (two widening casts, a product, a sum and the copy) it took 115 us
-// at 8 heads of 16384, in one pass 20 us.
+// at 8 heads of 16384, in one pass 20 us.  The products are summed as those
+// operations did, four at a time and then pairwise over the groups, so the
+// backward has the bits that it had with them.
 struct DeltaArgs {
   const bf16_t *dout, *o;
   bf16_t* copy;  // [BH, n, D] or null
@@ -163,6 +165,11 @@ struct DeltaArgs {
   int H, n, D;
   int chunks;  // blocks per (b, h)
 };
+
+__device__ __forceinline__ float sum4(const float* a, const float* b) {
+#pragma clang fp contract(off)
+  return ((a[0] * b[0] + a[1] * b[1]) + a[2] * b[2]) + a[3] * b[3];
+}
 
 template <typename T, typename Ln>
 __global__ __launch_bounds__(256) void attn_delta_kernel(const DeltaArgs a) {
@@ -179,8 +186,7 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(const DeltaArgs a) {
     float g[8], o[8];
     unpack8_t<T>(gv, g);
     unpack8_t<T>(ov, o);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) d = fmaf(g[e], o[e], d);
+    d = sum4(g, o) + sum4(g + 4, o + 4);
   }
 #pragma unroll
   for (int m = 1; m < Ln::LPR; m <<= 1) d += __shfl_xor(d, m, Ln::LPR);

@@ -320,6 +320,12 @@ def test_attn_delta(pkg, dev, D, dtype):
         # fp32 sums of D products of 16-bit values: D roundings at most
         bound = D * 2.0 ** -24 * (f.double() * o.double()).abs().sum(-1)
         assert bool(((delta.double() - ref).abs() <= bound).all()), f"form {i}"
+        # the order of the sum: four products after each other, then pairs of neighbours
+        p = torch.nn.functional.pad(f.float() * o.float(), (0, 128 - D)).unflatten(-1, (32, 4))
+        p = ((p[..., 0] + p[..., 1]) + p[..., 2]) + p[..., 3]
+        while p.shape[-1] > 1:
+            p = p[..., 0::2] + p[..., 1::2]
+        assert torch.equal(delta, p[..., 0]), f"form {i}: another order"
 
 
 @pytest.mark.parametrize("D,S,L,p,dtype", [(128, 1000, 3, 4, torch.bfloat16), (72, 257, 2, 2, torch.float16),
