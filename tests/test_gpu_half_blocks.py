@@ -3,6 +3,8 @@ workgroup of four waves; lh_attn.hip, half_blocks): forward, dQ and the unchange
 dK/dV against fp32 attention, at sizes around the 64-row tiles and the 128-row
 blocks, for few and for many heads; and bit for bit against whole blocks, so that
 a sequence has the same results alone and in a batch."""
+import ctypes
+
 import pytest
 import torch
 
@@ -95,27 +97,54 @@ def test_half_blocks_have_whole_blocks_bits(pkg, dev, n, H, D, dtype, gathered, 
         assert torch.equal(a, b), name
 
 
-def _kernel_names(f):
-    from torch.profiler import ProfilerActivity, profile
+class _Dim3(ctypes.Structure):
+    _fields_ = [(c, ctypes.c_uint) for c in "xyz"]
+
+
+class _KernelNode(ctypes.Structure):  # hipKernelNodeParams
+    _fields_ = [("block", _Dim3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", _Dim3),
+                ("params", ctypes.c_void_p), ("shared", ctypes.c_uint)]
+
+
+def _launches(pkg, f):
+    """(workgroups, threads) of every kernel that f launches, from a captured graph."""
+    hip = pkg._native.lib()  # the library's handle finds the runtime that it is linked with
     f()
     torch.cuda.synchronize()
-    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
         f()
-        torch.cuda.synchronize()
-    return [e.name for e in prof.events()]
+    raw, n = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(raw, None, ctypes.byref(n)) == 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(n)) == 0
+    out = []
+    for node in nodes:
+        kind, p = ctypes.c_int(), _KernelNode()
+        assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)) == 0
+        if kind.value == 0:  # a kernel
+            assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
+            out.append((p.grid.x, p.block.x))
+    return out
 
 
 def test_which_launches_take_half_blocks(pkg, dev):
-    """Waves of a workgroup by the kernels' names: four up to two half blocks per CU,
-    eight beyond, for one block of 128 rows, and in calls without the flag."""
-    cus = torch.cuda.get_device_properties(dev).multi_processor_count
-    rows = 2 * cus // 8 * 128  # 8 heads: two half blocks to a CU
-    for n, shaped, waves in ((129, True, 4), (rows, True, 4), (128, True, 8), (rows + 1, True, 8), (129, False, 8)):
-        xs, _, do = _inputs(n, 8, torch.bfloat16, dev, False)
-        names = _kernel_names(lambda: _calls(pkg, xs, None, do, n, 8, 128, shaped))
-        for kernel, args in (("attn_fwd_kernel", f", {waves}, 0>"), ("attn_bwd_dq_kernel", f", {waves}>")):
-            got = [x for x in names if kernel in x]
-            assert got and all(args in x for x in got), f"n={n} shaped={shaped}: {got}"
+    """Four waves to a workgroup and one block of 128 rows each, up to two of them per
+    CU; eight waves beyond, for one block of 128 rows, and in calls without the flag."""
+    N = pkg._native
+    H = 8
+    most = 2 * torch.cuda.get_device_properties(dev).multi_processor_count // H  # half blocks per head
+    for n, shaped, half in ((129, True, True), (most * 128, True, True), (128, True, False),
+                            (most * 128 + 1, True, False), (129, False, False)):
+        xs, _, do = _inputs(n, H, torch.bfloat16, dev, False)
+        rows = N.Rows(*xs, xs[0].stride()[:3])
+        lse = torch.zeros(1, H, n, device=dev)
+        for name, f in (("forward", lambda: N.attn_fwd(rows, None, 1, H, n, shaped=shaped)),
+                        ("dQ", lambda: N.attn_bwd_dq(rows, None, 1, H, n, do, lse, lse, shaped=shaped))):
+            got = _launches(pkg, f)
+            assert len(got) == 1 and got[0][1] == (256 if half else 512), f"{name}, n={n}, shaped={shaped}: {got}"
+            if half:
+                assert got[0][0] == H * -(-n // 128), f"{name}, n={n}: {got}"
 
 
 @pytest.mark.parametrize("D", [128, 64])
